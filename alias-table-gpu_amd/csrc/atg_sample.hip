@@ -23,6 +23,49 @@ __device__ __forceinline__ void load_row(const SampleArgs& a, int64_t row, doubl
     }
 }
 
+// Counters of sampled items, kept in LDS by one block.  A few items draw a
+// large share of the samples of a skewed table, and device atomics on one
+// address run one after another (1e7 samples of a 2^20-item Pareto(1.1) table
+// whose heaviest item has 4% of the mass: 2.4 ms).  A slot of the table
+// belongs to the first item that claims it and counts that item's samples;
+// other items of the slot go to the counters in HBM.  A hot item claims its
+// slot among the block's first samples, so what goes to HBM is spread thin.
+// Integer sums: the same counts in any order.
+constexpr int kHistSlots = 4096;        // 32 KB
+constexpr int kHistThreads = 512;       // 4 blocks, 32 waves a CU
+// Samples a block draws at least, so that clearing and flushing its slots
+// (8 per thread each) stays small beside them.
+constexpr int kHistMinPerBlock = 8192;
+
+struct HistCache {
+    int32_t* key;   // [kHistSlots] item, -1: free
+    uint32_t* cnt;  // [kHistSlots]
+    __device__ __forceinline__ void clear() {
+        for (int k = threadIdx.x; k < kHistSlots; k += blockDim.x) {
+            key[k] = -1;
+            cnt[k] = 0u;
+        }
+        __syncthreads();
+    }
+    __device__ __forceinline__ void add(uint32_t* hist, int32_t item) {
+        const int slot = item & (kHistSlots - 1);
+        int32_t k = *(volatile int32_t*)&key[slot];
+        if (k == -1) {
+            const int32_t was = (int32_t)atomicCAS((int*)&key[slot], -1, item);
+            k = was == -1 ? item : was;
+        }
+        if (k == item) atomicAdd(&cnt[slot], 1u);
+        else atomicAdd(&hist[item], 1u);
+    }
+    __device__ __forceinline__ void flush(uint32_t* hist) {
+        __syncthreads();
+        for (int k = threadIdx.x; k < kHistSlots; k += blockDim.x) {
+            const uint32_t c = cnt[k];
+            if (c) atomicAdd(&hist[key[k]], c);
+        }
+    }
+};
+
 __device__ __forceinline__ void emit(const SampleArgs& a, uint64_t g, int32_t item, uint64_t& csum) {
     if (a.out) a.out[g] = item;
     if (a.hist) atomicAdd(&a.hist[item], 1u);
@@ -36,10 +79,19 @@ __device__ __forceinline__ void flush_checksum(const SampleArgs& a, uint64_t csu
 }
 
 // ---------------------------------------------------------------------------
-// Basic sampling: one uniform row per sample over the whole table.
+// Basic sampling: one uniform row per sample over the whole table.  Without
+// counts it is bound by random row reads (1e7 samples from 2^20 rows: 0.135 ms,
+// 74 G rows/s out of the Infinity Cache); the counters of the cold items add
+// about as many random atomics (0.356 ms with them; 2.5-11 ms, by the weight
+// of the heaviest item, when every sample went to its counter in HBM).
 #define BASIC_UNROLL 4
-template <bool AOS>
-__global__ __launch_bounds__(256) void sample_basic(SampleArgs a) {
+// CACHED: the counts per item go through the block's LDS counters.
+template <bool AOS, bool CACHED>
+__global__ __launch_bounds__(CACHED ? kHistThreads : 256) void sample_basic(SampleArgs a) {
+    __shared__ int32_t hkey[CACHED ? kHistSlots : 1];
+    __shared__ uint32_t hcnt[CACHED ? kHistSlots : 1];
+    HistCache hc{hkey, hcnt};
+    if (CACHED) hc.clear();
     const double W_N = a.st->W_N;
     uint64_t csum = 0;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -61,9 +113,19 @@ __global__ __launch_bounds__(256) void sample_basic(SampleArgs a) {
 #pragma unroll
         for (int q = 0; q < BASIC_UNROLL; ++q) {
             const uint64_t g = g0 + (uint64_t)q * stride;
-            if (g < a.count) emit(a, g, decide(w[q], al[q], row[q], coin53(r[q]), W_N, a.n), csum);
+            if (g < a.count) {
+                const int32_t item = decide(w[q], al[q], row[q], coin53(r[q]), W_N, a.n);
+                if (CACHED) {
+                    if (a.out) a.out[g] = item;
+                    hc.add(a.hist, item);
+                    csum += (uint64_t)(uint32_t)item;
+                } else {
+                    emit(a, g, item, csum);
+                }
+            }
         }
     }
+    if (CACHED) hc.flush(a.hist);
     flush_checksum(a, csum);
 }
 
@@ -623,9 +685,17 @@ static inline unsigned grid_for(uint64_t count, unsigned block, unsigned cap) {
 }
 
 hipError_t launch_sample_basic(const SampleArgs& a, hipStream_t s) {
+    // Counts per item: through LDS once two blocks have their least share of
+    // samples; below that few samples meet on one counter.
+    if (a.hist && a.count >= 2 * (uint64_t)kHistMinPerBlock) {
+        const unsigned g = grid_for(a.count, kHistMinPerBlock, 256 * 4);
+        if (a.rows) hipLaunchKernelGGL((sample_basic<true, true>), dim3(g), dim3(kHistThreads), 0, s, a);
+        else hipLaunchKernelGGL((sample_basic<false, true>), dim3(g), dim3(kHistThreads), 0, s, a);
+        return hipGetLastError();
+    }
     const unsigned g = grid_for(a.count, 256, 256 * 64);
-    if (a.rows) hipLaunchKernelGGL(sample_basic<true>, dim3(g), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(sample_basic<false>, dim3(g), dim3(256), 0, s, a);
+    if (a.rows) hipLaunchKernelGGL((sample_basic<true, false>), dim3(g), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((sample_basic<false, false>), dim3(g), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
