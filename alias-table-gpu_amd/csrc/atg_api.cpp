@@ -706,7 +706,6 @@ atg_status atg_sample(atg_table* t, atg_sample_kind kind, uint64_t count, uint64
                 t->sec_counts_cap = a.nsec;
             }
             a.sec_counts = t->d_sec_counts;
-            HIPCHK(set_sample_lds_limit((int)(section_rows * sizeof(Row))));
             HIPCHK(launch_sample_sectioned(a, s));
         } else {
             return fail(ATG_EINVAL, "atg_sample: unknown kind %d", (int)kind);
@@ -936,7 +935,6 @@ atg_status atg_rejection_sample_sectioned(atg_table* t, uint64_t count, uint64_t
     a.checksum = checksum ? t->d_checksum : nullptr;
     if (checksum) HIPCHK(hipMemsetAsync(t->d_checksum, 0, 8, s));
     if (count > 0) {
-        HIPCHK(set_rej_sample_lds_limit((int)(section_slots * sizeof(RejEntry))));
         HIPCHK(launch_rejection_sample_sectioned(r, a, masses, s));
         t->rej_sec_valid = true;
         t->rej_sec_SS = section_slots;

@@ -25,23 +25,50 @@ struct u32x4 {
     uint32_t x, y, z, w;
 };
 
+// a ^ b ^ c in one instruction (v_bitop3_b32, truth table 0x96).
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+}
+
+// One round; the 32x32 -> 64-bit products (v_mad_u64_u32) give both halves at
+// once: half the multiply instructions of a separate mul_lo / mul_hi pair.
+__device__ __forceinline__ u32x4 philox_round(u32x4 c, uint32_t k0, uint32_t k1) {
+    const uint64_t p0 = (uint64_t)0xD2511F53u * c.x;
+    const uint64_t p1 = (uint64_t)0xCD9E8D57u * c.z;
+    return u32x4{xor3((uint32_t)(p1 >> 32), c.y, k0), (uint32_t)p1, xor3((uint32_t)(p0 >> 32), c.w, k1), (uint32_t)p0};
+}
+
 __device__ __forceinline__ u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1) {
 #pragma unroll
-    for (int r = 0; r < 10; ++r) {
-        if (r > 0) {
-            k0 += 0x9E3779B9u;
-            k1 += 0xBB67AE85u;
-        }
-        // One 32x32 -> 64-bit product (v_mad_u64_u32) gives both halves:
-        // half the multiply instructions of a separate mul_lo / mul_hi pair.
-        const uint64_t p0 = (uint64_t)0xD2511F53u * c.x;
-        const uint64_t p1 = (uint64_t)0xCD9E8D57u * c.z;
-        const uint32_t lo0 = (uint32_t)p0, hi0 = (uint32_t)(p0 >> 32);
-        const uint32_t lo1 = (uint32_t)p1, hi1 = (uint32_t)(p1 >> 32);
-        c = u32x4{hi1 ^ c.y ^ k0, lo1, hi0 ^ c.w ^ k1, lo0};
-    }
+    for (int r = 0; r < 10; ++r) c = philox_round(c, k0 + r * 0x9E3779B9u, k1 + r * 0xBB67AE85u);
     return c;
 }
+
+// Counters of one stream that share their high word, purpose and key, all
+// scalars: what the first two rounds make of those alone is scalar work done
+// once (one of 19 vector multiplies and three of 20 xors per block less).
+struct PhiloxStream {
+    uint32_t k0, k1;
+    uint32_t a, b;   // round 2 without its vector product: x = a ^ hi, z = b ^ w
+    uint32_t w2;     // the last word after round 2
+    __device__ __forceinline__ PhiloxStream(uint32_t hi, uint32_t purpose, uint64_t seed)
+        : k0((uint32_t)seed), k1((uint32_t)(seed >> 32)) {
+        const uint64_t p1 = (uint64_t)0xCD9E8D57u * purpose;
+        const uint64_t p0 = (uint64_t)0xD2511F53u * ((uint32_t)(p1 >> 32) ^ hi ^ k0);
+        a = (uint32_t)p1 ^ (k0 + 0x9E3779B9u);
+        b = (uint32_t)(p0 >> 32) ^ (k1 + 0xBB67AE85u);
+        w2 = (uint32_t)p0;
+    }
+    // The block at counter (lo, hi, purpose, extra).
+    __device__ __forceinline__ u32x4 at(uint32_t lo, uint32_t extra) const {
+        const uint64_t p0 = (uint64_t)0xD2511F53u * lo;
+        const uint64_t p1 = (uint64_t)0xCD9E8D57u * ((uint32_t)(p0 >> 32) ^ (extra ^ k1));
+        u32x4 c{(uint32_t)(p1 >> 32) ^ a, (uint32_t)p1, (uint32_t)p0 ^ b, w2};
+#pragma unroll
+        for (int r = 2; r < 10; ++r) c = philox_round(c, k0 + r * 0x9E3779B9u, k1 + r * 0xBB67AE85u);
+        return c;
+    }
+};
 
 __device__ __forceinline__ u32x4 philox_at(uint64_t idx, uint32_t purpose, uint32_t extra, uint64_t seed) {
     return philox4x32_10(u32x4{(uint32_t)idx, (uint32_t)(idx >> 32), purpose, extra}, (uint32_t)seed,
@@ -49,13 +76,20 @@ __device__ __forceinline__ u32x4 philox_at(uint64_t idx, uint32_t purpose, uint3
 }
 
 __device__ __forceinline__ uint64_t word64(u32x4 r) { return ((uint64_t)r.y << 32) | r.x; }
+__device__ __forceinline__ uint64_t coin64(u32x4 r) { return ((uint64_t)r.w << 32) | r.z; }
+// The coin's 53 bits v >> 11 as a double in [0, 1): the two words of v with
+// its low 11 bits cleared have 53 bits between them, so the sum is exact.
 __device__ __forceinline__ double coin53(u32x4 r) {
-    const uint64_t v = ((uint64_t)r.w << 32) | r.z;
-    return (double)(v >> 11) * 0x1.0p-53;
+    return __builtin_fma((double)r.w, 0x1.0p32, (double)(r.z & ~0x7FFu)) * 0x1.0p-64;
 }
 // floor(x * n / 2^64): a uniform row in [0, n) without the 2^-32 bias of a
 // 32-bit multiply-shift.
 __device__ __forceinline__ uint64_t scale64(uint64_t x, uint64_t n) { return __umul64hi(x, n); }
+// The same for n < 2^32, with two multiplies instead of six: x n / 2^64 =
+// (hi n + lo n / 2^32) / 2^32, floors at both divisions.
+__device__ __forceinline__ uint32_t scale64(uint64_t x, uint32_t n) {
+    return (uint32_t)(((x >> 32) * n + __umulhi((uint32_t)x, n)) >> 32);
+}
 
 // ---------------------------------------------------------------------------
 // Wavefront primitives (wave64).
@@ -205,7 +239,9 @@ __device__ __forceinline__ double u2d(uint64_t u) { return __longlong_as_double(
 // (the pack's heavy sentinel N) keeps the row.
 __device__ __forceinline__ int32_t decide(double rw, int32_t alias, int64_t row, double u, double W_N,
                                           int64_t n) {
-    return (rw < W_N && u * W_N >= rw && alias >= 0 && alias < n) ? alias : (int32_t)row;
+    // One straight run (n < 2^31): some lane of a wave always needs the coin.
+    const bool take = (int)(rw < W_N) & (int)(u * W_N >= rw) & (int)((uint32_t)alias < (uint32_t)n);
+    return take ? alias : (int32_t)row;
 }
 
 }  // namespace atg

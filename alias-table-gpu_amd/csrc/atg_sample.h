@@ -82,9 +82,7 @@ struct RejSecArgs {
 hipError_t launch_sample_basic(const SampleArgs& a, hipStream_t s);
 // masses: recompute the section masses and their prefix (a new A or section size).
 hipError_t launch_rejection_sample_sectioned(const RejSecArgs& a, const SampleArgs& sa, bool masses, hipStream_t s);
-hipError_t set_rej_sample_lds_limit(int bytes);
 hipError_t launch_sample_sectioned(const SampleArgs& a, hipStream_t s);
-hipError_t set_sample_lds_limit(int bytes);
 // The counts, their scan and the fill (with the incl pass and the model fit
 // the search fills need); launch_rejection_fill repeats the fill alone.
 hipError_t launch_rejection_build(const RejArgs& a, int fill, hipStream_t s);

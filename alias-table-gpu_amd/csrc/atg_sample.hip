@@ -31,24 +31,25 @@ __device__ __forceinline__ void load_row(const SampleArgs& a, int64_t row, doubl
 // other items of the slot go to the counters in HBM.  A hot item claims its
 // slot among the block's first samples, so what goes to HBM is spread thin.
 // Integer sums: the same counts in any order.
-constexpr int kHistSlots = 4096;        // 32 KB
-constexpr int kHistThreads = 512;       // 4 blocks, 32 waves a CU
+constexpr int kHistSlots = 4096;        // 32 KB: four blocks of kHistThreads, 32 waves a CU
+constexpr int kHistThreads = 512;
 // Samples a block draws at least, so that clearing and flushing its slots
 // (8 per thread each) stays small beside them.
 constexpr int kHistMinPerBlock = 8192;
 
+template <int SLOTS>
 struct HistCache {
-    int32_t* key;   // [kHistSlots] item, -1: free
-    uint32_t* cnt;  // [kHistSlots]
+    int32_t* key;   // [SLOTS] item, -1: free
+    uint32_t* cnt;  // [SLOTS]
     __device__ __forceinline__ void clear() {
-        for (int k = threadIdx.x; k < kHistSlots; k += blockDim.x) {
+        for (int k = threadIdx.x; k < SLOTS; k += blockDim.x) {
             key[k] = -1;
             cnt[k] = 0u;
         }
         __syncthreads();
     }
     __device__ __forceinline__ void add(uint32_t* hist, int32_t item) {
-        const int slot = item & (kHistSlots - 1);
+        const int slot = item & (SLOTS - 1);
         int32_t k = *(volatile int32_t*)&key[slot];
         if (k == -1) {
             const int32_t was = (int32_t)atomicCAS((int*)&key[slot], -1, item);
@@ -59,7 +60,7 @@ struct HistCache {
     }
     __device__ __forceinline__ void flush(uint32_t* hist) {
         __syncthreads();
-        for (int k = threadIdx.x; k < kHistSlots; k += blockDim.x) {
+        for (int k = threadIdx.x; k < SLOTS; k += blockDim.x) {
             const uint32_t c = cnt[k];
             if (c) atomicAdd(&hist[key[k]], c);
         }
@@ -90,7 +91,7 @@ template <bool AOS, bool CACHED>
 __global__ __launch_bounds__(CACHED ? kHistThreads : 256) void sample_basic(SampleArgs a) {
     __shared__ int32_t hkey[CACHED ? kHistSlots : 1];
     __shared__ uint32_t hcnt[CACHED ? kHistSlots : 1];
-    HistCache hc{hkey, hcnt};
+    HistCache<kHistSlots> hc{hkey, hcnt};
     if (CACHED) hc.clear();
     const double W_N = a.st->W_N;
     uint64_t csum = 0;
@@ -107,7 +108,7 @@ __global__ __launch_bounds__(CACHED ? kHistThreads : 256) void sample_basic(Samp
         for (int q = 0; q < BASIC_UNROLL; ++q) {
             const uint64_t g = g0 + (uint64_t)q * stride;
             r[q] = philox_at(g, PURPOSE_BASIC, 0, a.seed);
-            row[q] = (int64_t)scale64(word64(r[q]), (uint64_t)a.n);
+            row[q] = (int64_t)scale64(word64(r[q]), (uint32_t)a.n);
             if (g < a.count) load_row<AOS>(a, row[q], w[q], al[q]);
         }
 #pragma unroll
@@ -203,14 +204,46 @@ __global__ __launch_bounds__(64) void section_counts(SampleArgs a) {
     a.sec_counts[2 * s + 1] = o;
 }
 
-template <bool AOS>
+// body(base, hi, lo) for the outputs g of [off, off + cnt) that this thread of
+// a group of `threads` draws: (hi, lo) the words of g, hi a scalar, and g =
+// base + tid with base a scalar.
+template <typename Init, typename Body>
+__device__ __forceinline__ void for_outputs(uint64_t off, uint64_t cnt, uint32_t threads, uint32_t tid, Init init,
+                                            Body body) {
+    const uint64_t end = off + cnt;
+    for (uint64_t b = off; b < end;) {
+        const uint32_t hi = (uint32_t)(b >> 32);
+        const auto stream = init(hi);
+        const uint64_t seg_end = min(end, ((uint64_t)hi + 1) << 32);
+        // Whole rounds of the group without a test, then the rest.
+        for (; seg_end - b >= threads; b += threads) body(stream, b, (uint32_t)b + tid);
+        if (tid < (uint32_t)(seg_end - b)) body(stream, b, (uint32_t)b + tid);
+        b = seg_end;
+    }
+}
+
+// LDS counters of the sectioned samplers: 16 KB beside a 64 KB section keep
+// two blocks on a CU.
+constexpr int kSecHistSlots = 2048;
+
+// Bound by the VALU: 19 wide multiplies, 18 xors and about 20 other vector
+// instructions per sample (24, 36 and 30 before the shared part of the Philox
+// rounds, the three-way xors, the narrow row scaling and the straight decision:
+// 1e9 samples from 1e8 rows 2.20 -> 1.74 ms).  Of that 0.25 ms is the staging
+// of 1.6 GB.  Three blocks per CU with 12-byte rows, two samples per iteration
+// and non-temporal output stores were no faster.
+template <bool AOS, bool CACHED>
 __global__ __launch_bounds__(SECTIONED_THREADS) void sample_sectioned(SampleArgs a) {
     extern __shared__ Row sect[];
+    HistCache<kSecHistSlots> hc{reinterpret_cast<int32_t*>(sect + a.SS),
+                                reinterpret_cast<uint32_t*>(sect + a.SS) + kSecHistSlots};
+    if (CACHED) hc.clear();
     const int64_t s = blockIdx.x;
     const int64_t start = s * a.SS;
-    const int64_t len = min(a.n, start + a.SS) - start;
+    const uint32_t len = (uint32_t)(min(a.n, start + a.SS) - start);
+    const double W_N = a.st->W_N;
     // Stage the section's rows in LDS (SamplerGpuSectionedShared.cu:58-63).
-    for (int64_t k = threadIdx.x; k < len; k += blockDim.x) {
+    for (uint32_t k = threadIdx.x; k < len; k += blockDim.x) {
         if (AOS) {
             *reinterpret_cast<uint4*>(&sect[k]) = *reinterpret_cast<const uint4*>(&a.rows[start + k]);
         } else {
@@ -221,16 +254,145 @@ __global__ __launch_bounds__(SECTIONED_THREADS) void sample_sectioned(SampleArgs
     }
     __syncthreads();
     const uint64_t cnt = a.sec_counts[2 * s], off = a.sec_counts[2 * s + 1];
-    const double W_N = a.st->W_N;
     uint64_t csum = 0;
-    for (uint64_t t = threadIdx.x; t < cnt; t += blockDim.x) {
-        const uint64_t g = off + t;
-        const u32x4 r = philox_at(g, PURPOSE_SECTIONED, 0, a.seed);
-        const int64_t row = (int64_t)scale64(word64(r), (uint64_t)len);
+    const uint32_t t = threadIdx.x;
+    for_outputs(off, cnt, SECTIONED_THREADS, t, [&](uint32_t hi) { return PhiloxStream(hi, PURPOSE_SECTIONED, a.seed); },
+                [&](const PhiloxStream& ps, uint64_t b, uint32_t lo) {
+        const u32x4 r = ps.at(lo, 0);
+        const uint32_t row = scale64(word64(r), len);
         const uint4 v = *reinterpret_cast<const uint4*>(&sect[row]);
         const double w = __longlong_as_double(((long long)v.y << 32) | v.x);
-        emit(a, g, decide(w, (int32_t)v.z, start + row, coin53(r), W_N, a.n), csum);
+        const int32_t item = decide(w, (int32_t)v.z, start + row, coin53(r), W_N, a.n);
+        if (a.out) (a.out + b)[t] = item;
+        if (CACHED) hc.add(a.hist, item);
+        if (a.checksum) csum += (uint64_t)(uint32_t)item;
+    });
+    if (CACHED) hc.flush(a.hist);
+    flush_checksum(a, csum);
+}
+
+// ---------------------------------------------------------------------------
+// Sectioned sampling with few samples per row: staging a section would read
+// all its rows for the few that are drawn, so a wave per section reads the
+// drawn rows from HBM, and finds its section's count itself where that saves a
+// launch (65,536 samples from 1e7 rows: 39 -> 12 us).
+
+// Count and first output of section s by one wave: section_count with its
+// draws side by side.  The path to s, its nodes and their uniform sums do not
+// depend on the counts, so lane l prepares level l; what is left level by
+// level is the draw's arithmetic (and for counts of at most 32 its Bernoulli
+// trials, one a lane).
+__device__ __forceinline__ void section_count_wave(const SampleArgs& a, int64_t s, int lane, uint64_t& cnt,
+                                                   uint64_t& off) {
+    int64_t lo = 0, hi = a.nsec;
+    uint64_t node = 1, my_node = 1;
+    double my_q = 0.0;
+    uint64_t left = 0;  // bit l: the path goes left at level l
+    int levels = 0;
+    for (; hi - lo > 1; ++levels) {
+        const int64_t mid = lo + (hi - lo) / 2;
+        const bool mine = lane == levels;
+        const int64_t rl = min(a.n, mid * a.SS) - lo * a.SS;
+        const int64_t rt = min(a.n, hi * a.SS) - lo * a.SS;
+        if (mine) {
+            my_q = (double)rl / (double)rt;
+            my_node = node;
+        }
+        if (s < mid) {
+            left |= 1ull << levels;
+            hi = mid; node = 2 * node;
+        } else {
+            lo = mid; node = 2 * node + 1;
+        }
     }
+    double z = 0.0;
+    for (uint32_t d = 0; d < 3; ++d) {
+        const u32x4 x = philox_at(my_node, PURPOSE_SECTION_COUNTS, d, a.seed);
+        z = z + (double)x.x * 0x1.0p-32;
+        z = z + (double)x.y * 0x1.0p-32;
+        z = z + (double)x.z * 0x1.0p-32;
+        z = z + (double)x.w * 0x1.0p-32;
+    }
+    z = z - 6.0;
+    uint64_t c = a.count, o = 0;
+    for (int l = 0; l < levels && c != 0; ++l) {
+        const double q = readlane_d(my_q, l);
+        uint64_t x;
+        if (c <= 32) {
+            const uint64_t nd = readlane_u64(my_node, l);
+            const u32x4 y = philox_at(nd, PURPOSE_SECTION_COUNTS, (uint32_t)lane >> 2, a.seed);
+            const uint32_t word = ((lane & 3) == 0) ? y.x : ((lane & 3) == 1) ? y.y : ((lane & 3) == 2) ? y.z : y.w;
+            x = (uint64_t)__popcll(__ballot(lane < (int)c && (double)word * 0x1.0p-32 < q));
+        } else {
+            const double mean = (double)c * q;
+            const double sd = __builtin_sqrt(mean * (1.0 - q));
+            double r = floor((mean + sd * readlane_d(z, l)) + 0.5);
+            if (r < 0.0) r = 0.0;
+            if (r > (double)c) r = (double)c;
+            x = (uint64_t)r;
+            x = readlane_u64(x, 0);
+        }
+        if ((left >> l) & 1) {
+            c = x;
+        } else {
+            o += x; c = c - x;
+        }
+    }
+    cnt = c;
+    off = o;
+}
+
+// SPARSE_UNROLL rows per lane in flight.
+#define SPARSE_UNROLL 4
+// COUNTS: the section counts are found here, by the section's wave, instead of
+// by an earlier launch.
+template <bool AOS, bool CACHED, bool COUNTS>
+__global__ __launch_bounds__(CACHED ? kHistThreads : 256) void sample_sectioned_sparse(SampleArgs a) {
+    __shared__ int32_t hkey[CACHED ? kHistSlots : 1];
+    __shared__ uint32_t hcnt[CACHED ? kHistSlots : 1];
+    HistCache<kHistSlots> hc{hkey, hcnt};
+    if (CACHED) hc.clear();
+    const int lane = threadIdx.x & 63;
+    const double W_N = a.st->W_N;
+    uint64_t csum = 0;
+    const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
+    for (int64_t s = (int64_t)blockIdx.x * (blockDim.x >> 6) + wave_in_block(); s < a.nsec; s += waves) {
+        uint64_t cnt, off;
+        if (COUNTS) {
+            section_count_wave(a, s, lane, cnt, off);
+        } else {
+            cnt = a.sec_counts[2 * s];
+            off = a.sec_counts[2 * s + 1];
+        }
+        const int64_t start = s * a.SS;
+        const uint32_t len = (uint32_t)(min(a.n, start + a.SS) - start);
+        for (uint64_t t0 = 0; t0 < cnt; t0 += 64 * SPARSE_UNROLL) {
+            u32x4 r[SPARSE_UNROLL];
+            int64_t row[SPARSE_UNROLL];
+            double w[SPARSE_UNROLL];
+            int32_t al[SPARSE_UNROLL];
+#pragma unroll
+            for (int q = 0; q < SPARSE_UNROLL; ++q) {
+                if (t0 + 64 * q >= cnt) break;  // scalar
+                // Lanes past the last sample draw like the others and drop it.
+                r[q] = philox_at(off + t0 + 64 * q + lane, PURPOSE_SECTIONED, 0, a.seed);
+                row[q] = start + scale64(word64(r[q]), len);
+                load_row<AOS>(a, row[q], w[q], al[q]);
+            }
+#pragma unroll
+            for (int q = 0; q < SPARSE_UNROLL; ++q) {
+                const uint64_t t = t0 + 64 * q + lane;
+                if (t0 + 64 * q >= cnt) break;
+                if (t >= cnt) continue;
+                const int32_t item = decide(w[q], al[q], row[q], coin53(r[q]), W_N, a.n);
+                if (a.out) a.out[off + t] = item;
+                if (CACHED) hc.add(a.hist, item);
+                else if (a.hist) atomicAdd(&a.hist[item], 1u);
+                csum += (uint64_t)(uint32_t)item;
+            }
+        }
+    }
+    if (CACHED) hc.flush(a.hist);
     flush_checksum(a, csum);
 }
 
@@ -646,33 +808,57 @@ __global__ __launch_bounds__(64) void rej_section_counts(RejSecArgs a, uint64_t 
 // sample of the section makes trials t = 0, 1, ... with the Philox block at
 // counter (output position, PURPOSE_REJ_SECTIONED, t): a uniform slot of the
 // section from words 0-1 and the coin from words 2-3.
+// A slot is staged as the largest coin word that accepts it: the 53-bit coin
+// v >> 11 accepts iff v >> 11 <= accept 2^53, so iff v <= floor(accept 2^53)
+// 2^11 + 2^11 - 1 (every v when accept >= 1), and a trial compares integers.
+template <bool CACHED>
 __global__ __launch_bounds__(REJ_SEC_THREADS) void rej_sample_sectioned(RejSecArgs a, SampleArgs sa) {
-    extern __shared__ RejEntry rsect[];
+    extern __shared__ ulonglong2 rsect[];  // x: the largest accepting coin word, y: the item
+    HistCache<kSecHistSlots> hc{reinterpret_cast<int32_t*>(rsect + a.SS),
+                                reinterpret_cast<uint32_t*>(rsect + a.SS) + kSecHistSlots};
+    if (CACHED) hc.clear();
     const int64_t k = blockIdx.x;
     const uint64_t start = (uint64_t)k * (uint64_t)a.SS;
-    const uint64_t len = min(a.A_size, start + (uint64_t)a.SS) - start;
-    for (uint64_t s = threadIdx.x; s < len; s += blockDim.x)
-        *reinterpret_cast<uint4*>(&rsect[s]) = *reinterpret_cast<const uint4*>(&a.A[start + s]);
-    __syncthreads();
-    const uint64_t cnt = a.sec_counts[2 * k], off = a.sec_counts[2 * k + 1];
-    uint64_t csum = 0;
-    // One trial per iteration; a lane whose trial accepts goes on to its next
-    // sample at once, so no lane waits for another lane's rejected trials
-    // (the trials of every sample are those of the one-sample-at-a-time loop).
-    uint64_t t = threadIdx.x;
-    uint32_t tr = 0;
-    while (t < cnt) {
-        const uint64_t g = off + t;
-        const u32x4 r = philox_at(g, PURPOSE_REJ_SECTIONED, tr, sa.seed);
-        const uint4 v = *reinterpret_cast<const uint4*>(&rsect[scale64(word64(r), len)]);
+    const uint32_t len = (uint32_t)(min(a.A_size, start + (uint64_t)a.SS) - start);
+    for (uint32_t s = threadIdx.x; s < len; s += blockDim.x) {
+        const uint4 v = *reinterpret_cast<const uint4*>(&a.A[start + s]);
         const double acc = __longlong_as_double(((long long)v.y << 32) | v.x);
-        ++tr;
-        if (!(coin53(r) > acc) || tr >= REJ_SECTIONED_MAX_TRIALS) {
-            emit(sa, g, (int32_t)v.z, csum);
-            t += blockDim.x;
-            tr = 0;
-        }
+        ulonglong2 e;
+        e.x = acc >= 1.0 ? ~0ull : ((uint64_t)(acc * 0x1.0p53) << 11) | 0x7FFull;
+        e.y = v.z;
+        rsect[s] = e;
     }
+    __syncthreads();
+    const uint64_t cnt = a.sec_counts[2 * k], end = a.sec_counts[2 * k + 1] + cnt;
+    uint64_t csum = 0;
+    // Runs of outputs that share the counter's high word (one, nearly always).
+    for (uint64_t b = end - cnt; b < end;) {
+        const uint32_t hi = (uint32_t)(b >> 32);
+        const PhiloxStream ps(hi, PURPOSE_REJ_SECTIONED, sa.seed);
+        const uint64_t seg_end = min(end, ((uint64_t)hi + 1) << 32);
+        // One trial per iteration; a lane whose trial accepts goes on to its
+        // next sample at once, so no lane waits for another lane's rejected
+        // trials (the trials of every sample are those of the
+        // one-sample-at-a-time loop).
+        uint32_t left = (uint32_t)((seg_end - b + REJ_SEC_THREADS - 1 - threadIdx.x) / REJ_SEC_THREADS);
+        uint32_t t = threadIdx.x, tr = 0;
+        while (left != 0) {
+            const u32x4 r = ps.at((uint32_t)b + t, tr);
+            const ulonglong2 v = rsect[scale64(word64(r), len)];
+            ++tr;
+            if (coin64(r) <= v.x || tr >= REJ_SECTIONED_MAX_TRIALS) {
+                const int32_t item = (int32_t)v.y;
+                if (sa.out) (sa.out + b)[t] = item;
+                if (CACHED) hc.add(sa.hist, item);
+                if (sa.checksum) csum += (uint64_t)(uint32_t)item;
+                t += REJ_SEC_THREADS;
+                tr = 0;
+                --left;
+            }
+        }
+        b = seg_end;
+    }
+    if (CACHED) hc.flush(sa.hist);
     flush_checksum(sa, csum);
 }
 
@@ -699,20 +885,57 @@ hipError_t launch_sample_basic(const SampleArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_sample_sectioned(const SampleArgs& a, hipStream_t s) {
-    const size_t lds = (size_t)a.SS * sizeof(Row);
-    hipLaunchKernelGGL(section_counts, dim3((unsigned)((a.nsec + 63) / 64)), dim3(64), 0, s, a);
-    if (a.rows) hipLaunchKernelGGL(sample_sectioned<true>, dim3((unsigned)a.nsec), dim3(SECTIONED_THREADS), lds, s, a);
-    else hipLaunchKernelGGL(sample_sectioned<false>, dim3((unsigned)a.nsec), dim3(SECTIONED_THREADS), lds, s, a);
+// Up to one sample in kSparseRows rows, the drawn rows are read one by one: a
+// drawn row costs a 128-byte line of its eight rows (staged against read one
+// by one, us: 1e8 rows, n/16 samples 288 and 151, n/8 290 and 242, n/4 307
+// and 423; 2^20 rows, n/64 9.9 and 6.8, n/8 10.3 and 9.1, n/4 10.5 and 12.1).
+constexpr uint64_t kSparseRows = 8;
+// Sections whose counts the sampling waves find themselves: the descent takes
+// a wave about as long as one thread, so it pays while every section's wave
+// is resident at once.
+constexpr int64_t kSparseCounts = 4096;
+
+template <bool AOS>
+static void launch_sparse(const SampleArgs& a, hipStream_t s) {
+    const bool counts = a.nsec <= kSparseCounts;
+    if (!counts) hipLaunchKernelGGL(section_counts, dim3((unsigned)((a.nsec + 63) / 64)), dim3(64), 0, s, a);
+    if (a.hist && a.count >= 2 * (uint64_t)kHistMinPerBlock) {
+        const unsigned g = grid_for(min(a.count / kHistMinPerBlock, (uint64_t)(a.nsec + 7) / 8), 1, 256 * 4);
+        const dim3 b(kHistThreads);
+        if (counts) hipLaunchKernelGGL((sample_sectioned_sparse<AOS, true, true>), dim3(g), b, 0, s, a);
+        else hipLaunchKernelGGL((sample_sectioned_sparse<AOS, true, false>), dim3(g), b, 0, s, a);
+    } else {
+        const unsigned g = grid_for((uint64_t)a.nsec, 4, 256 * 8);
+        if (counts) hipLaunchKernelGGL((sample_sectioned_sparse<AOS, false, true>), dim3(g), dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((sample_sectioned_sparse<AOS, false, false>), dim3(g), dim3(256), 0, s, a);
+    }
+}
+
+// LDS of a block with a staged section of `rows` 16-byte rows (slots).
+static size_t sectioned_lds(int64_t rows, bool hist) { return (size_t)rows * sizeof(Row) + (hist ? 8 * kSecHistSlots : 0); }
+
+// A block per section with `lds` bytes; beyond 64 KB a kernel has to be
+// allowed its LDS first.
+template <typename... Args>
+static hipError_t launch_sectioned(void (*k)(Args...), int64_t nsec, int threads, size_t lds, hipStream_t s, Args... args) {
+    if (lds > 65536) {
+        const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(k, dim3((unsigned)nsec), dim3(threads), lds, s, args...);
     return hipGetLastError();
 }
 
-hipError_t set_sample_lds_limit(int bytes) {
-    hipError_t e = hipFuncSetAttribute((const void*)sample_sectioned<true>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e != hipSuccess) return e;
-    return hipFuncSetAttribute((const void*)sample_sectioned<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               bytes);
+hipError_t launch_sample_sectioned(const SampleArgs& a, hipStream_t s) {
+    if (a.count <= (uint64_t)a.n / kSparseRows) {
+        if (a.rows) launch_sparse<true>(a, s);
+        else launch_sparse<false>(a, s);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(section_counts, dim3((unsigned)((a.nsec + 63) / 64)), dim3(64), 0, s, a);
+    void (*k)(SampleArgs) = a.rows ? (a.hist ? sample_sectioned<true, true> : sample_sectioned<true, false>)
+                                   : (a.hist ? sample_sectioned<false, true> : sample_sectioned<false, false>);
+    return launch_sectioned(k, a.nsec, SECTIONED_THREADS, sectioned_lds(a.SS, a.hist != nullptr), s, a);
 }
 
 // rej_fill adds the long runs' tasks to a counter that the scan of the block
@@ -759,13 +982,8 @@ hipError_t launch_rejection_sample_sectioned(const RejSecArgs& a, const SampleAr
         hipLaunchKernelGGL(rej_mass_scan, dim3(1), dim3(1024), 0, s, a);
     }
     hipLaunchKernelGGL(rej_section_counts, dim3((unsigned)((a.nsec + 63) / 64)), dim3(64), 0, s, a, sa.count, sa.seed);
-    const size_t lds = (size_t)a.SS * sizeof(RejEntry);
-    hipLaunchKernelGGL(rej_sample_sectioned, dim3((unsigned)a.nsec), dim3(REJ_SEC_THREADS), lds, s, a, sa);
-    return hipGetLastError();
-}
-
-hipError_t set_rej_sample_lds_limit(int bytes) {
-    return hipFuncSetAttribute((const void*)rej_sample_sectioned, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    return launch_sectioned(sa.hist ? rej_sample_sectioned<true> : rej_sample_sectioned<false>, a.nsec, REJ_SEC_THREADS,
+                            sectioned_lds(a.SS, sa.hist != nullptr), s, a, sa);
 }
 
 hipError_t launch_rejection_sample(const RejArgs& a, const SampleArgs& sa, hipStream_t s) {

@@ -38,3 +38,31 @@ def test_histogram_counts_the_output(gpu, kind, n, dist, count):
     # The histogram alone: the same counts on top.
     draw(count, 77, hist=hist)
     np.testing.assert_array_equal(hist.cpu().numpy() - 1, 2 * np.bincount(got, minlength=n))
+
+
+@pytest.mark.parametrize("layout", ["aos", "soa"])
+@pytest.mark.parametrize("n,rows,count", [
+    (100_003, 4096, 12_500),       # n / 8 samples: the most that read their rows one by one
+    (100_003, 4096, 12_501),       # staged sections
+    (100_003, 64, 5_000),          # sections of a row count below a wave's lanes, a few samples each
+    (1, 4096, 0), (9, 4096, 1),    # one section: no descent
+    (1_000_003, 200, 125_000),     # 5,001 sections: their counts from a launch of their own
+    (800_000, 200, 100_000),       # 4,000 sections: counts by the sampling waves
+    (5_000_011, 4096, 33),         # at most 32 samples at every node of the descent
+    (3_000_000, 8192, 375_000),    # rounds of four full wave loads and a rest
+])
+def test_sparse_sections_match_oracle(gpu, oracle, layout, n, rows, count):
+    """Sectioned draws with few samples per row against the oracle's stream."""
+    torch = gpu
+    w = atg.generate_weights("pareto", n, seed=9, param=1.1)
+    t = atg.Table(n, layout=layout)
+    t.set_weights(w)
+    t.build()
+    tw, ta = t.table()
+    out = torch.full((max(count, 1),), -7, dtype=torch.int32, device="cuda")
+    hist = torch.zeros(n, dtype=torch.int32, device="cuda")
+    t.sample(count, 31, section_rows=rows, out=out)
+    exp = oracle.sample_sectioned(tw, ta, t.stats()["W_N"], rows, count, 31) if count else np.empty(0, np.int32)
+    np.testing.assert_array_equal(out.cpu().numpy()[:count], exp)
+    t.sample(count, 31, section_rows=rows, hist=hist)
+    np.testing.assert_array_equal(hist.cpu().numpy(), np.bincount(exp, minlength=n))
