@@ -288,8 +288,6 @@ atg_status atg_create(atg_table** out, int64_t n, atg_dtype dtype, atg_layout la
     ALLOC(t->d_sec_counts, 2 * t->sec_counts_cap);
 #undef ALLOC
     if (hipMemset(t->d_state, 0, sizeof(DevState)) != hipSuccess) return cleanup(fail(ATG_EDEVICE, "memset"));
-    if (set_partition_lds_limit(psa_lds_bytes(t->Ls)) != hipSuccess)
-        return cleanup(fail(ATG_EDEVICE, "partition LDS limit"));
     if (o.record_phases) {
         for (auto& e : t->ev)
             if (hipEventCreate(&e) != hipSuccess) return cleanup(fail(ATG_EDEVICE, "hipEventCreate"));

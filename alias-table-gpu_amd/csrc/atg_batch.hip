@@ -96,7 +96,7 @@ __global__ __launch_bounds__(256) void seg_sum_finish(SegArgs g, SegMap m) {
 
 // Sections of all tables, grid-stride over the phase's blocks (one section
 // each); a wave loads its next section while the current one's chains run.
-template <typename T>
+template <typename T, bool ROWS_LATER>
 __global__ __launch_bounds__(64) void seg_local(SegArgs g, SegMap m) {
     extern __shared__ double lds_raw[];
     const int lane = (int)threadIdx.x;
@@ -118,7 +118,7 @@ __global__ __launch_bounds__(64) void seg_local(SegArgs g, SegMap m) {
             next();
             continue;
         }
-        psa_section<T, true>(a, v - m.base[t], x, lds_raw, lane, next);
+        psa_section<T, true, PSA_MAX_LEN / 64, ROWS_LATER>(a, v - m.base[t], x, lds_raw, lane, next);
     }
 }
 
@@ -301,7 +301,7 @@ hipError_t launch_batch(const atg_batch* b, hipStream_t s) {
     hipLaunchKernelGGL(seg_reset_ticks, dim3((unsigned)std::min<int64_t>((b->ntables + 255) / 256, 4096)), dim3(256),
                        0, s, g);
     const size_t lds = psa_lds_bytes(b->Ls_max);
-    const int64_t resident = resident_blocks((const void*)seg_local<T>, 64, lds);
+    const int64_t resident = resident_blocks((const void*)seg_local<T, true>, 64, lds);
     const bool learned = b->opts.split_method == ATG_SPLIT_LEARNED;
     for (const BatchGroup& grp : b->groups) {
         const SegMap* M = grp.maps;
@@ -310,8 +310,10 @@ hipError_t launch_batch(const atg_batch* b, hipStream_t s) {
         // has no tree blocks).
         hipLaunchKernelGGL(seg_sum<T>, grid(M[MAP_SUM]), dim3(256), 0, s, g, M[MAP_SUM]);
         hipLaunchKernelGGL(seg_sum_finish, grid(M[MAP_ONE]), dim3(256), 0, s, g, M[MAP_ONE]);
-        hipLaunchKernelGGL(seg_local<T>, dim3((unsigned)std::min<int64_t>(M[MAP_LOCAL].blocks, resident)), dim3(64),
-                           lds, s, g, M[MAP_LOCAL]);
+        const bool later = rows_later_ok(M[MAP_LOCAL].blocks, resident);
+        hipLaunchKernelGGL((later ? seg_local<T, true> : seg_local<T, false>),
+                           dim3((unsigned)std::min<int64_t>(M[MAP_LOCAL].blocks, resident)), dim3(64), lds, s, g,
+                           M[MAP_LOCAL]);
         if (M[MAP_TREE].blocks > 0)
             for (int b0 = 0; (grp.G_max >> b0) > 1; b0 += 9)
                 hipLaunchKernelGGL(seg_tree, grid(M[MAP_TREE]), dim3(256), 0, s, g, M[MAP_TREE], b0);
@@ -570,10 +572,6 @@ atg_status atg_batch_create(atg_batch** out, const int64_t* offsets, int64_t nta
         hipMemset(b->d_state, 0, sizeof(BatchState) * ntables) != hipSuccess ||
         hipMemset(b->d_ticks, 0, sizeof(uint64_t) * 2 * ntables) != hipSuccess)
         return cleanup(fail(ATG_EDEVICE, "atg_batch_create: upload failed"));
-    const size_t lds = psa_lds_bytes(b->Ls_max);
-    const void* fn = dtype == ATG_F32 ? (const void*)seg_local<float> : (const void*)seg_local<double>;
-    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-        return cleanup(fail(ATG_EDEVICE, "atg_batch_create: LDS limit of %zu bytes", lds));
     int khz = 0;
     if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, b->device) == hipSuccess && khz > 0)
         b->wall_khz = khz;

@@ -103,10 +103,21 @@ inline int32_t learned_knots(int32_t opt, int64_t p_req) {
     return (int32_t)(k < opt ? k : opt);
 }
 
-size_t psa_lds_bytes(int64_t Ls_max);
+// LDS of one partition wave: weights (8 B) and local item indices (2 B), and
+// at least eight weights to read past the last.
+inline size_t psa_lds_bytes(int64_t Ls_max) {
+    const size_t need = (size_t)Ls_max * 10, past = ((size_t)Ls_max + 8) * 8;
+    return ((need > past ? need : past) + 15) & ~(size_t)15;
+}
+// Rows written after the chains rather than by each of their steps: pays
+// where the device is full of sections and HBM is what counts (1e8 items at
+// sections of 2048: the pass takes 0.74 against 0.82 ms; uniform weights at
+// sections of 1000: 0.74 against 1.12), costs the extra pass over the section
+// where each has a wave to itself from the start (101 sections: 21 against 18
+// us; 1,049 sections: the same).
+inline bool rows_later_ok(int64_t sections, int64_t resident) { return sections > resident; }
 int64_t resident_blocks(const void* f, int threads, size_t lds);
 int64_t block_tree_total(int64_t G);
-hipError_t set_partition_lds_limit(size_t bytes);
 hipError_t launch_sum(const BuildArgs& a, hipStream_t s);
 hipError_t launch_partition(const BuildArgs& a, hipStream_t s);
 hipError_t launch_partition_local(const BuildArgs& a, hipStream_t s);

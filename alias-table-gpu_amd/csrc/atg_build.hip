@@ -40,7 +40,7 @@ __global__ __launch_bounds__(1024) void sum_finish(BuildArgs a) {
 // ... and loads each next section while the current one's chains run.
 // XU: weights per lane held for a section (sections of up to 64 XU items);
 // the short-section kernel keeps fewer registers, so more waves fit a SIMD.
-template <typename T, bool AOS, int XU>
+template <typename T, bool AOS, int XU, bool ROWS_LATER>
 __global__ __launch_bounds__(64) void partition_local(BuildArgs a) {
     extern __shared__ double lds_raw[];
     if (a.st->error) return;
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(64) void partition_local(BuildArgs a) {
     if (s < a.G) section_load<T>(a, s, lane, x);
     for (; s < a.G; s += gridDim.x) {
         const int64_t sn = s + gridDim.x;
-        psa_section<T, AOS>(a, s, x, lds_raw, lane, [&]() {
+        psa_section<T, AOS, XU, ROWS_LATER>(a, s, x, lds_raw, lane, [&]() {
             if (sn < a.G) section_load<T>(a, sn, lane, x);
         });
     }
@@ -262,7 +262,6 @@ hipError_t launch_sum(const BuildArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// LDS of one partition wave: weights (8 B) and local item indices (2 B).
 // Workgroups of `threads` threads and `lds` bytes of dynamic LDS of kernel f
 // that the device holds at once.
 int64_t resident_blocks(const void* f, int threads, size_t lds) {
@@ -275,8 +274,6 @@ int64_t resident_blocks(const void* f, int threads, size_t lds) {
     return (int64_t)cus * per;
 }
 
-size_t psa_lds_bytes(int64_t Ls_max) { return (((size_t)Ls_max * 10) + 15) & ~(size_t)15; }
-
 int64_t block_tree_total(int64_t G) {
     int64_t total = 0;
     for (int b = 0; ((int64_t)1 << b) <= G; ++b) total += G >> b;
@@ -286,20 +283,23 @@ int64_t block_tree_total(int64_t G) {
 // The partition phase in its two passes: the local pass (partition, PSA+
 // chains, staged leftovers, level-0 block sums), then the block tree and the
 // placement of the leftover lists (and the split certificate).
+template <bool ROWS_LATER>
 static void (*partition_local_kernel(bool f32, bool aos, int64_t Ls_max))(BuildArgs) {
     constexpr int S = kShortSectionMax / 64, L = PSA_MAX_LEN / 64;
     if (Ls_max <= kShortSectionMax)
-        return f32 ? (aos ? partition_local<float, true, S> : partition_local<float, false, S>)
-                   : (aos ? partition_local<double, true, S> : partition_local<double, false, S>);
-    return f32 ? (aos ? partition_local<float, true, L> : partition_local<float, false, L>)
-               : (aos ? partition_local<double, true, L> : partition_local<double, false, L>);
+        return f32 ? (aos ? partition_local<float, true, S, ROWS_LATER> : partition_local<float, false, S, ROWS_LATER>)
+                   : (aos ? partition_local<double, true, S, ROWS_LATER> : partition_local<double, false, S, ROWS_LATER>);
+    return f32 ? (aos ? partition_local<float, true, L, ROWS_LATER> : partition_local<float, false, L, ROWS_LATER>)
+               : (aos ? partition_local<double, true, L, ROWS_LATER> : partition_local<double, false, L, ROWS_LATER>);
 }
 
 hipError_t launch_partition_local(const BuildArgs& a, hipStream_t s) {
     const size_t lds = psa_lds_bytes(a.Ls_max);
-    void (*k)(BuildArgs) = partition_local_kernel(a.dtype_f32 != 0, a.rows != nullptr, a.Ls_max);
-    const dim3 g((unsigned)std::min<int64_t>(a.G, resident_blocks((const void*)k, 64, lds)));
-    hipLaunchKernelGGL(k, g, dim3(64), lds, s, a);
+    const bool f32 = a.dtype_f32 != 0, aos = a.rows != nullptr;
+    void (*k)(BuildArgs) = partition_local_kernel<true>(f32, aos, a.Ls_max);
+    const int64_t resident = resident_blocks((const void*)k, 64, lds);
+    if (!rows_later_ok(a.G, resident)) k = partition_local_kernel<false>(f32, aos, a.Ls_max);
+    hipLaunchKernelGGL(k, dim3((unsigned)std::min<int64_t>(a.G, resident)), dim3(64), lds, s, a);
     return hipGetLastError();
 }
 
@@ -406,19 +406,6 @@ hipError_t launch_join_rows(const double* w, const int32_t* al, Row* rows, int64
     const int64_t g = std::min<int64_t>((n + 255) / 256, 8192);
     hipLaunchKernelGGL(join_rows, dim3(g > 0 ? g : 1), dim3(256), 0, s, w, al, rows, n);
     return hipGetLastError();
-}
-
-hipError_t set_partition_lds_limit(size_t bytes) {
-    constexpr int S = kShortSectionMax / 64, L = PSA_MAX_LEN / 64;
-    const void* fns[] = {(const void*)partition_local<double, true, L>, (const void*)partition_local<double, false, L>,
-                         (const void*)partition_local<float, true, L>, (const void*)partition_local<float, false, L>,
-                         (const void*)partition_local<double, true, S>, (const void*)partition_local<double, false, S>,
-                         (const void*)partition_local<float, true, S>, (const void*)partition_local<float, false, S>};
-    for (const void* f : fns) {
-        hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
 }
 
 }  // namespace atg

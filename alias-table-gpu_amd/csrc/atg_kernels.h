@@ -76,6 +76,18 @@ __device__ __forceinline__ double section_sum(const T* w, int64_t start, int64_t
 // Sections of at most this many items run the partition kernel that holds
 // half the weight registers.
 constexpr int64_t kShortSectionMax = 1024;
+// Lights of a chain a partition wave looks at together (2, 3, 6 and 8 were no
+// faster over Pareto, exponential, uniform and Zipf weights).
+constexpr int kRun = 4;
+// A section with at least one row in kWholeRows from its chains writes all its
+// rows: at 1e8 FP64 uniform weights (sections of 1000, six rows in ten from
+// the chains) the pass takes 0.75 ms whole and 0.90 ms in pieces, at 1% heavy
+// weights with 90% of the mass (one row in ten) 0.82 ms whole, 0.53 in pieces.
+constexpr int kWholeRows = 4;
+// Chunks of 64 rows a wave assembles at once: four, eight where the registers
+// of FP32 weights leave room.
+template <typename T, int XU>
+constexpr int row_chunks() { return sizeof(T) == 4 && XU == PSA_MAX_LEN / 64 ? 8 : 4; }
 // Chunks of 64 leftovers a wave keeps in flight at once when staging or
 // placing them.
 #define PLACE_GROUP 8
@@ -87,7 +99,8 @@ template <bool LEAN>
 constexpr int place_chunks() { return LEAN ? 4 : 8; }
 
 struct SecLDS {
-    double* w;      // [Ls]: lights from the front, heavies from the back
+    double* w;      // [Ls]: lights from the front, heavies from the back (before idx, so that
+                    // the up to kRun weights read past a chain's last light are LDS of its own)
     uint16_t* idx;  // [Ls]: local item index
     int len;
     __device__ double& Lw(int i) { return w[i]; }
@@ -294,7 +307,9 @@ __device__ __forceinline__ void stage_chunks(const BuildArgs& a, SecLDS& L, bool
 // aggregates (stored as the level-0 block of the dyadic section tree) and the
 // leftovers staged in rank order at the section's own range (lights, then
 // heavies).  Nothing here waits for another section's work.
-template <typename T, bool AOS, int XU, typename AfterPartition>
+// ROWS_LATER: the chains record their steps and the wave writes the rows
+// afterwards (rows_later_ok says when).
+template <typename T, bool AOS, int XU, bool ROWS_LATER, typename AfterPartition>
 __device__ __forceinline__ void psa_section(const BuildArgs& a, int64_t s, T (&x)[XU],
                                             double* lds_raw, int lane, AfterPartition after_partition) {
     DevState* st = a.st;
@@ -314,6 +329,7 @@ __device__ __forceinline__ void psa_section(const BuildArgs& a, int64_t s, T (&x
     // store the chains issued by then.
     __builtin_amdgcn_s_waitcnt(0x0F70);
     int nL = 0, nH = 0;
+    uint64_t lights = 0ull;  // lane u: the lights of chunk u
 #pragma unroll
     for (int u = 0; u < XU; ++u) {
         const int k = (u << 6) + lane;
@@ -331,23 +347,20 @@ __device__ __forceinline__ void psa_section(const BuildArgs& a, int64_t s, T (&x
             const int c = __popcll(bl);
             nL += c;
             nH += 64 - c;
+            if (ROWS_LATER) lights = lane == u ? bl : lights;
         } else if ((u << 6) < len) {
             const bool valid = k < len;
             const double xv = (double)x[u];
             const bool light = valid && xv <= W_N, heavy = valid && !(xv <= W_N);
             const uint64_t bl = __ballot(light), bh = __ballot(heavy);
-            if (light) {
-                const int pos = nL + __popcll(bl & lt);
-                L.Lw(pos) = xv;
-                L.Li(pos) = (uint16_t)k;
-            }
-            if (heavy) {
-                const int pos = nH + __popcll(bh & lt);
-                L.Hw(pos) = xv;
-                L.Hi(pos) = (uint16_t)k;
+            const int slot = light ? nL + __popcll(bl & lt) : len - 1 - (nH + __popcll(bh & lt));
+            if (valid) {
+                L.w[slot] = xv;
+                L.idx[slot] = (uint16_t)k;
             }
             nL += __popcll(bl);
             nH += __popcll(bh);
+            if (ROWS_LATER) lights = lane == u ? bl : lights;
         }
     }
     wave_lds_sync();
@@ -363,54 +376,194 @@ __device__ __forceinline__ void psa_section(const BuildArgs& a, int64_t s, T (&x
             iLo = t * stepsL; iHi = (t == C - 1) ? nL : (t + 1) * stepsL;
             jLo = t * stepsH; jHi = (t == C - 1) ? nH : (t + 1) * stepsH;
         }
-        if (t < C && iHi - iLo > 0 && jHi - jLo > 0) {
-            // Registers hold the chain's current heavy (residual wc, item hj),
-            // the next heavy (hw1, hi1) and the current light (lw, li); a step
-            // stores one row and reads the light and the next heavy at its
-            // new indices for the following step.
-            // The loop is one straight run of instructions besides its exit.
-            // Lights and heavies share one LDS array (heavy j at len-1-j).
-            // The next heavy j + 1 <= jHi <= nH sits at slot hn = len - 2 - j
-            // >= nL - 1 >= 0 (the chain has a light); past the chain's range
-            // it is read but never used.  The exit test is lane-mask logic.
+        const bool mine = t < C && iHi - iLo > 0 && jHi - jLo > 0;
+        if (ROWS_LATER) {
+            // A chain's step consumes the current heavy (its bucket is full: a
+            // row of the heavy, aliased to the next one) or the current light (a
+            // row of the light, aliased to the heavy).  The steps only record
+            // which, one bit a step, and the residual of the heavy in its slot;
+            // the rows are written afterwards by the whole wave.  A wave is alone
+            // or nearly so on its SIMD (LDS), so a step costs its instructions'
+            // latencies one after the other: the chains look at kRun lights at
+            // once and take as many as the bucket holds.
+            // A section whose chains consumed a large part of it writes all its
+            // rows in item order, the left-over ones too (the pack writes those
+            // again): rows written in pieces cost a read and a write of their
+            // lines in HBM, whole lines a write.  Below one row in kWholeRows the
+            // rows go out chain by chain.
+            // Lights and heavies share one LDS array (heavy j at len-1-j).  The
+            // next heavy j + 1 <= jHi <= nH sits at slot hn = len - 2 - j >= nL -
+            // 1 >= 0 (the chain has a light); past the chain's range it is read
+            // but never used.
             int i = iLo, hn = len - 2 - jLo;
-            double wc = L.Hw(jLo);
-            int hj = L.Hi(jLo);
-            double lw = L.Lw(i);
-            int li = L.Li(i);
-            double hw1 = L.w[hn];
-            int hi1 = L.idx[hn];
+            double wc = mine ? L.w[hn + 1] : 0.0;
             const double thr = W_N + ATG_EPSILON;
             const int iEnd = iHi - 1, hnEnd = len - 1 - jHi;
-            while (true) {
-                // Full bucket: the heavy's row, then the next heavy; else the
-                // light's row.  A step needs a further element on its side.
-                const bool ex = wc <= thr;
-                const uint64_t mEx = __ballot(ex), mH = __ballot(hn <= hnEnd), mL = __ballot(i >= iEnd);
-                if (__builtin_amdgcn_inverse_ballot_w64((mEx & mH) | (~mEx & mL))) break;
-                store_row<AOS>(a, start + (ex ? hj : li), ex ? wc : lw, (int32_t)(start + (ex ? hi1 : hj)));
-                wc += (ex ? hw1 : lw) - W_N;
-                hj = ex ? hi1 : hj;
-                hn -= (int)ex;
-                i += (int)!ex;
-                lw = L.Lw(i);
-                li = L.Li(i);
-                hw1 = L.w[hn];
-                hi1 = L.idx[hn];
+            bool done = !mine;
+            int whole = -1;  // whether the section's rows are written whole; not known yet
+            // Episodes of up to 64 steps a chain, their bits in one register pair.
+            while (__ballot(!done) != 0ull) {
+                const int i0 = i, hn0 = hn;
+                uint64_t bits = 0ull;
+                if (!done) {
+                    double l[kRun], h;
+#pragma unroll
+                    for (int q = 0; q < kRun; ++q) l[q] = L.w[i + q];
+                    h = L.w[hn];
+                    while (true) {
+                        // The residuals after 0, 1, ... of the next lights, and
+                        // how many are taken: up to the first that fills the
+                        // bucket, as far as the chain has lights.
+                        double v[kRun + 1];
+                        v[0] = wc;
+#pragma unroll
+                        for (int q = 0; q < kRun; ++q) v[q + 1] = v[q] + (l[q] - W_N);
+                        int k = kRun;
+#pragma unroll
+                        for (int q = kRun - 1; q >= 0; --q) k = v[q] <= thr ? q : k;
+                        const int avail = iEnd - i;
+                        const bool full = k < kRun && k <= avail;  // a heavy step follows
+                        const bool lacks = full ? hn <= hnEnd : k > avail;
+                        k = min(k, avail);
+                        wc = v[0];
+#pragma unroll
+                        for (int q = 1; q <= kRun; ++q) wc = k >= q ? v[q] : wc;
+                        L.w[hn + 1] = wc;
+                        i += k;
+                        done = lacks;
+                        if (full && !lacks) {
+                            bits |= 1ull << (uint32_t)(i - i0 + hn0 - hn);
+                            wc += h - W_N;
+                            --hn;
+                        }
+                        if (lacks || i - i0 + hn0 - hn > 63 - kRun) break;
+#pragma unroll
+                        for (int q = 0; q < kRun; ++q) l[q] = L.w[i + q];
+                        h = L.w[hn];
+                    }
+                }
+                const int ni = i - i0, nj = hn0 - hn;  // steps of each kind
+                if (whole < 0) {
+                    const uint32_t taken = wave_incl_scan_u32((uint32_t)(ni + nj));
+                    whole = kWholeRows * __builtin_amdgcn_readlane((int)taken, 63) >= len ? 1 : 0;
+                }
+                wave_lds_sync();
+                for (uint64_t todo = __ballot(ni + nj > 0); todo != 0ull; todo &= todo - 1) {
+                    const int c = __builtin_ctzll(todo);
+                    const uint64_t m = readlane_u64(bits, c);
+                    const int steps = __builtin_amdgcn_readlane(ni + nj, c);
+                    const int ci = __builtin_amdgcn_readlane(i0, c), ch = __builtin_amdgcn_readlane(hn0, c);
+                    if (lane < steps) {
+                        const int before = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                        const bool ex = __builtin_amdgcn_inverse_ballot_w64(m);
+                        const int hs = ch + 1 - before;  // the current heavy's slot
+                        const int slot = ex ? hs : ci + lane - before;
+                        const uint16_t alias = L.idx[ex ? hs - 1 : hs];
+                        // A slot's item is needed no more once its row is known:
+                        // a light's by its own row, a heavy's by its own and by
+                        // earlier steps.
+                        if (whole) L.idx[slot] = alias;
+                        else store_row<AOS>(a, start + L.idx[slot], L.w[slot], (int32_t)(start + alias));
+                    }
+                }
+                wave_lds_sync();
             }
-            const int j = len - 2 - hn;
-            // Remainder (PsaPlusNormal.cu:112-123): back to L when its
-            // residual is light and a consumed light slot can hold it,
-            // otherwise back to H in place.
-            if (wc <= thr && i > iLo) {
-                L.Lw(i - 1) = wc;
-                L.Li(i - 1) = (uint16_t)hj;
-                iLo = i - 1;
-                jLo = j + 1;
-            } else {
-                L.Hw(j) = wc;
-                iLo = i;
-                jLo = j;
+            if (whole > 0) {
+                constexpr int RC = row_chunks<T, XU>();
+                int rL = 0;  // lights before the chunk
+                for (int u0 = 0; (u0 << 6) < len; u0 += RC) {
+                    double rw[RC];
+                    int32_t ra[RC];
+#pragma unroll
+                    for (int q = 0; q < RC; ++q) {
+                        const int k0 = (u0 + q) << 6;
+                        const uint64_t bl = readlane_u64(lights, min(u0 + q, 63));
+                        const int before = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bl >> 32),
+                                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)bl, 0u));
+                        // The slots of the partition (a heavy's: len - 1 less the
+                        // heavies before it); lanes past the end read slot 0.
+                        const bool light = __builtin_amdgcn_inverse_ballot_w64(bl);
+                        int slot = before + (light ? rL : len - 1 - (k0 - rL) - lane);
+                        slot = k0 + lane < len ? slot : 0;
+                        rw[q] = L.w[slot];
+                        ra[q] = (int32_t)(start + L.idx[slot]);
+                        rL += __popcll(bl);
+                    }
+#pragma unroll
+                    for (int q = 0; q < RC; ++q) {
+                        const int k = ((u0 + q) << 6) + lane;
+                        if (k < len) store_row<AOS>(a, start + k, rw[q], ra[q]);
+                    }
+                }
+                wave_lds_sync();
+            }
+            if (mine) {
+                const int j = len - 2 - hn;
+                // Remainder (PsaPlusNormal.cu:112-123): back to L when its
+                // residual is light and a consumed light slot can hold it,
+                // otherwise back to H in place.
+                if (wc <= thr && i > iLo) {
+                    L.Lw(i - 1) = wc;
+                    L.Li(i - 1) = L.Hi(j);
+                    iLo = i - 1;
+                    jLo = j + 1;
+                } else {
+                    L.Hw(j) = wc;
+                    iLo = i;
+                    jLo = j;
+                }
+            }
+        } else {
+            if (mine) {
+                // Registers hold the chain's current heavy (residual wc, item hj),
+                // the next heavy (hw1, hi1) and the current light (lw, li); a step
+                // stores one row and reads the light and the next heavy at its
+                // new indices for the following step.
+                // The loop is one straight run of instructions besides its exit.
+                // Lights and heavies share one LDS array (heavy j at len-1-j).
+                // The next heavy j + 1 <= jHi <= nH sits at slot hn = len - 2 - j
+                // >= nL - 1 >= 0 (the chain has a light); past the chain's range
+                // it is read but never used.  The exit test is lane-mask logic.
+                int i = iLo, hn = len - 2 - jLo;
+                double wc = L.Hw(jLo);
+                int hj = L.Hi(jLo);
+                double lw = L.Lw(i);
+                int li = L.Li(i);
+                double hw1 = L.w[hn];
+                int hi1 = L.idx[hn];
+                const double thr = W_N + ATG_EPSILON;
+                const int iEnd = iHi - 1, hnEnd = len - 1 - jHi;
+                while (true) {
+                    // Full bucket: the heavy's row, then the next heavy; else the
+                    // light's row.  A step needs a further element on its side.
+                    const bool ex = wc <= thr;
+                    const uint64_t mEx = __ballot(ex), mH = __ballot(hn <= hnEnd), mL = __ballot(i >= iEnd);
+                    if (__builtin_amdgcn_inverse_ballot_w64((mEx & mH) | (~mEx & mL))) break;
+                    store_row<AOS>(a, start + (ex ? hj : li), ex ? wc : lw, (int32_t)(start + (ex ? hi1 : hj)));
+                    wc += (ex ? hw1 : lw) - W_N;
+                    hj = ex ? hi1 : hj;
+                    hn -= (int)ex;
+                    i += (int)!ex;
+                    lw = L.Lw(i);
+                    li = L.Li(i);
+                    hw1 = L.w[hn];
+                    hi1 = L.idx[hn];
+                }
+                const int j = len - 2 - hn;
+                // Remainder (PsaPlusNormal.cu:112-123): back to L when its
+                // residual is light and a consumed light slot can hold it,
+                // otherwise back to H in place.
+                if (wc <= thr && i > iLo) {
+                    L.Lw(i - 1) = wc;
+                    L.Li(i - 1) = (uint16_t)hj;
+                    iLo = i - 1;
+                    jLo = j + 1;
+                } else {
+                    L.Hw(j) = wc;
+                    iLo = i;
+                    jLo = j;
+                }
             }
         }
     } else if (lane == 0) {

@@ -153,7 +153,6 @@ extern "C" atg_status atg_build_noalloc(const void* weights, atg_dtype dtype, in
     a.pack_method = o.pack_method;
 
     hipStream_t s = (hipStream_t)stream;
-    HIPCHK(set_partition_lds_limit(psa_lds_bytes(Ls)));
     hipLaunchKernelGGL(clear_state, dim3(1), dim3(64), 0, s, a.st);
     HIPCHK(hipGetLastError());
     HIPCHK(launch_sum(a, s));
