@@ -72,6 +72,7 @@ struct atg_table_s {
     uint32_t* d_sec_loff = nullptr;  // lean light lists: lights before each section
     uint32_t* d_sec_ldir = nullptr;  // lean light lists: the section of every 1024th light
     bool placed = false;             // the staging and sec_loff of the last partition are current
+    bool lists_full = false;         // the last build left whole lists (no staging): a one-launch build
     double* d_stage_w = nullptr;
     int32_t* d_stage_i = nullptr;
     int32_t *d_Li = nullptr, *d_Hi = nullptr;
@@ -155,7 +156,7 @@ struct atg_table_s {
         a.pack_method = opts.pack_method;
         a.sec_loff = d_sec_loff;
         a.sec_ldir = d_sec_ldir;
-        a.lean_lights = d_sec_loff && d_sec_ldir && lean_lights_ok(n, p_req, opts.pack_method) ? 1 : 0;
+        a.lean_lights = d_sec_loff && d_sec_ldir && !lists_full && lean_lights_ok(n, p_req, opts.pack_method) ? 1 : 0;
         return a;
     }
 };
@@ -340,6 +341,8 @@ atg_status atg_build_phase(atg_table* t, int32_t phase, void* stream) {
     if (!t->weights_set) return fail(ATG_ESTATE, "atg_build_phase: weights not set");
     hipStream_t s = (hipStream_t)stream;
     t->last_stream = s;
+    if (phase == ATG_PHASE_PARTITION || phase == ATG_PHASE_PARTITION_LOCAL || phase == ATG_PHASE_PARTITION_PLACE)
+        t->lists_full = false;
     const BuildArgs a = t->args();
     switch (phase) {
         case ATG_PHASE_SUM: HIPCHK(launch_sum(a, s)); break;
@@ -405,7 +408,18 @@ atg_status atg_build(atg_table* t, void* stream) {
     if (!t->weights_set) return fail(ATG_ESTATE, "atg_build: weights not set");
     hipStream_t s = (hipStream_t)stream;
     t->last_stream = s;
+    // A small table in one launch.  Not where the phases are timed or overlapped
+    // on request, nor for the searches whose certificate the stats report.
+    if (t->opts.split_method == ATG_SPLIT_BISECT && !t->opts.interleave && !t->events &&
+        small_build_ok(t->n, t->G, t->Ls, t->p_req)) {
+        HIPCHK(launch_small(t->args(), true, nullptr, nullptr, s));
+        t->placed = false;
+        t->lists_full = true;
+        t->built = true;
+        return ATG_OK;
+    }
     if (t->opts.interleave && t->sp_stream && !t->events) {
+        t->lists_full = false;
         const BuildArgs a = t->args();
         HIPCHK(launch_sum(a, s));
         HIPCHK(launch_partition(a, s));

@@ -141,4 +141,18 @@ hipError_t launch_pack_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int
 hipError_t launch_split_rows(const Row* rows, double* w, int32_t* al, int64_t n, hipStream_t s);
 hipError_t launch_join_rows(const double* w, const int32_t* al, Row* rows, int64_t n, hipStream_t s);
 
+
+// A whole build by one workgroup with its lists in LDS (atg_small.h): the
+// state, rows, splits and (with lists) the leftover lists that the phases
+// above leave, in one launch.  W_out, error_out: nullable device copies.
+constexpr int kSmallMaxWaves = 16;  // waves of a workgroup, one per section: sections of up to 1024 items
+constexpr int kSmallLongWaves = 4;  // longer ones
+#ifndef SMALLMAX
+#define SMALLMAX 8192
+#endif
+constexpr int64_t kSmallMaxItems = SMALLMAX;
+constexpr size_t kSmallLdsMax = 156 * 1024;  // of 160 KB, static LDS aside
+bool small_build_ok(int64_t n, int64_t G, int64_t Ls, int64_t p_req);
+hipError_t launch_small(const BuildArgs& a, bool lists, double* W_out, uint32_t* error_out, hipStream_t s);
+
 }  // namespace atg

@@ -300,6 +300,76 @@ __device__ __forceinline__ void stage_chunks(const BuildArgs& a, SecLDS& L, bool
         if (g0 + 64 * u < m) agg = agg + readlane_d(t8, u);
 }
 
+// Count slices of a section's nL lights and nH heavies, lane t's for chain t
+// (empty from the chain count on).
+__device__ __forceinline__ void chain_ranges(int C, int nL, int nH, int t, int& iLo, int& iHi, int& jLo, int& jHi) {
+    iLo = iHi = jLo = jHi = 0;
+    if (t < C) {
+        const int stepsL = nL / C, stepsH = nH / C;
+        iLo = t * stepsL; iHi = (t == C - 1) ? nL : (t + 1) * stepsL;
+        jLo = t * stepsH; jHi = (t == C - 1) ? nH : (t + 1) * stepsH;
+    }
+}
+
+// The greedy chains of a section (PsaPlusNormal.cu:51-123), lane t its own
+// chain over lights [iLo, iHi) and heavies [jLo, jHi) of L, each step storing
+// its row; iLo and jLo come back past what the chain consumed.
+template <bool AOS>
+__device__ __forceinline__ void psa_chain_rows(const BuildArgs& a, SecLDS& L, int64_t start, double W_N,
+                                               bool mine, int& iLo, int iHi, int& jLo, int jHi) {
+    const int len = L.len;
+    if (mine) {
+        // Registers hold the chain's current heavy (residual wc, item hj),
+        // the next heavy (hw1, hi1) and the current light (lw, li); a step
+        // stores one row and reads the light and the next heavy at its
+        // new indices for the following step.
+        // The loop is one straight run of instructions besides its exit.
+        // Lights and heavies share one LDS array (heavy j at len-1-j).
+        // The next heavy j + 1 <= jHi <= nH sits at slot hn = len - 2 - j
+        // >= nL - 1 >= 0 (the chain has a light); past the chain's range
+        // it is read but never used.  The exit test is lane-mask logic.
+        int i = iLo, hn = len - 2 - jLo;
+        double wc = L.Hw(jLo);
+        int hj = L.Hi(jLo);
+        double lw = L.Lw(i);
+        int li = L.Li(i);
+        double hw1 = L.w[hn];
+        int hi1 = L.idx[hn];
+        const double thr = W_N + ATG_EPSILON;
+        const int iEnd = iHi - 1, hnEnd = len - 1 - jHi;
+        while (true) {
+            // Full bucket: the heavy's row, then the next heavy; else the
+            // light's row.  A step needs a further element on its side.
+            const bool ex = wc <= thr;
+            const uint64_t mEx = __ballot(ex), mH = __ballot(hn <= hnEnd), mL = __ballot(i >= iEnd);
+            if (__builtin_amdgcn_inverse_ballot_w64((mEx & mH) | (~mEx & mL))) break;
+            store_row<AOS>(a, start + (ex ? hj : li), ex ? wc : lw, (int32_t)(start + (ex ? hi1 : hj)));
+            wc += (ex ? hw1 : lw) - W_N;
+            hj = ex ? hi1 : hj;
+            hn -= (int)ex;
+            i += (int)!ex;
+            lw = L.Lw(i);
+            li = L.Li(i);
+            hw1 = L.w[hn];
+            hi1 = L.idx[hn];
+        }
+        const int j = len - 2 - hn;
+        // Remainder (PsaPlusNormal.cu:112-123): back to L when its
+        // residual is light and a consumed light slot can hold it,
+        // otherwise back to H in place.
+        if (wc <= thr && i > iLo) {
+            L.Lw(i - 1) = wc;
+            L.Li(i - 1) = (uint16_t)hj;
+            iLo = i - 1;
+            jLo = j + 1;
+        } else {
+            L.Hw(j) = wc;
+            iLo = i;
+            jLo = j;
+        }
+    }
+}
+
 // Partition pass 1, section s by one wave, its weights in x (section_load):
 // stable light/heavy partition into LDS, then after_partition() (x is free
 // from there on: the caller loads its next section into it), PSA+ greedy
@@ -369,14 +439,8 @@ __device__ __forceinline__ void psa_section(const BuildArgs& a, int64_t s, T (&x
     int iLo = 0, iHi = 0, jLo = 0, jHi = 0;
     if (a.psa_plus) {
         // Greedy chains (PsaPlusNormal.cu:51-123), lane t runs chain t.
-        const int C = a.chains;
-        const int t = lane;
-        if (t < C) {
-            const int stepsL = nL / C, stepsH = nH / C;
-            iLo = t * stepsL; iHi = (t == C - 1) ? nL : (t + 1) * stepsL;
-            jLo = t * stepsH; jHi = (t == C - 1) ? nH : (t + 1) * stepsH;
-        }
-        const bool mine = t < C && iHi - iLo > 0 && jHi - jLo > 0;
+        chain_ranges(a.chains, nL, nH, lane, iLo, iHi, jLo, jHi);
+        const bool mine = iHi - iLo > 0 && jHi - jLo > 0;
         if (ROWS_LATER) {
             // A chain's step consumes the current heavy (its bucket is full: a
             // row of the heavy, aliased to the next one) or the current light (a
@@ -515,56 +579,7 @@ __device__ __forceinline__ void psa_section(const BuildArgs& a, int64_t s, T (&x
                 }
             }
         } else {
-            if (mine) {
-                // Registers hold the chain's current heavy (residual wc, item hj),
-                // the next heavy (hw1, hi1) and the current light (lw, li); a step
-                // stores one row and reads the light and the next heavy at its
-                // new indices for the following step.
-                // The loop is one straight run of instructions besides its exit.
-                // Lights and heavies share one LDS array (heavy j at len-1-j).
-                // The next heavy j + 1 <= jHi <= nH sits at slot hn = len - 2 - j
-                // >= nL - 1 >= 0 (the chain has a light); past the chain's range
-                // it is read but never used.  The exit test is lane-mask logic.
-                int i = iLo, hn = len - 2 - jLo;
-                double wc = L.Hw(jLo);
-                int hj = L.Hi(jLo);
-                double lw = L.Lw(i);
-                int li = L.Li(i);
-                double hw1 = L.w[hn];
-                int hi1 = L.idx[hn];
-                const double thr = W_N + ATG_EPSILON;
-                const int iEnd = iHi - 1, hnEnd = len - 1 - jHi;
-                while (true) {
-                    // Full bucket: the heavy's row, then the next heavy; else the
-                    // light's row.  A step needs a further element on its side.
-                    const bool ex = wc <= thr;
-                    const uint64_t mEx = __ballot(ex), mH = __ballot(hn <= hnEnd), mL = __ballot(i >= iEnd);
-                    if (__builtin_amdgcn_inverse_ballot_w64((mEx & mH) | (~mEx & mL))) break;
-                    store_row<AOS>(a, start + (ex ? hj : li), ex ? wc : lw, (int32_t)(start + (ex ? hi1 : hj)));
-                    wc += (ex ? hw1 : lw) - W_N;
-                    hj = ex ? hi1 : hj;
-                    hn -= (int)ex;
-                    i += (int)!ex;
-                    lw = L.Lw(i);
-                    li = L.Li(i);
-                    hw1 = L.w[hn];
-                    hi1 = L.idx[hn];
-                }
-                const int j = len - 2 - hn;
-                // Remainder (PsaPlusNormal.cu:112-123): back to L when its
-                // residual is light and a consumed light slot can hold it,
-                // otherwise back to H in place.
-                if (wc <= thr && i > iLo) {
-                    L.Lw(i - 1) = wc;
-                    L.Li(i - 1) = (uint16_t)hj;
-                    iLo = i - 1;
-                    jLo = j + 1;
-                } else {
-                    L.Hw(j) = wc;
-                    iLo = i;
-                    jLo = j;
-                }
-            }
+            psa_chain_rows<AOS>(a, L, start, W_N, mine, iLo, iHi, jLo, jHi);
         }
     } else if (lane == 0) {
         iHi = nL;

@@ -153,6 +153,10 @@ extern "C" atg_status atg_build_noalloc(const void* weights, atg_dtype dtype, in
     a.pack_method = o.pack_method;
 
     hipStream_t s = (hipStream_t)stream;
+    if (small_build_ok(n, G, Ls, p_req)) {
+        HIPCHK(launch_small(a, false, W_out, error_out, s));
+        return ATG_OK;
+    }
     hipLaunchKernelGGL(clear_state, dim3(1), dim3(64), 0, s, a.st);
     HIPCHK(hipGetLastError());
     HIPCHK(launch_sum(a, s));

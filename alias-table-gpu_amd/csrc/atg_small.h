@@ -1,0 +1,286 @@
+// The whole construction of a small table by one workgroup, its lists in LDS:
+// one launch instead of eight or more, and no global round trip between the
+// phases.  The same canonical association as the kernels of atg_build.hip,
+// so the same rows, lists and splits.
+//
+// A section has a wave (so at most as many sections as waves), a split and a
+// pack chain a thread.  Each phase ends at a barrier that every thread of the
+// workgroup reaches; nothing waits for another workgroup.  With one wave the
+// barriers cost nothing.
+#pragma once
+
+#include "atg_kernels.h"
+
+namespace atg {
+
+// LDS of a table of n items and p_req requested splits.  The section weights
+// and, later, the prefixes share one array.
+struct SmallLds {
+    int64_t items;  // entries of a list array: n items and two sentinels, even
+    int64_t splits;
+    __host__ __device__ SmallLds(int64_t n, int64_t p_req) : items((n + 3) & ~(int64_t)1), splits(p_req + 1) {}
+    __host__ __device__ size_t bytes() const { return (size_t)items * (8 + 8 + 2 + 2) + (size_t)splits * 16; }
+};
+
+// The light list followed by the heavy list (from entry numL) in LDS.
+struct SmallLists {
+    const double* w;
+    const uint16_t* item;
+    int numL;
+    __device__ int li(int i) const { return item[i]; }
+    __device__ double lw(int i) const { return w[i]; }
+    __device__ int hi(int j) const { return item[numL + j]; }
+    __device__ double hw(int j) const { return w[numL + j]; }
+};
+
+// XU: weights a lane holds (sections of up to 64 XU items).  LISTS: the lists
+// and splits go to HBM as well (for the copy-out of a single table).
+// W_out, error_out: nullable copies of the state's fields.
+template <typename T, bool AOS, int XU, bool LISTS>
+__device__ __forceinline__ void small_build(const BuildArgs& a, double* W_out, uint32_t* error_out, double* lds) {
+    __shared__ double ssum[kSmallMaxWaves], sagg[2][kSmallMaxWaves];
+    __shared__ uint32_t scnt[2][kSmallMaxWaves];
+    __shared__ uint32_t sfall;
+    const SmallLds lay(a.n, a.p_req);
+    double* A = lds;              // section weights, then prefixes (lights, then heavies)
+    double* B = A + lay.items;    // list weights
+    Split* sp = reinterpret_cast<Split*>(B + lay.items);
+    uint16_t* idx = reinterpret_cast<uint16_t*>(sp + lay.splits);  // section items, local to the section
+    uint16_t* item = idx + lay.items;                              // list items
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = wave_in_block();
+    const int G = (int)a.G, s = wave;
+    const bool has = s < G;
+    const int64_t start = min(a.n, s * a.Ls);
+    const int len = has ? (int)(min(a.n, (s + 1) * a.Ls) - start) : 0;
+
+    // 1. The section's weights and their sum (section_sum's order).
+    T x[XU];
+    if (has) section_load<T>(a, s, lane, x);
+    {
+        double acc = 0.0;
+        bool bad = false;
+#pragma unroll
+        for (int u = 0; u < XU; ++u) {
+            if ((u << 6) + lane < len) {
+                const double v = (double)x[u];
+                bad |= !(v >= 0.0) || (v == __builtin_inf());
+                acc = acc + v;
+            }
+        }
+        double sum = wave_tree_sum(acc);
+        if (__ballot(bad) != 0ull) sum = __builtin_nan("");
+        if (has && lane == 0) ssum[s] = sum;
+        if (tid == 0) sfall = 0u;
+    }
+    __syncthreads();
+    const double W = wave_tree_sum(lane < G ? ssum[lane] : 0.0);
+    const double W_N = W / (double)a.n;
+    uint32_t err = 0;
+    if (W != W) err = ERR_BAD_WEIGHT;
+    else if (!(W > 0.0) || W == __builtin_inf()) err = ERR_BAD_SUM;
+    if (tid == 0) {
+        DevState* st = a.st;
+        st->W = W;
+        st->W_N = W_N;
+        st->error = err;
+        st->degenerate = 0;
+        st->cert_max_dL = 0ull;
+        st->cert_min_dH = 0x7FF0000000000000ull;
+        st->cert_done = 0;
+        st->split_fallbacks = 0;
+        st->learned_fallbacks = 0;
+        if (W_out) *W_out = W;
+        if (error_out) *error_out = err;
+    }
+    if (err) return;  // the same in every thread
+
+    // 2. Stable partition, chains, leftover counts (psa_section's).
+    SecLDS L;
+    L.w = A + start;
+    L.idx = idx + start;
+    L.len = len;
+    int iLo = 0, iHi = 0, jLo = 0, jHi = 0, offL = 0, offH = 0, mL = 0, mH = 0;
+    if (has) {
+        const uint64_t lt = lanemask_lt();
+        int nL = 0, nH = 0;
+#pragma unroll
+        for (int u = 0; u < XU; ++u) {
+            if ((u << 6) < len) {
+                const int k = (u << 6) + lane;
+                const double xv = (double)x[u];
+                const bool valid = k < len, light = valid && xv <= W_N;
+                const uint64_t bl = __ballot(light), bh = __ballot(valid && !light);
+                const int slot = light ? nL + __popcll(bl & lt) : len - 1 - (nH + __popcll(bh & lt));
+                if (valid) {
+                    L.w[slot] = xv;
+                    L.idx[slot] = (uint16_t)k;
+                }
+                nL += __popcll(bl);
+                nH += __popcll(bh);
+            }
+        }
+        wave_lds_sync();
+        if (a.psa_plus) {
+            chain_ranges(a.chains, nL, nH, lane, iLo, iHi, jLo, jHi);
+            psa_chain_rows<AOS>(a, L, start, W_N, iHi - iLo > 0 && jHi - jLo > 0, iLo, iHi, jLo, jHi);
+        } else if (lane == 0) {
+            iHi = nL;
+            jHi = nH;
+        }
+        const int cl = iHi - iLo, ch = jHi - jLo;
+        const uint32_t cp = (uint32_t)cl | ((uint32_t)ch << 16);
+        const uint32_t incl = wave_incl_scan_u32(cp), excl = incl - cp;
+        const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        offL = (int)(excl & 0xFFFFu);
+        offH = (int)(excl >> 16);
+        mL = (int)(tot & 0xFFFFu);
+        mH = (int)(tot >> 16);
+        if (lane == 0) {
+            scnt[0][s] = (uint32_t)mL;
+            scnt[1][s] = (uint32_t)mH;
+        }
+        wave_lds_sync();
+    }
+    __syncthreads();
+
+    // 3. The lists in rank order: lights [0, numL), heavies from numL on, the
+    //    sentinels last (AliasTableSplitGpu.cu:366-385).
+    const uint32_t inclL = wave_incl_scan_u32(lane < G ? scnt[0][lane] : 0u);
+    const uint32_t inclH = wave_incl_scan_u32(lane < G ? scnt[1][lane] : 0u);
+    const int nLr = __builtin_amdgcn_readlane((int)inclL, 63), nHr = __builtin_amdgcn_readlane((int)inclH, 63);
+    const int numL = nLr + 1, numH = nHr + 1;
+    const int sl = has ? s : 0;
+    const int goffL = __builtin_amdgcn_readlane((int)inclL, sl) - mL;
+    const int goffH = numL + __builtin_amdgcn_readlane((int)inclH, sl) - mH;
+    int first = 1;
+    while (2 * first < a.chains) first *= 2;
+    if (has) {
+        for (int hv = 0; hv < 2; ++hv) {
+            const int m = hv ? mH : mL, dst = hv ? goffH : goffL;
+            for (int g0 = 0; g0 < m; g0 += 64 * 4) {
+                int pos[4];
+                if (a.psa_plus) {
+                    chain_positions<4>(g0 + lane, hv ? offH : offL, hv ? jLo : iLo, pos, first);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) pos[u] = g0 + 64 * u + lane;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int r = g0 + 64 * u + lane;
+                    if (r < m) {
+                        B[dst + r] = hv ? L.Hw(pos[u]) : L.Lw(pos[u]);
+                        item[dst + r] = (uint16_t)(start + (hv ? L.Hi(pos[u]) : L.Li(pos[u])));
+                    }
+                }
+            }
+        }
+    }
+    if (tid == 0) {
+        B[nLr] = 0.0;
+        item[nLr] = (uint16_t)(a.n + 1);
+        B[numL + nHr] = __builtin_inf();
+        item[numL + nHr] = (uint16_t)a.n;
+    }
+    __syncthreads();
+
+    // 4. Local prefixes into A (the section weights are all in B by now), the
+    //    sections' aggregates, then P(s) + local.
+    if (has) {
+        for (int hv = 0; hv < 2; ++hv) {
+            const int m = hv ? mH : mL, dst = hv ? goffH : goffL;
+            double carry = 0.0;
+            for (int r0 = 0; r0 < m; r0 += 64) {
+                const int r = r0 + lane;
+                const double inc = wave_scan(r < m ? B[dst + r] : 0.0);
+                const double local = carry + wave_shr1(inc);
+                if (r < m) A[dst + r] = local;
+                carry = carry + readlane_d(inc, 63);
+            }
+            if (lane == 0) sagg[hv][s] = carry;
+        }
+    }
+    __syncthreads();
+    // Lane c of level b holds the sum of sections [c, c + 2^b) for c a
+    // multiple of 2^b; P(k) folds the blocks of k's binary digits from the
+    // highest to the lowest (block_prefix_done).
+    double tot[2];
+    for (int hv = 0; hv < 2; ++hv) {
+        double t[5];
+        t[0] = lane < G ? sagg[hv][lane] : 0.0;
+#pragma unroll
+        for (int b = 1; b < 5; ++b) t[b] = t[b - 1] + __shfl(t[b - 1], (lane + (1 << (b - 1))) & 63, 64);
+        double P = 0.0, Q = 0.0;
+#pragma unroll
+        for (int b = 4; b >= 0; --b) {
+            if ((s >> b) & 1) P = P + readlane_d(t[b], (s >> (b + 1)) << (b + 1));
+            if ((G >> b) & 1) Q = Q + readlane_d(t[b], (G >> (b + 1)) << (b + 1));
+        }
+        tot[hv] = Q;
+        if (has) {
+            const int m = hv ? mH : mL, dst = hv ? goffH : goffL;
+            for (int r = lane; r < m; r += 64) {
+                const double pref = P + A[dst + r];
+                A[dst + r] = pref;
+                if (LISTS) {
+                    const int g = hv ? dst + r - numL : dst + r;
+                    (hv ? a.Hi : a.Li)[g] = (int32_t)item[dst + r];
+                    (hv ? a.Hw : a.Lw)[g] = B[dst + r];
+                    (hv ? a.Hp : a.Lp)[g] = pref;
+                }
+            }
+        }
+    }
+    const bool degenerate = nLr == 0 || nHr == 0;
+    int64_t p = a.p_req;
+    if (a.psa_plus) { p = min<int64_t>(p, (numL + numH) / 10); if (p < 2) p = 2; }
+    const int64_t nToSplit = numL + numH - 2;
+    const double wToSplit = tot[0] + tot[1];
+    if (tid == 0) {
+        A[nLr] = tot[0];
+        A[numL + nHr] = tot[1];
+        DevState* st = a.st;
+        st->numL = numL;
+        st->numH = numH;
+        st->degenerate = degenerate ? 1u : 0u;
+        st->p = degenerate ? 0 : p;
+        st->nToSplit = nToSplit;
+        st->wToSplit = wToSplit;
+        if (LISTS) {
+            a.Li[nLr] = (int32_t)(a.n + 1); a.Lw[nLr] = 0.0; a.Lp[nLr] = tot[0];
+            a.Hi[nHr] = (int32_t)a.n; a.Hw[nHr] = __builtin_inf(); a.Hp[nHr] = tot[1];
+        }
+    }
+    __syncthreads();
+
+    if (degenerate) {  // the same in every thread
+        // Every leftover row carries its own mass.
+        for (int t = tid; t < nLr + nHr; t += (int)blockDim.x) {
+            const int e = t < nLr ? t : t + 1;  // past the light sentinel
+            store_row<AOS>(a, item[e], B[e], (int32_t)item[e]);
+        }
+        return;
+    }
+
+    // 5. Splits, a thread each.
+    for (int64_t k = tid; k <= p; k += blockDim.x) {
+        Split r;
+        if (k == 0) {
+            r = Split{0, 0, 0.0};
+        } else if (k == p) {
+            r = Split{numL - 1, numH - 1, 0.0};
+        } else if (!bisect_split(k, p, nToSplit, wToSplit, A, numL, A + numL, B + numL, numH, r)) {
+            atomicAdd(&sfall, 1u);
+        }
+        sp[k] = r;
+        if (LISTS) a.splits[k] = r;
+    }
+    __syncthreads();
+
+    // 6. Pack chains, a thread each.
+    const SmallLists lists{B, item, numL};
+    for (int64_t k = tid; k < p; k += blockDim.x) pack_chain<AOS>(a, lists, sp[k], sp[k + 1], W_N);
+    if (tid == 0 && sfall != 0u) a.st->split_fallbacks = sfall;
+}
+
+}  // namespace atg
