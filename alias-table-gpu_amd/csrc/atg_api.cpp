@@ -148,6 +148,7 @@ struct atg_table_s {
         a.ta = d_ta;
         a.psa_plus = opts.psa_plus;
         a.chains = opts.chains;
+        a.chain_mul = chain_multiplier(opts.chains);
         a.p_req = p_req;
         a.splits = d_splits;
         a.pack_cap = pack_cap_items(n, p_req);

@@ -558,6 +558,7 @@ atg_status atg_batch_create(atg_batch** out, const int64_t* offsets, int64_t nta
         a.ta = nullptr;
         a.psa_plus = o.psa_plus;
         a.chains = o.chains;
+        a.chain_mul = chain_multiplier(o.chains);
         a.p_req = z.p_req;
         a.pack_cap = pack_cap_items(n, z.p_req);
         b->pack_cap_max = std::max(b->pack_cap_max, a.pack_cap);

@@ -35,6 +35,7 @@ struct BuildArgs {
     double* tw; int32_t* ta;  // SoA table or null
     int32_t psa_plus;
     int32_t chains;
+    uint32_t chain_mul;       // chain_multiplier(chains)
     int64_t p_req;            // p after the N/10 clamp (grid bound for split/pack)
     Split* splits;            // capacity p_req + 1
     int32_t pack_cap;         // list items one pack wave stages in LDS (pack_cap_items)
@@ -59,6 +60,10 @@ inline int64_t light_dir_size(int64_t n) { return (n >> kLightDirShift) + 2; }
 inline bool lean_lights_ok(int64_t n, int64_t p_req, int32_t pack_method) {
     return pack_method == PACK_CHUNKED && p_req > 0 && n / p_req <= 256;
 }
+
+// x / chains = x chain_mul >> 20 for x <= 2048 and chains <= 64: with M =
+// ceil(2^20 / C), x (M C - 2^20) < 2048 64 < 2^20.
+inline uint32_t chain_multiplier(int32_t chains) { return ((1u << 20) + (uint32_t)chains - 1) / (uint32_t)chains; }
 
 // Section layout of PSA+ (AliasTableSplitGpu.cu:356-357, PsaPlusNormal.cu:27-29).
 inline void section_layout(int64_t n, int64_t param, int64_t* G, int64_t* Ls) {
@@ -147,10 +152,7 @@ hipError_t launch_join_rows(const double* w, const int32_t* al, Row* rows, int64
 // above leave, in one launch.  W_out, error_out: nullable device copies.
 constexpr int kSmallMaxWaves = 16;  // waves of a workgroup, one per section: sections of up to 1024 items
 constexpr int kSmallLongWaves = 4;  // longer ones
-#ifndef SMALLMAX
-#define SMALLMAX 8192
-#endif
-constexpr int64_t kSmallMaxItems = SMALLMAX;
+constexpr int64_t kSmallMaxItems = 8192;
 constexpr size_t kSmallLdsMax = 156 * 1024;  // of 160 KB, static LDS aside
 bool small_build_ok(int64_t n, int64_t G, int64_t Ls, int64_t p_req);
 hipError_t launch_small(const BuildArgs& a, bool lists, double* W_out, uint32_t* error_out, hipStream_t s);

@@ -302,10 +302,12 @@ __device__ __forceinline__ void stage_chunks(const BuildArgs& a, SecLDS& L, bool
 
 // Count slices of a section's nL lights and nH heavies, lane t's for chain t
 // (empty from the chain count on).
-__device__ __forceinline__ void chain_ranges(int C, int nL, int nH, int t, int& iLo, int& iHi, int& jLo, int& jHi) {
+__device__ __forceinline__ void chain_ranges(const BuildArgs& a, int nL, int nH, int t, int& iLo, int& iHi, int& jLo,
+                                             int& jHi) {
+    const int C = a.chains;
     iLo = iHi = jLo = jHi = 0;
     if (t < C) {
-        const int stepsL = nL / C, stepsH = nH / C;
+        const int stepsL = (int)((uint32_t)nL * a.chain_mul >> 20), stepsH = (int)((uint32_t)nH * a.chain_mul >> 20);
         iLo = t * stepsL; iHi = (t == C - 1) ? nL : (t + 1) * stepsL;
         jLo = t * stepsH; jHi = (t == C - 1) ? nH : (t + 1) * stepsH;
     }
@@ -439,7 +441,7 @@ __device__ __forceinline__ void psa_section(const BuildArgs& a, int64_t s, T (&x
     int iLo = 0, iHi = 0, jLo = 0, jHi = 0;
     if (a.psa_plus) {
         // Greedy chains (PsaPlusNormal.cu:51-123), lane t runs chain t.
-        chain_ranges(a.chains, nL, nH, lane, iLo, iHi, jLo, jHi);
+        chain_ranges(a, nL, nH, lane, iLo, iHi, jLo, jHi);
         const bool mine = iHi - iLo > 0 && jHi - jLo > 0;
         if (ROWS_LATER) {
             // A chain's step consumes the current heavy (its bucket is full: a

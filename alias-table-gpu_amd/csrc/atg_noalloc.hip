@@ -147,6 +147,7 @@ extern "C" atg_status atg_build_noalloc(const void* weights, atg_dtype dtype, in
     }
     a.psa_plus = o.psa_plus;
     a.chains = o.chains;
+    a.chain_mul = chain_multiplier(o.chains);
     a.p_req = p_req;
     a.pack_cap = pack_cap_items(n, p_req);
     a.learned_segments = learned_knots(o.learned_segments, p_req);

@@ -5,8 +5,11 @@
 //
 // A section has a wave (so at most as many sections as waves), a split and a
 // pack chain a thread.  Each phase ends at a barrier that every thread of the
-// workgroup reaches; nothing waits for another workgroup.  With one wave the
-// barriers cost nothing.
+// workgroup reaches; nothing waits for another workgroup.
+// Bound by latency, much of it that of fetching instructions: each launch
+// runs through the code about once, so loops stay loops (the classes of a
+// list, the chunks of a section) and a kernel holds as few chunks of a
+// section as its sections have.
 #pragma once
 
 #include "atg_kernels.h"
@@ -121,7 +124,7 @@ __device__ __forceinline__ void small_build(const BuildArgs& a, double* W_out, u
         }
         wave_lds_sync();
         if (a.psa_plus) {
-            chain_ranges(a.chains, nL, nH, lane, iLo, iHi, jLo, jHi);
+            chain_ranges(a, nL, nH, lane, iLo, iHi, jLo, jHi);
             psa_chain_rows<AOS>(a, L, start, W_N, iHi - iLo > 0 && jHi - jLo > 0, iLo, iHi, jLo, jHi);
         } else if (lane == 0) {
             iHi = nL;
@@ -155,18 +158,21 @@ __device__ __forceinline__ void small_build(const BuildArgs& a, double* W_out, u
     int first = 1;
     while (2 * first < a.chains) first *= 2;
     if (has) {
+        constexpr int U = XU < 4 ? XU : 4;
+#pragma unroll 1
         for (int hv = 0; hv < 2; ++hv) {
             const int m = hv ? mH : mL, dst = hv ? goffH : goffL;
-            for (int g0 = 0; g0 < m; g0 += 64 * 4) {
-                int pos[4];
+#pragma unroll 1
+            for (int g0 = 0; g0 < m; g0 += 64 * U) {
+                int pos[U];
                 if (a.psa_plus) {
-                    chain_positions<4>(g0 + lane, hv ? offH : offL, hv ? jLo : iLo, pos, first);
+                    chain_positions<U>(g0 + lane, hv ? offH : offL, hv ? jLo : iLo, pos, first);
                 } else {
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) pos[u] = g0 + 64 * u + lane;
+                    for (int u = 0; u < U; ++u) pos[u] = g0 + 64 * u + lane;
                 }
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
+                for (int u = 0; u < U; ++u) {
                     const int r = g0 + 64 * u + lane;
                     if (r < m) {
                         B[dst + r] = hv ? L.Hw(pos[u]) : L.Lw(pos[u]);
@@ -187,9 +193,11 @@ __device__ __forceinline__ void small_build(const BuildArgs& a, double* W_out, u
     // 4. Local prefixes into A (the section weights are all in B by now), the
     //    sections' aggregates, then P(s) + local.
     if (has) {
+#pragma unroll 1
         for (int hv = 0; hv < 2; ++hv) {
             const int m = hv ? mH : mL, dst = hv ? goffH : goffL;
             double carry = 0.0;
+#pragma unroll 1
             for (int r0 = 0; r0 < m; r0 += 64) {
                 const int r = r0 + lane;
                 const double inc = wave_scan(r < m ? B[dst + r] : 0.0);
@@ -204,7 +212,8 @@ __device__ __forceinline__ void small_build(const BuildArgs& a, double* W_out, u
     // Lane c of level b holds the sum of sections [c, c + 2^b) for c a
     // multiple of 2^b; P(k) folds the blocks of k's binary digits from the
     // highest to the lowest (block_prefix_done).
-    double tot[2];
+    double tot[2] = {0.0, 0.0};
+#pragma unroll 1
     for (int hv = 0; hv < 2; ++hv) {
         double t[5];
         t[0] = lane < G ? sagg[hv][lane] : 0.0;
@@ -216,9 +225,11 @@ __device__ __forceinline__ void small_build(const BuildArgs& a, double* W_out, u
             if ((s >> b) & 1) P = P + readlane_d(t[b], (s >> (b + 1)) << (b + 1));
             if ((G >> b) & 1) Q = Q + readlane_d(t[b], (G >> (b + 1)) << (b + 1));
         }
-        tot[hv] = Q;
+        if (hv) tot[1] = Q;
+        else tot[0] = Q;
         if (has) {
             const int m = hv ? mH : mL, dst = hv ? goffH : goffL;
+#pragma unroll 1
             for (int r = lane; r < m; r += 64) {
                 const double pref = P + A[dst + r];
                 A[dst + r] = pref;

@@ -17,8 +17,9 @@ template <typename T, bool AOS, bool LISTS>
 static hipError_t launch_small_t(const BuildArgs& a, double* W_out, uint32_t* error_out, hipStream_t s) {
     const bool shorts = a.Ls <= kShortSectionMax;
     void (*k)(BuildArgs, double*, uint32_t*) =
-        shorts ? build_small<T, AOS, kShortSectionMax / 64, 64 * kSmallMaxWaves, LISTS>
-               : build_small<T, AOS, PSA_MAX_LEN / 64, 64 * kSmallLongWaves, LISTS>;
+        a.Ls <= 128 ? build_small<T, AOS, 2, 64 * kSmallMaxWaves, LISTS>
+        : shorts    ? build_small<T, AOS, kShortSectionMax / 64, 64 * kSmallMaxWaves, LISTS>
+                    : build_small<T, AOS, PSA_MAX_LEN / 64, 64 * kSmallLongWaves, LISTS>;
     const size_t lds = SmallLds(a.n, a.p_req).bytes();
     if (lds > 65536 - 1024) {  // beyond 64 KB, static LDS included
         const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
