@@ -22,6 +22,7 @@
 #include "atg_host.h"
 #include "atg_kernels.h"
 #include "atg_sample.h"
+#include "atg_small.h"
 
 namespace atg {
 
@@ -206,6 +207,20 @@ __global__ __launch_bounds__(64) void seg_pack(SegArgs g, SegMap m) {
     tick_end(g, t);
 }
 
+// Small tables, a workgroup of one wave each from start to end (atg_small.h),
+// bound by the latency of its chains (30 us for 2,000 items).  16,384 tables
+// of 16 to 4,096 items, half of the items in tables of one section: 0.51 ms
+// through the phases alone, 0.39 with the classes before them, 0.30 with the
+// classes beside them.
+template <typename T, int XU>
+__global__ __launch_bounds__(64) void seg_small(SegArgs g, SegMap m) {
+    extern __shared__ double lds_raw[];
+    const int64_t t = m.tab[blockIdx.x];
+    if (threadIdx.x == 0) g.ticks[2 * t] = (uint64_t)wall_clock64();
+    small_build<T, true, XU, false>(table_args(g, t), nullptr, nullptr, lds_raw);
+    if (threadIdx.x == 0) g.ticks[2 * t + 1] = (uint64_t)wall_clock64();
+}
+
 // Basic alias sampling of every table: sample k of table t uses the Philox
 // block at counter (t * per_table + k, PURPOSE_BATCH); the result is an item
 // index local to the table (-1 when the table failed to build).
@@ -233,7 +248,19 @@ __global__ __launch_bounds__(256) void batch_sample(BatchSampleArgs a) {
 
 using namespace atg;
 
-enum { MAP_SUM, MAP_LOCAL, MAP_PLACE, MAP_DEG, MAP_SPLIT, MAP_KNOTS, MAP_PACK, MAP_TREE, MAP_ONE, MAP_COUNT };
+enum { MAP_SUM, MAP_LOCAL, MAP_PLACE, MAP_DEG, MAP_SPLIT, MAP_KNOTS, MAP_PACK, MAP_TREE, MAP_ONE, MAP_SMALL, MAP_COUNT = MAP_SMALL + 4 };
+
+// Classes of tables built by seg_small, by their one section's length: chunks
+// of 64 items a lane holds.  A class has one launch, with the LDS of its
+// largest table, so that small tables are not held to the occupancy of larger
+// ones.
+constexpr int kSmallClasses = MAP_COUNT - MAP_SMALL;
+constexpr int kSmallChunks[kSmallClasses] = {2, 8, 16, 32};
+constexpr size_t kBatchSmallLds = 50 * 1024;
+// Small tables hold at least one item in this many, or go through the phases
+// (100 of them among 1,024 tables of up to 2^20 items: 3.06 ms in the phases,
+// 3.10 by themselves).
+constexpr int64_t kBatchSmallShare = 8;
 
 // The launches of one group: a block->table map per phase (MAP_ONE: one block
 // per table) and the group's most sections of a table (tree levels).
@@ -253,6 +280,12 @@ struct atg_batch_s {
     std::vector<BuildArgs> args;        // host copy (pointers into the pools below)
     int64_t Ls_max = 1;
     int32_t pack_cap_max = 16;          // largest pack LDS pool of the tables (items)
+    std::vector<int8_t> small_class;    // table -> class of seg_small, -1: the phases
+    size_t small_lds[kSmallClasses] = {};  // LDS of the class's largest table
+    // Streams the small classes run on beside the phases, forked from and
+    // joined to the build's stream.
+    hipStream_t side[2] = {};
+    hipEvent_t ev_fork = nullptr, ev_join[2] = {};
     double wall_khz = 100000.0;
     std::vector<BatchGroup> groups;     // launched in order
     std::vector<int32_t> group_of;      // table -> group
@@ -293,6 +326,11 @@ void drop_graph(atg_batch* b) {
 
 void free_batch(atg_batch* b) {
     drop_graph(b);
+    for (int k = 0; k < 2; ++k) {
+        if (b->side[k]) (void)hipStreamDestroy(b->side[k]);
+        if (b->ev_join[k]) (void)hipEventDestroy(b->ev_join[k]);
+    }
+    if (b->ev_fork) (void)hipEventDestroy(b->ev_fork);
     void* ptrs[] = {b->d_weights_owned, b->d_args, b->d_offsets, b->d_ticks, b->d_state, b->d_rows,
                     b->d_dpool, b->d_slots, b->d_ipool, b->d_splits, b->d_maptab, b->d_mapbase};
     for (void* p : ptrs)
@@ -306,6 +344,20 @@ void bind_weights(atg_batch* b) {
         b->args[t].weights = (const char*)b->d_weights + (size_t)b->offsets[t] * es;
 }
 
+// The tables of class C of a group.
+template <typename T, int C>
+void launch_class(const atg_batch* b, const SegArgs& g, const BatchGroup& grp, hipStream_t s) {
+    const SegMap& m = grp.maps[MAP_SMALL + C];
+    if (m.blocks > 0)
+        hipLaunchKernelGGL((seg_small<T, kSmallChunks[C]>), dim3((unsigned)m.blocks), dim3(64), b->small_lds[C], s, g, m);
+}
+
+#define HIP_TRY(call)                        \
+    do {                                     \
+        const hipError_t e_ = (call);        \
+        if (e_ != hipSuccess) return e_;     \
+    } while (0)
+
 template <typename T>
 hipError_t launch_batch(const atg_batch* b, hipStream_t s) {
     SegArgs g{b->d_args, b->ntables, b->d_ticks};
@@ -317,29 +369,57 @@ hipError_t launch_batch(const atg_batch* b, hipStream_t s) {
     const bool learned = b->opts.split_method == ATG_SPLIT_LEARNED;
     for (const BatchGroup& grp : b->groups) {
         const SegMap* M = grp.maps;
-        // Every group holds at least one table, so each map below has blocks
-        // (MAP_KNOTS and MAP_TREE are checked: a group of one-section tables
-        // has no tree blocks).
-        hipLaunchKernelGGL(seg_sum<T>, grid(M[MAP_SUM]), dim3(256), 0, s, g, M[MAP_SUM]);
-        hipLaunchKernelGGL(seg_sum_finish, grid(M[MAP_ONE]), dim3(256), 0, s, g, M[MAP_ONE]);
-        const bool later = rows_later_ok(M[MAP_LOCAL].blocks, resident);
-        hipLaunchKernelGGL((later ? seg_local<T, true> : seg_local<T, false>),
-                           dim3((unsigned)std::min<int64_t>(M[MAP_LOCAL].blocks, resident)), dim3(64), lds, s, g,
-                           M[MAP_LOCAL]);
-        if (M[MAP_TREE].blocks > 0)
-            for (int b0 = 0; (grp.G_max >> b0) > 1; b0 += 9)
-                hipLaunchKernelGGL(seg_tree, grid(M[MAP_TREE]), dim3(256), 0, s, g, M[MAP_TREE], b0);
-        hipLaunchKernelGGL(seg_place, grid(M[MAP_PLACE]), dim3(256), 0, s, g, M[MAP_PLACE]);
-        if (learned) hipLaunchKernelGGL(seg_cert, grid(M[MAP_ONE]), dim3(256), 0, s, g, M[MAP_ONE]);
-        hipLaunchKernelGGL(seg_degenerate, grid(M[MAP_DEG]), dim3(256), 0, s, g, M[MAP_DEG]);
-        if (learned) {
-            if (M[MAP_KNOTS].blocks > 0)
-                hipLaunchKernelGGL(seg_knots, grid(M[MAP_KNOTS]), dim3(256), 0, s, g, M[MAP_KNOTS]);
-            hipLaunchKernelGGL(seg_learned, grid(M[MAP_SPLIT]), dim3(256), 0, s, g, M[MAP_SPLIT]);
-        } else {
-            hipLaunchKernelGGL(seg_split, grid(M[MAP_SPLIT]), dim3(256), 0, s, g, M[MAP_SPLIT]);
+        // A group with tables that go through the phases has blocks in each
+        // map below (MAP_KNOTS and MAP_TREE are checked: a group of
+        // one-section tables has no tree blocks).
+        // The small classes share nothing with the phases or each other, and
+        // each is a few rounds of latency: they run beside the phases, the
+        // class of the longest tables by itself, and join the stream before
+        // the group ends.
+        const bool classes[2] = {M[MAP_SMALL + 3].blocks > 0,
+                                 M[MAP_SMALL].blocks + M[MAP_SMALL + 1].blocks + M[MAP_SMALL + 2].blocks > 0};
+        const bool phases = M[MAP_SUM].blocks > 0;
+        hipStream_t on[2] = {s, s};
+        if (phases || (classes[0] && classes[1])) {
+            if (classes[0] || classes[1]) HIP_TRY(hipEventRecord(b->ev_fork, s));
+            for (int k = 0; k < 2; ++k)
+                if (classes[k] && (phases || k == 0)) {
+                    on[k] = b->side[k];
+                    HIP_TRY(hipStreamWaitEvent(on[k], b->ev_fork, 0));
+                }
         }
-        hipLaunchKernelGGL(seg_pack, grid(M[MAP_PACK]), dim3(64), pack_lds_bytes(b->pack_cap_max), s, g, M[MAP_PACK]);
+        static_assert(kSmallClasses == 4, "a launch per class");
+        launch_class<T, 3>(b, g, grp, on[0]);
+        launch_class<T, 2>(b, g, grp, on[1]);
+        launch_class<T, 1>(b, g, grp, on[1]);
+        launch_class<T, 0>(b, g, grp, on[1]);
+        if (phases) {
+            hipLaunchKernelGGL(seg_sum<T>, grid(M[MAP_SUM]), dim3(256), 0, s, g, M[MAP_SUM]);
+            hipLaunchKernelGGL(seg_sum_finish, grid(M[MAP_ONE]), dim3(256), 0, s, g, M[MAP_ONE]);
+            const bool later = rows_later_ok(M[MAP_LOCAL].blocks, resident);
+            hipLaunchKernelGGL((later ? seg_local<T, true> : seg_local<T, false>),
+                               dim3((unsigned)std::min<int64_t>(M[MAP_LOCAL].blocks, resident)), dim3(64), lds, s, g,
+                               M[MAP_LOCAL]);
+            if (M[MAP_TREE].blocks > 0)
+                for (int b0 = 0; (grp.G_max >> b0) > 1; b0 += 9)
+                    hipLaunchKernelGGL(seg_tree, grid(M[MAP_TREE]), dim3(256), 0, s, g, M[MAP_TREE], b0);
+            hipLaunchKernelGGL(seg_place, grid(M[MAP_PLACE]), dim3(256), 0, s, g, M[MAP_PLACE]);
+            if (learned) hipLaunchKernelGGL(seg_cert, grid(M[MAP_ONE]), dim3(256), 0, s, g, M[MAP_ONE]);
+            hipLaunchKernelGGL(seg_degenerate, grid(M[MAP_DEG]), dim3(256), 0, s, g, M[MAP_DEG]);
+            if (learned) {
+                if (M[MAP_KNOTS].blocks > 0)
+                    hipLaunchKernelGGL(seg_knots, grid(M[MAP_KNOTS]), dim3(256), 0, s, g, M[MAP_KNOTS]);
+                hipLaunchKernelGGL(seg_learned, grid(M[MAP_SPLIT]), dim3(256), 0, s, g, M[MAP_SPLIT]);
+            } else {
+                hipLaunchKernelGGL(seg_split, grid(M[MAP_SPLIT]), dim3(256), 0, s, g, M[MAP_SPLIT]);
+            }
+            hipLaunchKernelGGL(seg_pack, grid(M[MAP_PACK]), dim3(64), pack_lds_bytes(b->pack_cap_max), s, g, M[MAP_PACK]);
+        }
+        for (int k = 0; k < 2; ++k)
+            if (on[k] != s) {
+                HIP_TRY(hipEventRecord(b->ev_join[k], on[k]));
+                HIP_TRY(hipStreamWaitEvent(s, b->ev_join[k], 0));
+            }
     }
     return hipGetLastError();
 }
@@ -374,11 +454,13 @@ atg_status make_groups(atg_batch* b, int64_t group_items) {
         }
         for (int64_t t = 0; t < ntables; ++t) members[group_of[t]].push_back(t);
         for (int64_t g = 0; g < ngroups; ++g)
-            for (int64_t t : members[g]) groups[g].G_max = std::max(groups[g].G_max, b->args[t].G);
+            for (int64_t t : members[g])
+                if (b->small_class[t] < 0) groups[g].G_max = std::max(groups[g].G_max, b->args[t].G);
     }
     auto blocks_of = [&](int ph, int64_t t) -> int64_t {
         const BuildArgs& a = b->args[t];
         const int64_t K = std::min<int64_t>(a.learned_segments, a.p_req);
+        if (ph >= MAP_SMALL || b->small_class[t] >= 0) return ph == MAP_SMALL + b->small_class[t] ? 1 : 0;
         switch (ph) {
             case MAP_SUM: return (a.G + 3) / 4;
             case MAP_LOCAL: return a.G;
@@ -488,6 +570,7 @@ atg_status atg_batch_create(atg_batch** out, const int64_t* offsets, int64_t nta
     b->opts = o;
     b->offsets.assign(offsets, offsets + ntables + 1);
     b->args.resize((size_t)ntables);
+    b->small_class.assign((size_t)ntables, -1);
     (void)hipGetDevice(&b->device);
     auto cleanup = [&](atg_status st) { free_batch(b); delete b; return st; };
 
@@ -578,9 +661,28 @@ atg_status atg_batch_create(atg_batch** out, const int64_t* offsets, int64_t nta
         a.p_req = z.p_req;
         a.pack_cap = pack_cap_items(n, z.p_req);
         b->pack_cap_max = std::max(b->pack_cap_max, a.pack_cap);
+        // One section and its lists within what leaves a CU three workgroups.
+        const size_t lds = SmallLds(n, z.p_req).bytes();
+        if (z.G == 1 && lds <= kBatchSmallLds) {
+            int c = 0;
+            while (n > 64 * kSmallChunks[c]) ++c;
+            b->small_class[t] = (int8_t)c;
+            b->small_lds[c] = std::max(b->small_lds[c], lds);
+        }
         a.splits = b->d_splits + osp[t];
         a.learned_segments = learned_knots(o.learned_segments, z.p_req);
     }
+    // A few small tables among large ones cost a launch more than they save.
+    int64_t small_items = 0;
+    for (int64_t t = 0; t < ntables; ++t)
+        if (b->small_class[t] >= 0) small_items += offsets[t + 1] - offsets[t];
+    if (kBatchSmallShare * small_items < b->total) b->small_class.assign((size_t)ntables, -1);
+    else if (hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) != hipSuccess)
+        return cleanup(fail(ATG_EDEVICE, "atg_batch_create: events"));
+    for (int k = 0; k < 2 && b->ev_fork; ++k)
+        if (hipStreamCreateWithFlags(&b->side[k], hipStreamNonBlocking) != hipSuccess ||
+            hipEventCreateWithFlags(&b->ev_join[k], hipEventDisableTiming) != hipSuccess)
+            return cleanup(fail(ATG_EDEVICE, "atg_batch_create: side streams"));
     {
         const atg_status rc = make_groups(b, o.batch_group_items);
         if (rc != ATG_OK) return cleanup(rc);
