@@ -150,8 +150,8 @@ __global__ __launch_bounds__(256) void seg_place(SegArgs g, SegMap m) {
     if (s >= a.G) return;
     // Lean lists as in a single table (1.3e8 leftovers of a 1,024-table FP32
     // batch: 0.88 -> 0.46 ms, its pack 1.19 -> 1.08).
-    if (a.lean_lights) place_section<true>(a, s, (int)(threadIdx.x & 63));
-    else place_section<false>(a, s, (int)(threadIdx.x & 63));
+    if (a.lean_lights) place_section<true, false>(a, s, (int)(threadIdx.x & 63));
+    else place_section<false, false>(a, s, (int)(threadIdx.x & 63));
 }
 
 __global__ __launch_bounds__(256) void seg_degenerate(SegArgs g, SegMap m) {

@@ -24,7 +24,7 @@ struct BuildArgs {
     double* section_sums;     // G
     double* tree_scratch;     // 2 * tree_scratch_half
     int64_t tree_scratch_half;
-    uint64_t* slots;          // dyadic block sums (counts, light, heavy) + arrival counters
+    uint64_t* slots;          // dyadic block sums (counts, light, heavy)
     double* stage_w;          // n: leftovers staged by partition pass 1 (weights)
     int32_t* stage_i;         // n: leftovers staged by partition pass 1 (items)
     uint64_t* sec_cert;       // 6 G: per-section split-certificate data (bit patterns)
@@ -54,11 +54,16 @@ struct BuildArgs {
 constexpr int kLightDirShift = 10;
 inline int64_t light_dir_size(int64_t n) { return (n >> kLightDirShift) + 2; }
 
+// Tables below this many items keep whole lists: finding a light in the
+// staging takes the pack a few dependent reads, which the smaller writes pay
+// for only where bandwidth counts (builds, us, lean against whole: 100,003
+// items 51.3 and 46.0, 2^20 71.1 and 71.0, 3e6 95.2 and 95.1, 1e7 244 and 253).
+constexpr int64_t kLeanMin = (int64_t)1 << 21;
 // The lean light lists need every pack chain to fit the staged pack's LDS
 // pool (chains hold at most n / p + 3 items, the pool at least
 // min(64 (n / p + 1), 1024)).
 inline bool lean_lights_ok(int64_t n, int64_t p_req, int32_t pack_method) {
-    return pack_method == PACK_CHUNKED && p_req > 0 && n / p_req <= 256;
+    return n >= kLeanMin && pack_method == PACK_CHUNKED && p_req > 0 && n / p_req <= 256;
 }
 
 // x / chains = x chain_mul >> 20 for x <= 2048 and chains <= 64: with M =
@@ -99,6 +104,14 @@ inline bool pack_windowed_ok(int64_t n, int64_t p_req, int32_t pack_method) {
 // spare weight slot the light steps record into (16 B keep the alignment).
 inline size_t pack_lds_bytes(int32_t cap) { return (size_t)cap * 16 + 16; }
 
+// A split by four lanes, which look two levels of the bisection ahead: half
+// the dependent reads for half as many probes again.  Pays while the reads
+// wait for nothing else (whole builds, us: 100,003 items with 10,000 splits
+// 54.6 -> 51.0, 3e5 items with 30,000 57.6 -> 55.3; 2^20 items with 81,920
+// 70.6 -> 71.2).  The lanes keep positions in 32 bits.
+constexpr int kWideLevels = 2;
+inline bool split_wide_ok(int64_t n, int64_t p_req) { return p_req <= (1 << 15) && n <= ((int64_t)1 << 29); }
+
 // Knots of the learned split index: at most `opt`, and at most one per 16
 // requested splits (at least 64).  Each knot is a full bisection, so a table
 // with few splits would otherwise bisect nearly every split twice; the
@@ -122,6 +135,11 @@ inline size_t psa_lds_bytes(int64_t Ls_max) {
 // us; 1,049 sections: the same).
 inline bool rows_later_ok(int64_t sections, int64_t resident) { return sections > resident; }
 int64_t resident_blocks(const void* f, int threads, size_t lds);
+// Up to this many sections the placement folds P(s) from the sections' own
+// sums, without the tree's launches (builds, us, with and without the tree:
+// 101 sections 46.1 and 43.1, 1,049 sections 70.4 and 66.1, 3,001 sections
+// 94.2 and 97.6: a wave reads up to 24 bytes per section before its own).
+constexpr int64_t kDirectPrefixMax = 2048;
 int64_t block_tree_total(int64_t G);
 hipError_t launch_sum(const BuildArgs& a, hipStream_t s);
 hipError_t launch_partition(const BuildArgs& a, hipStream_t s);
@@ -138,6 +156,7 @@ hipError_t launch_lean_lights_fill(const BuildArgs& a, hipStream_t s);
 // split_blocks (256 splits each) or pack_blocks (64 chains each).
 int64_t split_blocks(const BuildArgs& a);
 int64_t pack_blocks(const BuildArgs& a);
+int64_t fill_blocks(int64_t n);
 hipError_t launch_split_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1);
 hipError_t launch_split_knots(const BuildArgs& a, hipStream_t s);
 hipError_t launch_split_learned_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1);

@@ -69,12 +69,12 @@ __global__ __launch_bounds__(256) void cert_reduce(BuildArgs a) {
 }
 
 // Four sections per block, one per wave.
-template <bool LEAN>
+template <bool LEAN, bool DIRECT>
 __global__ __launch_bounds__(256) void partition_place(BuildArgs a) {
     if (a.st->error) return;
     const int64_t s = (int64_t)blockIdx.x * 4 + wave_in_block();
     if (s >= a.G) return;
-    place_section<LEAN>(a, s, (int)(threadIdx.x & 63));
+    place_section<LEAN, DIRECT>(a, s, (int)(threadIdx.x & 63));
 }
 
 // ---------------------------------------------------------------------------
@@ -87,8 +87,25 @@ __global__ void degenerate_fill(BuildArgs a) {
 // ---------------------------------------------------------------------------
 // 3b. Split: bisection per k with the reference's predicate; 64 probes bound
 //     the loop (the reference spins forever when FOUND is unreachable).
-__global__ __launch_bounds__(256) void split_bisect(BuildArgs a, int64_t blk0) {
+//     fill: the launch also fills the rows of a degenerate table, which has
+//     no splits, with all its blocks.
+template <bool AOS>
+__global__ __launch_bounds__(256) void split_bisect(BuildArgs a, int64_t blk0, int fill) {
+    if (fill && a.st->degenerate) {
+        degenerate_block<AOS>(a, blockIdx.x, gridDim.x);
+        return;
+    }
     split_bisect_block(a, blk0 + blockIdx.x);
+}
+
+// The same with several lanes per split (split_wide_ok).
+template <bool AOS>
+__global__ __launch_bounds__(256) void split_bisect_wide(BuildArgs a) {
+    if (a.st->degenerate) {
+        degenerate_block<AOS>(a, blockIdx.x, gridDim.x);
+        return;
+    }
+    split_bisect_wide_block<kWideLevels>(a, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -310,10 +327,16 @@ hipError_t launch_partition(const BuildArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_partition_place(const BuildArgs& a, hipStream_t s) {
-    for (int b0 = 0; (a.G >> b0) > 1; b0 += 9)
-        hipLaunchKernelGGL(block_tree, dim3(blocks_for(a.G >> b0, 512)), dim3(256), 0, s, a, b0);
-    if (a.lean_lights) hipLaunchKernelGGL(partition_place<true>, dim3(blocks_for(a.G, 4)), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(partition_place<false>, dim3(blocks_for(a.G, 4)), dim3(256), 0, s, a);
+    const dim3 g(blocks_for(a.G, 4)), b(256);
+    if (a.G <= kDirectPrefixMax) {
+        if (a.lean_lights) hipLaunchKernelGGL((partition_place<true, true>), g, b, 0, s, a);
+        else hipLaunchKernelGGL((partition_place<false, true>), g, b, 0, s, a);
+    } else {
+        for (int b0 = 0; (a.G >> b0) > 1; b0 += 9)
+            hipLaunchKernelGGL(block_tree, dim3(blocks_for(a.G >> b0, 512)), b, 0, s, a, b0);
+        if (a.lean_lights) hipLaunchKernelGGL((partition_place<true, false>), g, b, 0, s, a);
+        else hipLaunchKernelGGL((partition_place<false, false>), g, b, 0, s, a);
+    }
     if (a.want_cert)
         hipLaunchKernelGGL(cert_reduce, dim3(blocks_for(a.G, 256)), dim3(256), 0, s, a);  // a section per thread
     return hipGetLastError();
@@ -338,15 +361,27 @@ hipError_t launch_degenerate(const BuildArgs& a, hipStream_t s) {
 int64_t split_blocks(const BuildArgs& a) { return a.p_req >= 2 ? blocks_for(a.p_req - 1, 256) : 0; }
 int64_t pack_blocks(const BuildArgs& a) { return blocks_for(a.p_req, 64); }
 
+// Blocks of a launch that also fills a degenerate table's rows: 4096 items a
+// block, at most 1024 blocks (each walks on from there).
+int64_t fill_blocks(int64_t n) { return std::min<int64_t>(1024, blocks_for(n, 4096)); }
+
 hipError_t launch_split_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1) {
-    if (b1 > b0) hipLaunchKernelGGL(split_bisect, dim3((unsigned)(b1 - b0)), dim3(256), 0, s, a, b0);
+    if (b1 > b0) hipLaunchKernelGGL(split_bisect<true>, dim3((unsigned)(b1 - b0)), dim3(256), 0, s, a, b0, 0);
     return hipGetLastError();
 }
 
 hipError_t launch_split(const BuildArgs& a, hipStream_t s) {
-    hipError_t e = launch_degenerate(a, s);
-    if (e != hipSuccess) return e;
-    return launch_split_blocks(a, s, 0, split_blocks(a));  // effective p <= p_req
+    const int64_t fill = fill_blocks(a.n);  // effective p <= p_req
+    if (split_wide_ok(a.n, a.p_req)) {
+        const dim3 g((unsigned)std::max<int64_t>(blocks_for(a.p_req, 256 >> kWideLevels), fill));
+        if (a.rows) hipLaunchKernelGGL(split_bisect_wide<true>, g, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL(split_bisect_wide<false>, g, dim3(256), 0, s, a);
+        return hipGetLastError();
+    }
+    const dim3 g((unsigned)std::max<int64_t>(split_blocks(a), fill));
+    if (a.rows) hipLaunchKernelGGL(split_bisect<true>, g, dim3(256), 0, s, a, (int64_t)0, 1);
+    else hipLaunchKernelGGL(split_bisect<false>, g, dim3(256), 0, s, a, (int64_t)0, 1);
+    return hipGetLastError();
 }
 
 hipError_t launch_pack_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1) {

@@ -1,6 +1,6 @@
 // Device-side building blocks shared by the gfx950 kernels: Philox4x32-10,
 // 64-lane wavefront primitives for FP64, the canonical pairwise tree and
-// Kogge-Stone scan, and agent-scope self-validating slots for look-back.
+// Kogge-Stone scan, and the stores of the block sums.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -10,11 +10,6 @@
 
 #define ATG_WAVE 64
 #define ATG_EPSILON 1e-10  // construction/SamplingAlgorithm.cuh:14
-
-// A published 64-bit slot holds this pattern until its owner writes it.  Sums
-// of validated (finite, non-negative) weights and packed counts (< 2^31 per
-// half) never produce it.
-#define ATG_NOT_READY 0xFFFFFFFFFFFFFFFFull
 
 namespace atg {
 
@@ -220,15 +215,11 @@ __device__ __forceinline__ T wave_excl_scan_int(T v) {
 }
 
 // ---------------------------------------------------------------------------
-// Agent-scope self-validating slots.  Each slot is written exactly once per
-// build by its owner; readers poll until the value differs from ATG_NOT_READY.
-// Relaxed agent-scope atomics compile to sc1 loads/stores on gfx950, which are
-// coherent across the XCDs without an L2 writeback.
+// Stores of the block sums, which later launches read from any XCD: relaxed
+// agent-scope atomics compile to sc1 stores on gfx950, coherent across the
+// XCDs without an L2 write-back.
 __device__ __forceinline__ void slot_store(uint64_t* p, uint64_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint64_t slot_load(const uint64_t* p) {
-    return __hip_atomic_load(const_cast<uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ uint64_t d2u(double d) { return (uint64_t)__double_as_longlong(d); }
 __device__ __forceinline__ double u2d(uint64_t u) { return __longlong_as_double((long long)u); }

@@ -167,6 +167,60 @@ __device__ __forceinline__ Prefix block_prefix_done(const BuildArgs& a, int64_t 
     return P;
 }
 
+// P = the sums of the dyadic blocks of k's binary digits, from the highest
+// digit to the lowest, added to P: lane c of v holds the level-0 block c
+// (c < k < 2^LEVELS; other lanes are not read).
+template <int LEVELS>
+__device__ __forceinline__ double fold_blocks(double P, double v, int k, int lane) {
+    double t[LEVELS];  // level b: lane c, a multiple of 2^b, the block [c, c + 2^b)
+    t[0] = v;
+#pragma unroll
+    for (int b = 1; b < LEVELS; ++b) t[b] = t[b - 1] + __shfl(t[b - 1], (lane + (1 << (b - 1))) & 63, 64);
+#pragma unroll
+    for (int b = LEVELS - 1; b >= 0; --b)
+        if ((k >> b) & 1) P = P + readlane_d(t[b], (k >> (b + 1)) << (b + 1));
+    return P;
+}
+
+// P(s) from the sections' own sums (the level-0 blocks), for s <= 4096: the
+// blocks of 64 sections are the wave's pairwise trees, the larger and the
+// smaller ones come from lane exchanges.  The same blocks in the same order
+// as block_prefix_done.
+__device__ __forceinline__ Prefix block_prefix_direct(const BuildArgs& a, int s, int lane) {
+    const int full = s >> 6, rem = s & 63;
+    const uint64_t *C = a.slots, *Lv = C + a.tree_total, *Hv = Lv + a.tree_total;
+    uint64_t cnt = 0;
+    double l6 = 0.0, h6 = 0.0;  // lane c: sections [64 c, 64 c + 64)
+    for (int g0 = 0; g0 < full; g0 += 8) {
+        double l[8], h[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int i = (g0 + u) * 64 + lane;
+            const bool in = g0 + u < full;
+            cnt += in ? C[i] : 0ull;
+            l[u] = in ? u2d(Lv[i]) : 0.0;
+            h[u] = in ? u2d(Hv[i]) : 0.0;
+        }
+        const double l8 = wave_tree_sum8(l, lane), h8 = wave_tree_sum8(h, lane);
+        if ((lane & ~7) == g0) {
+            l6 = l8;
+            h6 = h8;
+        }
+    }
+    double l0 = 0.0, h0 = 0.0;
+    if (lane < rem) {
+        const int i = full * 64 + lane;
+        cnt += C[i];
+        l0 = u2d(Lv[i]);
+        h0 = u2d(Hv[i]);
+    }
+    Prefix P;
+    P.c = wave_sum_int<uint64_t>(cnt);
+    P.l = fold_blocks<6>(fold_blocks<7>(0.0, l6, full, lane), l0, rem, lane);
+    P.h = fold_blocks<6>(fold_blocks<7>(0.0, h6, full, lane), h0, rem, lane);
+    return P;
+}
+
 // Levels b0 + 1 .. b0 + 9 of the dyadic block tree, T(b, c) = T(b - 1, 2c) +
 // T(b - 1, 2c + 1), over the level-b0 blocks [512 q, 512 q + 512) (one
 // block of 256 threads; only complete blocks, c < G >> b, exist).
@@ -637,14 +691,15 @@ __device__ __forceinline__ void psa_section(const BuildArgs& a, int64_t s, T (&x
 // and for the last section the totals, sentinels and split inputs.
 // LEAN: the lean light lists (a.lean_lights), fixed at compile time so that
 // each kernel carries one path.
-template <bool LEAN>
+// DIRECT: P(s) from the sections' own sums (no tree was built).
+template <bool LEAN, bool DIRECT>
 __device__ __forceinline__ void place_section(const BuildArgs& a, int64_t s, int lane) {
     DevState* st = a.st;
     const int64_t start = min(a.n, s * a.Ls);
     // The block sums were completed by the previous launch.
     const uint64_t c0 = a.slots[s];  // this section's own counts
     const int mL = (int)(uint32_t)c0, mH = (int)(c0 >> 32);
-    const Prefix P = block_prefix_done(a, s, lane);
+    const Prefix P = DIRECT ? block_prefix_direct(a, (int)s, lane) : block_prefix_done(a, s, lane);
     const int64_t goffL = (int64_t)(uint32_t)P.c, goffH = (int64_t)(P.c >> 32);
     // Split certificate (learned split only): the extreme increments between
     // consecutive stored prefixes inside the section, and the section's first
@@ -758,7 +813,7 @@ __device__ __forceinline__ void place_section(const BuildArgs& a, int64_t s, int
     }
     if (s == a.G - 1) {
         // Totals P(G), sentinels (AliasTableSplitGpu.cu:366-385) and the split inputs.
-        const Prefix Tot = block_prefix_done(a, a.G, lane);
+        const Prefix Tot = DIRECT ? block_prefix_direct(a, (int)a.G, lane) : block_prefix_done(a, a.G, lane);
         if (lane == 0) {
             const int64_t nLr = (int64_t)(uint32_t)Tot.c, nHr = (int64_t)(Tot.c >> 32);
             if (LEAN) a.sec_loff[a.G] = (uint32_t)nLr;
@@ -780,8 +835,7 @@ __device__ __forceinline__ void place_section(const BuildArgs& a, int64_t s, int
 
 // ---------------------------------------------------------------------------
 // W, pass 1: section sums, one wave per section (block blk of nblk holds
-// sections 4 blk .. 4 blk + 3), and the reset of the dyadic block sums and
-// their arrival counters for the partition.
+// sections 4 blk .. 4 blk + 3).
 template <typename T>
 __device__ __forceinline__ void sum_sections_block(const BuildArgs& a, int64_t blk, int64_t nblk) {
     const int lane = threadIdx.x & 63, wave = wave_in_block();
@@ -791,9 +845,6 @@ __device__ __forceinline__ void sum_sections_block(const BuildArgs& a, int64_t b
         const double sum = section_sum<T>(w, min(a.n, s * a.Ls), min(a.n, (s + 1) * a.Ls), lane);
         if (lane == 0) a.section_sums[s] = sum;
     }
-    const int64_t nvals = 3 * a.tree_total, ncnt = (a.tree_total + 1) / 2;
-    for (int64_t i = blk * blockDim.x + threadIdx.x; i < nvals + ncnt; i += nblk * blockDim.x)
-        a.slots[i] = (i < nvals) ? ATG_NOT_READY : 0ull;
 }
 
 // W, pass 2 (one block): the 64-ary tree over the section sums, 64 values per
@@ -1285,6 +1336,25 @@ __device__ __forceinline__ void split_bisect_block(const BuildArgs& a, int64_t b
     if (k >= p) return;
     Split sp;
     const bool ok = bisect_split(k, p, st->nToSplit, st->wToSplit, a.Lp, numL, a.Hp, a.Hw, numH, sp);
+    a.splits[k] = sp;
+    if (!ok) atomicAdd((unsigned long long*)&st->split_fallbacks, 1ull);
+}
+
+// The same with 2^LEVELS lanes per split.
+template <int LEVELS>
+__device__ __forceinline__ void split_bisect_wide_block(const BuildArgs& a, int64_t blk) {
+    DevState* st = a.st;
+    if (st->error || st->degenerate) return;
+    const int64_t p = st->p, numL = st->numL, numH = st->numH;
+    const int64_t k = (blk * blockDim.x + threadIdx.x) / (1 << LEVELS) + 1;
+    const int g = threadIdx.x % (1 << LEVELS);
+    if (k == 1 && g == 0) {
+        a.splits[0] = Split{0, 0, 0.0};
+        a.splits[p] = Split{(int32_t)(numL - 1), (int32_t)(numH - 1), 0.0};
+    }
+    Split sp;
+    const bool ok = bisect_split_wide<LEVELS>(k < p, g, k, p, st->nToSplit, st->wToSplit, a.Lp, numL, a.Hp, a.Hw, numH, sp);
+    if (k >= p || g != 0) return;
     a.splits[k] = sp;
     if (!ok) atomicAdd((unsigned long long*)&st->split_fallbacks, 1ull);
 }

@@ -209,22 +209,11 @@ __device__ __forceinline__ void small_build(const BuildArgs& a, double* W_out, u
         }
     }
     __syncthreads();
-    // Lane c of level b holds the sum of sections [c, c + 2^b) for c a
-    // multiple of 2^b; P(k) folds the blocks of k's binary digits from the
-    // highest to the lowest (block_prefix_done).
     double tot[2] = {0.0, 0.0};
 #pragma unroll 1
     for (int hv = 0; hv < 2; ++hv) {
-        double t[5];
-        t[0] = lane < G ? sagg[hv][lane] : 0.0;
-#pragma unroll
-        for (int b = 1; b < 5; ++b) t[b] = t[b - 1] + __shfl(t[b - 1], (lane + (1 << (b - 1))) & 63, 64);
-        double P = 0.0, Q = 0.0;
-#pragma unroll
-        for (int b = 4; b >= 0; --b) {
-            if ((s >> b) & 1) P = P + readlane_d(t[b], (s >> (b + 1)) << (b + 1));
-            if ((G >> b) & 1) Q = Q + readlane_d(t[b], (G >> (b + 1)) << (b + 1));
-        }
+        const double v = lane < G ? sagg[hv][lane] : 0.0;
+        const double P = fold_blocks<5>(0.0, v, s, lane), Q = fold_blocks<5>(0.0, v, G, lane);
         if (hv) tot[1] = Q;
         else tot[0] = Q;
         if (has) {

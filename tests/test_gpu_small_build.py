@@ -98,3 +98,30 @@ def test_small_noalloc_equals_table(gpu, layout, split):
             ra = al.cpu().numpy()
         assert np.array_equal(bits(rw), bits(tw)) and np.array_equal(ra, ta)
         assert W.item() == t.stats()["W"] and err.item() == 0
+
+
+@pytest.mark.parametrize("n,section,dist,p", [
+    (9_000, 0, "exponential", 0),              # the smallest default table built by the phases
+    (20_000, 313, "pareto", 0),                # 64 sections: one whole block of 64
+    (20_000, 312, "pareto", 500),              # 65
+    (60_000, 29, "unit_uniform", 32_768),      # 2,069 sections: through the block tree
+    (60_000, 30, "unit_uniform", 6_000),       # 2,001 sections: from the sections' sums
+    (65_504, 32, "pareto", 0),                 # 2,048
+    (400_000, 1000, "heavy_mix", 32_768),      # the most splits with four lanes each
+    (400_000, 1000, "heavy_mix", 32_769),
+    (50_000, 1000, "best_worst", 2),           # one split to find
+    ((1 << 21) - 1, 2048, "pareto", 40_000),   # whole light lists
+    (1 << 21, 2048, "pareto", 40_000),         # lean ones
+    (300_000, 1000, "all_equal", 0),           # degenerate: filled by the split's launch
+])
+def test_mid_size_routes_match_oracle(gpu, oracle, n, section, dist, p):
+    w = np.full(n, 2.5) if dist == "all_equal" else weights(n, dist)
+    p_req = p if p > 0 else 81920
+    for layout in ("aos", "soa"):
+        t = gpu_build(w, layout=layout, section_size=section, num_splits=p_req)
+        ref = oracle.build(w, section_size=section, num_splits=p_req)
+        assert_same_build(t, ref, n)
+        t.build_phase("split")
+        t.build_phase("pack")
+        t.sync()
+        assert_same_build(t, ref, n)
