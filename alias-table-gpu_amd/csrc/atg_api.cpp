@@ -422,8 +422,7 @@ atg_status atg_build(atg_table* t, void* stream) {
     if (t->opts.interleave && t->sp_stream && !t->events) {
         t->lists_full = false;
         const BuildArgs a = t->args();
-        HIPCHK(launch_sum(a, s));
-        HIPCHK(launch_partition(a, s));
+        HIPCHK(launch_front(a, s));
         t->placed = true;
         hipError_t err = hipSuccess;
         if (build_split_pack_interleaved(t, a, s, err)) {
@@ -438,7 +437,14 @@ atg_status atg_build(atg_table* t, void* stream) {
     // Events follow TableSplitTimer's phases (utils/Timer.cu:62-77); the
     // prefix sums are fused into the partition, so that phase reads 0.
     static const int before[4] = {0, 1, 3, 4};  // event recorded before each phase
-    for (int ph = 0; ph < 4; ++ph) {
+    int first = 0;
+    if (!t->events) {
+        t->lists_full = false;
+        HIPCHK(launch_front(t->args(), s));
+        t->placed = true;
+        first = ATG_PHASE_SPLIT;
+    }
+    for (int ph = first; ph < 4; ++ph) {
         if (t->events && ph == 2) HIPCHK(hipEventRecord(t->ev[2], s));
         if (t->events) HIPCHK(hipEventRecord(t->ev[before[ph]], s));
         atg_status rc = atg_build_phase(t, ph, stream);

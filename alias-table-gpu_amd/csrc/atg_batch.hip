@@ -128,7 +128,7 @@ __global__ __launch_bounds__(64) void seg_local(SegArgs g, SegMap m) {
             next();
             continue;
         }
-        psa_section<T, true, PSA_MAX_LEN / 64, ROWS_LATER>(a, v - m.base[t], x, lds_raw, lane, next);
+        psa_section<T, true, PSA_MAX_LEN / 64, ROWS_LATER>(a, a.st->W_N, v - m.base[t], x, lds_raw, lane, next);
     }
 }
 

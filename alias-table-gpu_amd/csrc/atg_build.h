@@ -143,6 +143,11 @@ constexpr int64_t kDirectPrefixMax = 2048;
 int64_t block_tree_total(int64_t G);
 hipError_t launch_sum(const BuildArgs& a, hipStream_t s);
 hipError_t launch_partition(const BuildArgs& a, hipStream_t s);
+// launch_sum and launch_partition, up to kOwnSumMax sections without the
+// launch that finishes the sum: every partition wave does, while its weights
+// are on their way (builds, us: 100,003 items 43.8 -> 40.6, 2^20 65.1 -> 63.0).
+constexpr int64_t kOwnSumMax = 2048;
+hipError_t launch_front(const BuildArgs& a, hipStream_t s);
 hipError_t launch_partition_local(const BuildArgs& a, hipStream_t s);
 hipError_t launch_partition_place(const BuildArgs& a, hipStream_t s);
 hipError_t launch_degenerate(const BuildArgs& a, hipStream_t s);

@@ -40,17 +40,29 @@ __global__ __launch_bounds__(1024) void sum_finish(BuildArgs a) {
 // ... and loads each next section while the current one's chains run.
 // XU: weights per lane held for a section (sections of up to 64 XU items);
 // the short-section kernel keeps fewer registers, so more waves fit a SIMD.
-template <typename T, bool AOS, int XU, bool ROWS_LATER>
+// OWN_W: every wave sums the section sums to W itself, and the first one
+// writes the state (no sum_finish before).
+template <typename T, bool AOS, int XU, bool ROWS_LATER, bool OWN_W>
 __global__ __launch_bounds__(64) void partition_local(BuildArgs a) {
     extern __shared__ double lds_raw[];
-    if (a.st->error) return;
     const int lane = (int)threadIdx.x;
     T x[XU];
     int64_t s = blockIdx.x;
-    if (s < a.G) section_load<T>(a, s, lane, x);
+    double W_N;
+    if (OWN_W) {
+        if (s < a.G) section_load<T>(a, s, lane, x);
+        const double W = wave_weight_sum(a, lane);
+        if (s == 0 && lane == 0) sum_state(a, W);
+        if (sum_error(a, W)) return;
+        W_N = W / (double)a.n;
+    } else {
+        if (a.st->error) return;
+        if (s < a.G) section_load<T>(a, s, lane, x);
+        W_N = a.st->W_N;
+    }
     for (; s < a.G; s += gridDim.x) {
         const int64_t sn = s + gridDim.x;
-        psa_section<T, AOS, XU, ROWS_LATER>(a, s, x, lds_raw, lane, [&]() {
+        psa_section<T, AOS, XU, ROWS_LATER>(a, W_N, s, x, lds_raw, lane, [&]() {
             if (sn < a.G) section_load<T>(a, sn, lane, x);
         });
     }
@@ -271,10 +283,14 @@ __global__ __launch_bounds__(64) void pack_windowed(BuildArgs a, int64_t blk0) {
 // Host-side launchers.
 static inline unsigned blocks_for(int64_t items, int per) { return (unsigned)((items + per - 1) / per); }
 
-hipError_t launch_sum(const BuildArgs& a, hipStream_t s) {
+static void launch_sum_sections(const BuildArgs& a, hipStream_t s) {
     const unsigned g = blocks_for(a.G, 4);
     if (a.dtype_f32) hipLaunchKernelGGL(sum_sections<float>, dim3(g), dim3(256), 0, s, a);
     else hipLaunchKernelGGL(sum_sections<double>, dim3(g), dim3(256), 0, s, a);
+}
+
+hipError_t launch_sum(const BuildArgs& a, hipStream_t s) {
+    launch_sum_sections(a, s);
     hipLaunchKernelGGL(sum_finish, dim3(1), dim3(1024), 0, s, a);
     return hipGetLastError();
 }
@@ -300,24 +316,37 @@ int64_t block_tree_total(int64_t G) {
 // The partition phase in its two passes: the local pass (partition, PSA+
 // chains, staged leftovers, level-0 block sums), then the block tree and the
 // placement of the leftover lists (and the split certificate).
-template <bool ROWS_LATER>
-static void (*partition_local_kernel(bool f32, bool aos, int64_t Ls_max))(BuildArgs) {
+template <bool ROWS_LATER, bool OWN_W>
+static void (*partition_local_kernel(const BuildArgs& a))(BuildArgs) {
     constexpr int S = kShortSectionMax / 64, L = PSA_MAX_LEN / 64;
-    if (Ls_max <= kShortSectionMax)
-        return f32 ? (aos ? partition_local<float, true, S, ROWS_LATER> : partition_local<float, false, S, ROWS_LATER>)
-                   : (aos ? partition_local<double, true, S, ROWS_LATER> : partition_local<double, false, S, ROWS_LATER>);
-    return f32 ? (aos ? partition_local<float, true, L, ROWS_LATER> : partition_local<float, false, L, ROWS_LATER>)
-               : (aos ? partition_local<double, true, L, ROWS_LATER> : partition_local<double, false, L, ROWS_LATER>);
+    const bool f32 = a.dtype_f32 != 0, aos = a.rows != nullptr;
+    if (a.Ls_max <= kShortSectionMax)
+        return f32 ? (aos ? partition_local<float, true, S, ROWS_LATER, OWN_W> : partition_local<float, false, S, ROWS_LATER, OWN_W>)
+                   : (aos ? partition_local<double, true, S, ROWS_LATER, OWN_W> : partition_local<double, false, S, ROWS_LATER, OWN_W>);
+    return f32 ? (aos ? partition_local<float, true, L, ROWS_LATER, OWN_W> : partition_local<float, false, L, ROWS_LATER, OWN_W>)
+               : (aos ? partition_local<double, true, L, ROWS_LATER, OWN_W> : partition_local<double, false, L, ROWS_LATER, OWN_W>);
 }
 
-hipError_t launch_partition_local(const BuildArgs& a, hipStream_t s) {
+static hipError_t launch_partition_kernel(const BuildArgs& a, bool own_w, hipStream_t s) {
     const size_t lds = psa_lds_bytes(a.Ls_max);
-    const bool f32 = a.dtype_f32 != 0, aos = a.rows != nullptr;
-    void (*k)(BuildArgs) = partition_local_kernel<true>(f32, aos, a.Ls_max);
+    void (*k)(BuildArgs) = partition_local_kernel<true, false>(a);
     const int64_t resident = resident_blocks((const void*)k, 64, lds);
-    if (!rows_later_ok(a.G, resident)) k = partition_local_kernel<false>(f32, aos, a.Ls_max);
+    if (own_w) k = partition_local_kernel<false, true>(a);
+    else if (!rows_later_ok(a.G, resident)) k = partition_local_kernel<false, false>(a);
     hipLaunchKernelGGL(k, dim3((unsigned)std::min<int64_t>(a.G, resident)), dim3(64), lds, s, a);
     return hipGetLastError();
+}
+
+hipError_t launch_partition_local(const BuildArgs& a, hipStream_t s) { return launch_partition_kernel(a, false, s); }
+
+hipError_t launch_front(const BuildArgs& a, hipStream_t s) {
+    if (a.G > kOwnSumMax) {
+        const hipError_t e = launch_sum(a, s);
+        return e != hipSuccess ? e : launch_partition(a, s);
+    }
+    launch_sum_sections(a, s);
+    const hipError_t e = launch_partition_kernel(a, true, s);
+    return e != hipSuccess ? e : launch_partition_place(a, s);
 }
 
 hipError_t launch_partition(const BuildArgs& a, hipStream_t s) {

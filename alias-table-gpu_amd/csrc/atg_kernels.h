@@ -436,12 +436,10 @@ __device__ __forceinline__ void psa_chain_rows(const BuildArgs& a, SecLDS& L, in
 // ROWS_LATER: the chains record their steps and the wave writes the rows
 // afterwards (rows_later_ok says when).
 template <typename T, bool AOS, int XU, bool ROWS_LATER, typename AfterPartition>
-__device__ __forceinline__ void psa_section(const BuildArgs& a, int64_t s, T (&x)[XU],
+__device__ __forceinline__ void psa_section(const BuildArgs& a, double W_N, int64_t s, T (&x)[XU],
                                             double* lds_raw, int lane, AfterPartition after_partition) {
-    DevState* st = a.st;
     const int64_t start = min(a.n, s * a.Ls);
     const int len = (int)(min(a.n, (s + 1) * a.Ls) - start);
-    const double W_N = st->W_N;
     SecLDS L;
     L.w = lds_raw;
     L.idx = reinterpret_cast<uint16_t*>(lds_raw + a.Ls_max);
@@ -847,6 +845,29 @@ __device__ __forceinline__ void sum_sections_block(const BuildArgs& a, int64_t b
     }
 }
 
+// The error bits of a weight sum.
+__device__ __forceinline__ uint32_t sum_error(const BuildArgs& a, double W) {
+    uint32_t err = 0;
+    if (W != W) err = ERR_BAD_WEIGHT;
+    else if (!(W > 0.0) || W == __builtin_inf()) err = ERR_BAD_SUM;
+    if (a.Ls > a.Ls_max) err |= ERR_SECTION_TOO_LONG;
+    return err;
+}
+
+// The state at the start of a build with weight sum W.
+__device__ __forceinline__ void sum_state(const BuildArgs& a, double W) {
+    DevState* st = a.st;
+    st->W = W;
+    st->W_N = W / (double)a.n;
+    st->error = sum_error(a, W);
+    st->degenerate = 0;
+    st->cert_max_dL = 0ull;                    // +0.0
+    st->cert_min_dH = 0x7FF0000000000000ull;   // +inf
+    st->cert_done = 0;
+    st->split_fallbacks = 0;
+    st->learned_fallbacks = 0;
+}
+
 // W, pass 2 (one block): the 64-ary tree over the section sums, 64 values per
 // wave and level, zero-padded; W, W/N, the error bits and the state resets.
 __device__ __forceinline__ void sum_finish_block(const BuildArgs& a) {
@@ -876,25 +897,27 @@ __device__ __forceinline__ void sum_finish_block(const BuildArgs& a) {
         count = groups;
         if (count == 1) break;
     }
-    if (threadIdx.x == 0) {
-        const double W = src[0];
-        DevState* st = a.st;
-        uint32_t err = 0;
-        if (W != W) err = ERR_BAD_WEIGHT;
-        else if (!(W > 0.0) || W == __builtin_inf()) err = ERR_BAD_SUM;
-        if (a.Ls > a.Ls_max) err |= ERR_SECTION_TOO_LONG;
-        st->W = W;
-        st->W_N = W / (double)a.n;
-        st->error = err;
-        st->degenerate = 0;
-        st->cert_max_dL = 0ull;                    // +0.0
-        st->cert_min_dH = 0x7FF0000000000000ull;   // +inf
-        st->cert_done = 0;
-        st->split_fallbacks = 0;
-        st->learned_fallbacks = 0;
-    }
+    if (threadIdx.x == 0) sum_state(a, src[0]);
 }
 
+// W from the section sums by one wave, for at most 4096 sections: the tree of
+// sum_finish_block (two levels; one level's sum goes through the second, over
+// zeros, unchanged).
+__device__ __forceinline__ double wave_weight_sum(const BuildArgs& a, int lane) {
+    const int G = (int)a.G, groups = (G + 63) >> 6;
+    double t = 0.0;  // lane c: group c
+    for (int g0 = 0; g0 < groups; g0 += 8) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int i = (g0 + u) * 64 + lane;
+            v[u] = i < G ? a.section_sums[i] : 0.0;
+        }
+        const double t8 = wave_tree_sum8(v, lane);
+        if ((lane & ~7) == g0) t = t8;
+    }
+    return wave_tree_sum(t);
+}
 
 // ---------------------------------------------------------------------------
 // Pack helpers.

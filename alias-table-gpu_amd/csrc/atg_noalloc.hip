@@ -160,8 +160,7 @@ extern "C" atg_status atg_build_noalloc(const void* weights, atg_dtype dtype, in
     }
     hipLaunchKernelGGL(clear_state, dim3(1), dim3(64), 0, s, a.st);
     HIPCHK(hipGetLastError());
-    HIPCHK(launch_sum(a, s));
-    HIPCHK(launch_partition(a, s));
+    HIPCHK(launch_front(a, s));
     HIPCHK(o.split_method == ATG_SPLIT_LEARNED ? launch_split_learned(a, s)
            : o.split_method == ATG_SPLIT_PARY  ? launch_split_pary(a, s)
                                                : launch_split(a, s));

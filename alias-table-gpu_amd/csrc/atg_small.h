@@ -78,20 +78,9 @@ __device__ __forceinline__ void small_build(const BuildArgs& a, double* W_out, u
     __syncthreads();
     const double W = wave_tree_sum(lane < G ? ssum[lane] : 0.0);
     const double W_N = W / (double)a.n;
-    uint32_t err = 0;
-    if (W != W) err = ERR_BAD_WEIGHT;
-    else if (!(W > 0.0) || W == __builtin_inf()) err = ERR_BAD_SUM;
+    const uint32_t err = sum_error(a, W);
     if (tid == 0) {
-        DevState* st = a.st;
-        st->W = W;
-        st->W_N = W_N;
-        st->error = err;
-        st->degenerate = 0;
-        st->cert_max_dL = 0ull;
-        st->cert_min_dH = 0x7FF0000000000000ull;
-        st->cert_done = 0;
-        st->split_fallbacks = 0;
-        st->learned_fallbacks = 0;
+        sum_state(a, W);
         if (W_out) *W_out = W;
         if (error_out) *error_out = err;
     }
