@@ -54,6 +54,18 @@ struct BuildArgs {
 constexpr int kLightDirShift = 10;
 inline int64_t light_dir_size(int64_t n) { return (n >> kLightDirShift) + 2; }
 
+// The windowed pack runs every chain (of up to n / p items) at once; the staged
+// one as many as fit its pool, so in rounds whose number grows with n / p, and
+// the more waves there are, the more of that they hide for each other.  Whole
+// builds, staged and windowed, us: 1e7 items at n / p = 122 268 and 242, at
+// 100 246 and 254, at 200 447 and 249; 3e6 at 100 146 and 109; 3e7 at 200 769
+// and 702, at 122 652 and 694; 1e8 at 200 2,080 and 2,203, at 256 2,244 and
+// 2,198.
+inline bool pack_windowed_ok(int64_t n, int64_t p_req, int32_t pack_method) {
+    if (pack_method != PACK_CHUNKED || p_req <= 0) return false;
+    const int64_t per = n / p_req;
+    return per > 256 || (per >= 32 && 11 * per * per > p_req);
+}
 // Tables below this many items keep whole lists: finding a light in the
 // staging takes the pack a few dependent reads, which the smaller writes pay
 // for only where bandwidth counts (builds, us, lean against whole: 100,003
@@ -63,7 +75,7 @@ constexpr int64_t kLeanMin = (int64_t)1 << 21;
 // pool (chains hold at most n / p + 3 items, the pool at least
 // min(64 (n / p + 1), 1024)).
 inline bool lean_lights_ok(int64_t n, int64_t p_req, int32_t pack_method) {
-    return n >= kLeanMin && pack_method == PACK_CHUNKED && p_req > 0 && n / p_req <= 256;
+    return n >= kLeanMin && pack_method == PACK_CHUNKED && p_req > 0 && !pack_windowed_ok(n, p_req, pack_method);
 }
 
 // x / chains = x chain_mul >> 20 for x <= 2048 and chains <= 64: with M =
@@ -93,13 +105,6 @@ inline int32_t pack_cap_items(int64_t n, int64_t p_req) {
 // A pack round that fits fewer chains than this into the pool hands the
 // wave's remaining chains to their lanes, each reading the lists from HBM.
 constexpr int kPackMinStagedChains = 8;
-// Chains of more than this many items (n / p) run the windowed pack: so few
-// of them fit a pool round that the staged pack would hand nearly all of them
-// to their lanes.
-constexpr int64_t kPackWindowedItems = 256;
-inline bool pack_windowed_ok(int64_t n, int64_t p_req, int32_t pack_method) {
-    return pack_method == PACK_CHUNKED && p_req > 0 && n / p_req > kPackWindowedItems;
-}
 // Weight (8 B), item (4 B) and recorded alias (4 B) per pool item, and the
 // spare weight slot the light steps record into (16 B keep the alignment).
 inline size_t pack_lds_bytes(int32_t cap) { return (size_t)cap * 16 + 16; }

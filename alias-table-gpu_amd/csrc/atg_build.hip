@@ -159,19 +159,27 @@ __global__ __launch_bounds__(64) void pack_basic(BuildArgs a, int64_t blk0) {
 //     weight), and finally the wave writes the round's rows.  Windows are
 //     loaded and rows written a few chains per instruction, consecutive list
 //     entries on consecutive lanes, so that an instruction touches few lines.
-//     Blocks of 64 chains, as pack_staged.
-constexpr int kWinL = 16, kWinH = 8;
+//     Half a wave of chains to a wave: twice the waves load and write the
+//     windows (1e7 items, 50,000 chains, us: 64 chains a wave 97, 32 86, 16
+//     94; windows of 32 lights were no faster).  1e8 items at the default
+//     shape are bound by memory, the 12R bytes of the lists and the lines of
+//     the table read and written: 0.82 ms at R/N = 0.62, 0.96 ms (1.14 before
+//     the padded rows) at 0.90.
+constexpr int kWinChains = 32, kWinL = 16, kWinH = 8;
 template <bool AOS>
 __global__ __launch_bounds__(64) void pack_windowed(BuildArgs a, int64_t blk0) {
-    __shared__ double wl[kWinL][64], wh[kWinH][64];
-    __shared__ int32_t il[kWinL][64], ih[kWinH][64], al[kWinL][64], ah[kWinH][64];
+    constexpr int CH = kWinChains, NL = kWinL * CH / 64, NH = kWinH * CH / 64;
+    // A chain's window is a column; the odd row length keeps the accesses that
+    // run along a window off one bank.
+    __shared__ double wl[kWinL][CH + 1], wh[kWinH][CH + 1];
+    __shared__ int32_t il[kWinL][CH + 1], ih[kWinH][CH + 1], al[kWinL][CH + 1], ah[kWinH][CH + 1];
     const DevState* st = a.st;
     if (st->error || st->degenerate) return;
     const int64_t p = st->p;
     const int lane = (int)threadIdx.x;
-    const int64_t k0 = (blk0 + blockIdx.x) * 64;
+    const int64_t k0 = (blk0 + blockIdx.x) * CH;
     if (k0 + 1 > p) return;
-    const bool mine = k0 + lane < p;
+    const bool mine = lane < CH && k0 + lane < p;
     Split prev{0, 0, 0.0}, cur{0, 0, 0.0};
     if (mine) {
         prev = a.splits[k0 + lane];
@@ -193,38 +201,38 @@ __global__ __launch_bounds__(64) void pack_windowed(BuildArgs a, int64_t blk0) {
     while (__ballot(run) != 0ull) {
         // The windows: lights i .. i + kWinL - 1, heavies j .. j + kWinH - 1
         // (slot 0: the current heavy, whose residual is w).
-        // Staged a window at a time: one load instruction covers the window
+        // Staged a window at a time: one load instruction covers the windows
         // of 64 / kWinL chains (heavies: 64 / kWinH), kWinL consecutive list
         // entries each, so that it touches few lines.
         const int i0 = i, j0 = j;
         {
-            double vw[kWinL], hw[kWinH];
-            int32_t vi[kWinL], hv[kWinH];
+            double vw[NL], hw[NH];
+            int32_t vi[NL], hv[NH];
 #pragma unroll
-            for (int k = 0; k < kWinL; ++k) {
-                const int c = k * (64 / kWinL) + lane / kWinL, t = lane % kWinL;
+            for (int k = 0; k < NL; ++k) {
+                const int c = (k * 64 + lane) / kWinL, t = lane % kWinL;
                 const int q = min(__shfl(i0, c, 64) + t, __shfl(iLast, c, 64));
                 const bool load = __shfl((int)run, c, 64) != 0;
                 vw[k] = load ? a.Lw[q] : 0.0;
                 vi[k] = load ? a.Li[q] : 0;
             }
 #pragma unroll
-            for (int k = 0; k < kWinH; ++k) {
-                const int c = k * (64 / kWinH) + lane / kWinH, t = lane % kWinH;
+            for (int k = 0; k < NH; ++k) {
+                const int c = (k * 64 + lane) / kWinH, t = lane % kWinH;
                 const int q = min(__shfl(j0, c, 64) + t, __shfl(jUpper, c, 64));
                 const bool load = __shfl((int)run, c, 64) != 0;
                 hw[k] = load ? a.Hw[q] : 0.0;
                 hv[k] = load ? a.Hi[q] : 0;
             }
 #pragma unroll
-            for (int k = 0; k < kWinL; ++k) {
-                const int c = k * (64 / kWinL) + lane / kWinL, t = lane % kWinL;
+            for (int k = 0; k < NL; ++k) {
+                const int c = (k * 64 + lane) / kWinL, t = lane % kWinL;
                 wl[t][c] = vw[k];
                 il[t][c] = vi[k];
             }
 #pragma unroll
-            for (int k = 0; k < kWinH; ++k) {
-                const int c = k * (64 / kWinH) + lane / kWinH, t = lane % kWinH;
+            for (int k = 0; k < NH; ++k) {
+                const int c = (k * 64 + lane) / kWinH, t = lane % kWinH;
                 wh[t][c] = hw[k];
                 ih[t][c] = hv[k];
             }
@@ -264,14 +272,14 @@ __global__ __launch_bounds__(64) void pack_windowed(BuildArgs a, int64_t blk0) {
         // touches few table lines.
         const int nl = i - i0, nh = j - j0;
 #pragma unroll
-        for (int k = 0; k < kWinL; ++k) {
-            const int c = k * (64 / kWinL) + lane / kWinL, t = lane % kWinL;
+        for (int k = 0; k < NL; ++k) {
+            const int c = (k * 64 + lane) / kWinL, t = lane % kWinL;
             const int it = il[t][c];
             if (t < __shfl(nl, c, 64) && (uint32_t)it < (uint32_t)a.n) store_row<AOS>(a, it, wl[t][c], al[t][c]);
         }
 #pragma unroll
-        for (int k = 0; k < kWinH; ++k) {
-            const int c = k * (64 / kWinH) + lane / kWinH, t = lane % kWinH;
+        for (int k = 0; k < NH; ++k) {
+            const int c = (k * 64 + lane) / kWinH, t = lane % kWinH;
             const int it = ih[t][c];
             if (t < __shfl(nh, c, 64) && (uint32_t)it < (uint32_t)a.n) store_row<AOS>(a, it, wh[t][c], ah[t][c]);
         }
@@ -429,8 +437,10 @@ hipError_t launch_pack_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int
             else hipLaunchKernelGGL((pack_basic<false, true, double>), g, b, 0, s, a, b0);
         }
     } else if (pack_windowed_ok(a.n, a.p_req, a.pack_method) && !a.lean_lights) {
-        if (a.rows) hipLaunchKernelGGL(pack_windowed<true>, g, b, 0, s, a, b0);
-        else hipLaunchKernelGGL(pack_windowed<false>, g, b, 0, s, a, b0);
+        constexpr int64_t per = 64 / kWinChains;  // blocks of kWinChains chains
+        const dim3 gw((unsigned)((b1 - b0) * per));
+        if (a.rows) hipLaunchKernelGGL(pack_windowed<true>, gw, b, 0, s, a, b0 * per);
+        else hipLaunchKernelGGL(pack_windowed<false>, gw, b, 0, s, a, b0 * per);
     } else {
         if (a.rows) hipLaunchKernelGGL(pack_staged<true>, g, b, lds, s, a, b0);
         else hipLaunchKernelGGL(pack_staged<false>, g, b, lds, s, a, b0);

@@ -112,6 +112,10 @@ def test_small_noalloc_equals_table(gpu, layout, split):
     (50_000, 1000, "best_worst", 2),           # one split to find
     ((1 << 21) - 1, 2048, "pareto", 40_000),   # whole light lists
     (1 << 21, 2048, "pareto", 40_000),         # lean ones
+    (1_000_000, 1000, "pareto", 19_000),       # windowed pack, 52 items a chain
+    (1_000_000, 1000, "pareto", 26_000),       # staged, 38 items
+    (3_000_000, 1000, "zipf_shuffled", 30_000),  # windowed where the staged pack would have lean lists
+    (700_001, 2048, "exponential", 5_000),     # a last window block with one chain
     (300_000, 1000, "all_equal", 0),           # degenerate: filled by the split's launch
 ])
 def test_mid_size_routes_match_oracle(gpu, oracle, n, section, dist, p):
