@@ -651,7 +651,7 @@ atg_status atg_batch_create(atg_batch** out, const int64_t* offsets, int64_t nta
         a.Li = ip; a.Hi = ip + icap; a.stage_i = ip + 2 * icap; a.knot_j = ip + 3 * icap;
         a.sec_loff = reinterpret_cast<uint32_t*>(a.knot_j + align_up(o.learned_segments + 2, 64));
         a.sec_ldir = a.sec_loff + align_up(z.G + 1, 64);
-        a.lean_lights = lean_lights_ok(n, z.p_req, PACK_CHUNKED) ? 1 : 0;
+        a.lean_lights = batch_lean_ok(n, z.p_req) ? 1 : 0;
         a.rows = b->d_rows + offsets[t];
         a.tw = nullptr;
         a.ta = nullptr;

@@ -56,27 +56,36 @@ inline int64_t light_dir_size(int64_t n) { return (n >> kLightDirShift) + 2; }
 
 // The windowed pack runs every chain (of up to n / p items) at once; the staged
 // one as many as fit its pool, so in rounds whose number grows with n / p, and
-// the more waves there are, the more of that they hide for each other.  Whole
-// builds, staged and windowed, us: 1e7 items at n / p = 122 268 and 242, at
-// 100 246 and 254, at 200 447 and 249; 3e6 at 100 146 and 109; 3e7 at 200 769
-// and 702, at 122 652 and 694; 1e8 at 200 2,080 and 2,203, at 256 2,244 and
-// 2,198.
+// the more waves there are, the more of that they hide for each other.  Builds
+// with few and with many lights to a heavy, staged / windowed, us: 1e6 items
+// at n / p = 33 69.6 / 67.2 and 76.4 / 72.2; 3e6 at 50 105.6 / 100.8 and 115.6
+// / 111.1; 1e7 at 64 (staged by the rule) 237.8 / 244.2 and 283.2 / 258.6; 3e7
+// at 100 670 / 658 and 754 / 664; 1e8 at 100 (staged) 2,080 / 2,128 and 2,261 /
+// 2,120, at 150 2,041 / 2,062 and 2,542 / 2,141, at 200 2,077 / 2,055 and 2,826
+// / 2,116.
 inline bool pack_windowed_ok(int64_t n, int64_t p_req, int32_t pack_method) {
     if (pack_method != PACK_CHUNKED || p_req <= 0) return false;
     const int64_t per = n / p_req;
-    return per > 256 || (per >= 32 && 11 * per * per > p_req);
+    return per > 256 || (per >= 32 && 30 * per * per > p_req);
 }
 // Tables below this many items keep whole lists: finding a light in the
 // staging takes the pack a few dependent reads, which the smaller writes pay
 // for only where bandwidth counts (builds, us, lean against whole: 100,003
-// items 51.3 and 46.0, 2^20 71.1 and 71.0, 3e6 95.2 and 95.1, 1e7 244 and 253).
-constexpr int64_t kLeanMin = (int64_t)1 << 21;
-// The lean light lists need every pack chain to fit the staged pack's LDS
-// pool (chains hold at most n / p + 3 items, the pool at least
-// min(64 (n / p + 1), 1024)).
+// items 51.3 and 46.0, 2^20 71.1 and 71.0, 3e6 95.2 and 95.1, 1e7 244 and 253;
+// with the windowed pack 3e6 113.0 and 110.7, 5e6 158.2 and 159.0, 1e7 235.8
+// and 241.4, 1e8 of R/N = 0.62 and 0.90 1,977 and 2,159, 1,990 and 2,295).
+constexpr int64_t kLeanMin = (int64_t)1 << 21, kLeanMinWindowed = (int64_t)1 << 22;
 inline bool lean_lights_ok(int64_t n, int64_t p_req, int32_t pack_method) {
-    return n >= kLeanMin && pack_method == PACK_CHUNKED && p_req > 0 && !pack_windowed_ok(n, p_req, pack_method);
+    return pack_method == PACK_CHUNKED && p_req > 0 && n >= (pack_windowed_ok(n, p_req, pack_method) ? kLeanMinWindowed : kLeanMin);
 }
+
+// A batch packs with the staged kernel alone, whose LDS pool every chain of
+// a lean list has to fit (chains hold at most n / p + 3 items, the pool at
+// least min(64 (n / p + 1), 1024)).  Its tables share the card's bandwidth, so
+// they are lean at any size (us, lean against whole: 2,000 tables of 20,000
+// items 1,067 and 1,112, 512 of 200,000 2,404 and 2,507, 100 of 1e6 2,720 and
+// 2,800).
+inline bool batch_lean_ok(int64_t n, int64_t p_req) { return p_req > 0 && n / p_req <= 256; }
 
 // x / chains = x chain_mul >> 20 for x <= 2048 and chains <= 64: with M =
 // ceil(2^20 / C), x (M C - 2^20) < 2048 64 < 2^20.

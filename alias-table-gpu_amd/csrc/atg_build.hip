@@ -166,7 +166,10 @@ __global__ __launch_bounds__(64) void pack_basic(BuildArgs a, int64_t blk0) {
 //     the table read and written: 0.82 ms at R/N = 0.62, 0.96 ms (1.14 before
 //     the padded rows) at 0.90.
 constexpr int kWinChains = 32, kWinL = 16, kWinH = 8;
-template <bool AOS>
+//     LEAN: the lights come from the staging.  A chain's lights lie in one or
+//     few sections, so a lane keeps the staging position of its light list's
+//     start (lb) and the end of the section (le), where its window ends too.
+template <bool AOS, bool LEAN>
 __global__ __launch_bounds__(64) void pack_windowed(BuildArgs a, int64_t blk0) {
     constexpr int CH = kWinChains, NL = kWinL * CH / 64, NH = kWinH * CH / 64;
     // A chain's window is a column; the odd row length keeps the accesses that
@@ -186,14 +189,19 @@ __global__ __launch_bounds__(64) void pack_windowed(BuildArgs a, int64_t blk0) {
         cur = a.splits[k0 + lane + 1];
     }
     const double W_N = st->W_N;
-    const GlobalLists gl{a.Li, a.Hi, a.Lw, a.Hw};
     if (__ballot(mine && !(prev.i <= cur.i && prev.j <= cur.j)) != 0ull) {
-        if (mine) pack_chain<AOS>(a, gl, prev, cur, W_N);  // a bisection fell back: no windows
+        // A bisection fell back: no windows.
+        if (mine) {
+            if (LEAN) pack_chain<AOS>(a, LeanLists{a.Hi, a.Hw, a.sec_loff, a.stage_w, a.stage_i, a.G, a.Ls, a.n}, prev, cur, W_N);
+            else pack_chain<AOS>(a, GlobalLists{a.Li, a.Hi, a.Lw, a.Hw}, prev, cur, W_N);
+        }
         return;
     }
+    const double* lightW = LEAN ? a.stage_w : a.Lw;
+    const int32_t* lightI = LEAN ? a.stage_i : a.Li;
     const int iUpper = cur.i, jUpper = cur.j;
     int i = prev.i, j = prev.j;
-    const int iLast = max(iUpper - 1, i);  // list reads are clamped as in pack_chain
+    int lb = 0, le = LEAN ? i : iUpper;  // light q < le is at lb + q
     double w = prev.spill;
     if (mine && prev.spill == 0) w = a.Hw[j];
     bool run = mine;
@@ -205,16 +213,18 @@ __global__ __launch_bounds__(64) void pack_windowed(BuildArgs a, int64_t blk0) {
         // of 64 / kWinL chains (heavies: 64 / kWinH), kWinL consecutive list
         // entries each, so that it touches few lines.
         const int i0 = i, j0 = j;
+        if (LEAN && run && i < iUpper && i >= le) light_section(a, st->numL - 1, i, lb, le);
+        const int nw = run ? min(min(le, iUpper) - i, kWinL) : 0;  // lights in the window
         {
             double vw[NL], hw[NH];
             int32_t vi[NL], hv[NH];
 #pragma unroll
             for (int k = 0; k < NL; ++k) {
                 const int c = (k * 64 + lane) / kWinL, t = lane % kWinL;
-                const int q = min(__shfl(i0, c, 64) + t, __shfl(iLast, c, 64));
-                const bool load = __shfl((int)run, c, 64) != 0;
-                vw[k] = load ? a.Lw[q] : 0.0;
-                vi[k] = load ? a.Li[q] : 0;
+                const int q = __shfl(lb + i0, c, 64) + t;
+                const bool load = t < __shfl(nw, c, 64);
+                vw[k] = load ? lightW[q] : 0.0;
+                vi[k] = load ? lightI[q] : 0;
             }
 #pragma unroll
             for (int k = 0; k < NH; ++k) {
@@ -248,7 +258,7 @@ __global__ __launch_bounds__(64) void pack_windowed(BuildArgs a, int64_t blk0) {
             // a heavy remains; a light step otherwise (pack_chain's rule).
             const bool ex = idone || (w <= thr && !jdone);
             const int sl = i - i0, sh = j - j0;
-            if (ex ? sh + 1 >= kWinH : sl >= kWinL) break;  // past the window: restage
+            if (ex ? sh + 1 >= kWinH : sl >= nw) break;  // past the window: restage
             // sh < kWinH always (a heavy step needs slot sh + 1); sl can
             // reach kWinL on a heavy step, whose light is not used.
             const int tl = min(sl, kWinL - 1), th1 = min(sh + 1, kWinH - 1);
@@ -436,11 +446,16 @@ hipError_t launch_pack_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int
             if (a.rows) hipLaunchKernelGGL((pack_basic<true, true, double>), g, b, 0, s, a, b0);
             else hipLaunchKernelGGL((pack_basic<false, true, double>), g, b, 0, s, a, b0);
         }
-    } else if (pack_windowed_ok(a.n, a.p_req, a.pack_method) && !a.lean_lights) {
+    } else if (pack_windowed_ok(a.n, a.p_req, a.pack_method)) {
         constexpr int64_t per = 64 / kWinChains;  // blocks of kWinChains chains
         const dim3 gw((unsigned)((b1 - b0) * per));
-        if (a.rows) hipLaunchKernelGGL(pack_windowed<true>, gw, b, 0, s, a, b0 * per);
-        else hipLaunchKernelGGL(pack_windowed<false>, gw, b, 0, s, a, b0 * per);
+        if (a.lean_lights) {
+            if (a.rows) hipLaunchKernelGGL((pack_windowed<true, true>), gw, b, 0, s, a, b0 * per);
+            else hipLaunchKernelGGL((pack_windowed<false, true>), gw, b, 0, s, a, b0 * per);
+        } else {
+            if (a.rows) hipLaunchKernelGGL((pack_windowed<true, false>), gw, b, 0, s, a, b0 * per);
+            else hipLaunchKernelGGL((pack_windowed<false, false>), gw, b, 0, s, a, b0 * per);
+        }
     } else {
         if (a.rows) hipLaunchKernelGGL(pack_staged<true>, g, b, lds, s, a, b0);
         else hipLaunchKernelGGL(pack_staged<false>, g, b, lds, s, a, b0);

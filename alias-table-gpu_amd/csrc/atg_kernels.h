@@ -1015,6 +1015,22 @@ __device__ __forceinline__ int64_t light_positions(const BuildArgs& a, int64_t s
     }
 }
 
+// Lean lists, per lane: the section that holds light i < nL, as the base lb
+// (light q of the section lies at lb + q) and the end le > i of its lights.
+// The section lies between those of the directory entries around i.
+__device__ __forceinline__ void light_section(const BuildArgs& a, int64_t nL, int i, int& lb, int& le) {
+    const int64_t q = i >> kLightDirShift;
+    int lo = (int)a.sec_ldir[q];
+    int hi = ((q + 1) << kLightDirShift) < nL ? (int)a.sec_ldir[q + 1] : (int)(a.G - 1);
+    while (lo < hi) {
+        const int mid = (int)(((int64_t)lo + hi + 1) >> 1);
+        if (a.sec_loff[mid] <= (uint32_t)i) lo = mid;
+        else hi = mid - 1;
+    }
+    lb = (int)(min(a.n, lo * a.Ls) - (int64_t)a.sec_loff[lo]);
+    le = (int)a.sec_loff[lo + 1];
+}
+
 // Per-lane access to lean lists (the pack's fallback for non-monotone
 // splits): a bisection over sec_loff per light.
 struct LeanLists {

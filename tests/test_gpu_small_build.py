@@ -111,15 +111,25 @@ def test_small_noalloc_equals_table(gpu, layout, split):
     (400_000, 1000, "heavy_mix", 32_769),
     (50_000, 1000, "best_worst", 2),           # one split to find
     ((1 << 21) - 1, 2048, "pareto", 40_000),   # whole light lists
-    (1 << 21, 2048, "pareto", 40_000),         # lean ones
-    (1_000_000, 1000, "pareto", 19_000),       # windowed pack, 52 items a chain
-    (1_000_000, 1000, "pareto", 26_000),       # staged, 38 items
-    (3_000_000, 1000, "zipf_shuffled", 30_000),  # windowed where the staged pack would have lean lists
+    (1 << 21, 2048, "pareto", 100_000),        # lean ones
+    (1_000_000, 1000, "pareto", 30_700),       # windowed pack, 32 items a chain
+    (1_000_000, 1000, "pareto", 31_000),       # staged
+    ((1 << 22) - 1, 2048, "pareto", 40_000),   # windowed with whole light lists
+    (1 << 22, 2048, "pareto", 40_000),         # with lean ones
+    (4_300_000, 90, "unit_uniform", 2_000),    # lean: sections of few lights or none
+    (4_300_000, 2048, "ascending", 9_001),     # lean: the lights in the first sections
+    (4_300_000, 1024, "descending", 9_001),    # lean: in the last
+    (4_300_000, 500, "heavy_mix", 5),          # lean: long chains over many sections
     (700_001, 2048, "exponential", 5_000),     # a last window block with one chain
     (300_000, 1000, "all_equal", 0),           # degenerate: filled by the split's launch
 ])
 def test_mid_size_routes_match_oracle(gpu, oracle, n, section, dist, p):
-    w = np.full(n, 2.5) if dist == "all_equal" else weights(n, dist)
+    if dist == "all_equal":
+        w = np.full(n, 2.5)
+    elif dist in ("ascending", "descending"):
+        w = np.sort(weights(n, "pareto"))[::1 if dist == "ascending" else -1].copy()
+    else:
+        w = weights(n, dist)
     p_req = p if p > 0 else 81920
     for layout in ("aos", "soa"):
         t = gpu_build(w, layout=layout, section_size=section, num_splits=p_req)
