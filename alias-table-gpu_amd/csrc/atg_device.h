@@ -93,6 +93,21 @@ __device__ __forceinline__ int lane_id() { return __lane_id(); }
 // section per wave) stay uniform, so tests on them are scalar branches.
 __device__ __forceinline__ int wave_in_block() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
+// Lanes below this one whose bit of m is set.
+__device__ __forceinline__ int lanes_below(uint64_t m) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// Orders one wave's LDS writes before its later LDS reads by other lanes.  A
+// wave's LDS operations execute in issue order, so wavefront-scope fences
+// (compiler barriers, no wait instructions) suffice; a workgroup-scope fence
+// would also wait for every outstanding global store of the wave.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ double shfl_xor_d(double v, int m) { return __shfl_xor(v, m, ATG_WAVE); }
 __device__ __forceinline__ double shfl_up_d(double v, int d) { return __shfl_up(v, d, ATG_WAVE); }
 __device__ __forceinline__ double shfl_d(double v, int src) { return __shfl(v, src, ATG_WAVE); }

@@ -10,16 +10,6 @@
 
 namespace atg {
 
-// Orders one wave's LDS writes before its later LDS reads by other lanes.  A
-// wave's LDS operations execute in issue order, so wavefront-scope fences
-// (compiler barriers, no wait instructions) suffice; a workgroup-scope fence
-// would also wait for every outstanding global store of the wave.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // ---------------------------------------------------------------------------
 // 1. Section sums.  Lane l of the wave that owns a section adds items
 //    l, l+64, ... in order; the lane sums meet in the pairwise tree.  A NaN,

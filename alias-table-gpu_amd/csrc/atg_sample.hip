@@ -406,11 +406,12 @@ __global__ __launch_bounds__(CACHED ? kHistThreads : 256) void sample_sectioned_
 #define REJ_TASK 4096   // slots per task
 #define REJ_LONG_BLOCKS 1024
 
-// A is written once and read only by a later sampling launch: streaming
-// (non-temporal) 16-byte stores.
+// A slot in one 16-byte store.  A pass's 64 slots begin and end inside a line;
+// the cache joins the pieces, which streaming stores would send to memory one
+// by one (fill of 2e7 items, 3.5e7 slots: 175 us streaming, 153 cached).
 typedef unsigned int rej_u4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void rej_store(RejEntry* p, const RejEntry& e) {
-    __builtin_nontemporal_store(*reinterpret_cast<const rej_u4*>(&e), reinterpret_cast<rej_u4*>(p));
+    *reinterpret_cast<rej_u4*>(p) = *reinterpret_cast<const rej_u4*>(&e);
 }
 
 // Per-block totals of the counts.  The block's 16 loads per thread are issued
@@ -500,13 +501,17 @@ __global__ __launch_bounds__(1024) void rej_scan_totals(RejArgs a) {
 // lanes.  In a wave with more than REJ_WAVE_BUDGET slots, the rest of a run
 // longer than REJ_WAVE slots becomes tasks of REJ_TASK slots for
 // rej_fill_long, so that heavy items, however clustered, hold up no wave for
-// long; a wave within the budget writes every run itself.
+// long; a wave within the budget writes every run itself.  2e7 items (160 MB),
+// 3.5e7 slots (560 MB): 153 us, 199 with a search per slot and streaming
+// stores.
 template <typename T>
 __global__ __launch_bounds__(REJ_THREADS) void rej_fill(RejArgs a) {
     constexpr int U = REJ_ITEMS / REJ_THREADS;
     __shared__ uint64_t wtot[REJ_THREADS / 64];
     __shared__ uint32_t wtask[REJ_THREADS / 64];
     __shared__ uint32_t task_base;
+    __shared__ double marks[REJ_THREADS / 64][64];
+    constexpr double kNoStart = 2.0;
     if (a.st->error) return;
     const double W = a.st->W;
     const T* w = (const T*)a.weights;
@@ -554,19 +559,24 @@ __global__ __launch_bounds__(REJ_THREADS) void rej_fill(RejArgs a) {
         t_run = task_base;
         for (int q = 0; q < wave; ++q) t_run += wtask[q];
     }
+    double* mark = marks[wave];
+    mark[lane] = kNoStart;
     for (int u = 0; u < U; ++u) {
         const int k = u * 64 + lane;
         // A round's counts sum to at most |A| <= 2n < 2^32: 32-bit scans.
         const uint32_t cu = c[u];
         const uint32_t incl = wave_incl_scan_u32(cu);
         const uint64_t first = first0 + (incl - cu);
+        const uint64_t round0 = first0;
         first0 += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
         const int32_t item = (int32_t)(base + k);
         const double x = ((double)a.n * (double)wr[u]) / W;
         const double frac = x - floor(x);
         // The round's slots in the wave, long runs counted by their first slot
-        // only: lane v of each pass writes the v-th of them, owned by the
-        // last item whose local start is <= v (a search over the 64 starts).
+        // only: lane v of each pass writes the v-th of them.  The items leave
+        // their fractions (below 1) at their first slots' places in LDS, so
+        // that the owner of a slot is the number of starts up to it (a search
+        // over the 64 starts takes six dependent exchanges).
         const bool long_run = k < cnt && cu > long_min;
         const uint64_t any_long = __ballot(long_run);
         uint32_t lex = incl - cu, L = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
@@ -576,26 +586,26 @@ __global__ __launch_bounds__(REJ_THREADS) void rej_fill(RejArgs a) {
             lex = il - ell;
             L = (uint32_t)__builtin_amdgcn_readlane((int)il, 63);
         }
+        int o0 = (int)(base + u * 64) - 1;  // the item of the last start before the pass
         for (uint32_t v0 = 0; v0 < L; v0 += 64) {
             const uint32_t v = v0 + lane;
-            int o = 0;
-            uint32_t lo_start = 0;
-#pragma unroll
-            for (int step = 32; step >= 1; step >>= 1) {
-                const uint32_t st = (uint32_t)__shfl((int)lex, o + step, 64);
-                if (st <= v) {
-                    o += step;
-                    lo_start = st;
-                }
-            }
-            const uint64_t f = (uint64_t)__shfl((unsigned long long)first, o, 64);
-            const double fr = __shfl(frac, o, 64);
+            if (cu != 0 && lex - v0 < 64u) mark[lex - v0] = frac;
+            wave_lds_sync();
+            const double m = mark[lane];
+            mark[lane] = kNoStart;
+            wave_lds_sync();
+            const bool start = m < 1.0;
+            const uint64_t starts = __ballot(start);
+            const int o = o0 + lanes_below(starts) + (start ? 1 : 0);
+            o0 += __popcll(starts);
+            uint64_t f = round0;
+            if (any_long != 0ull) f = (uint64_t)__shfl((unsigned long long)(first - lex), o & 63, 64);
             if (v < L) {
                 RejEntry e;
-                e.accept = (v == lo_start) ? fr : 1.0;
-                e.item = (int32_t)(base + u * 64 + o);
+                e.accept = start ? m : 1.0;
+                e.item = o;
                 e.pad = 0;
-                rej_store(&a.A[f + (v - lo_start)], e);
+                rej_store(&a.A[f + v], e);
             }
         }
         if (any_long != 0ull) {
@@ -831,30 +841,37 @@ __global__ __launch_bounds__(REJ_SEC_THREADS) void rej_sample_sectioned(RejSecAr
     __syncthreads();
     const uint64_t cnt = a.sec_counts[2 * k], end = a.sec_counts[2 * k + 1] + cnt;
     uint64_t csum = 0;
+    const int lane = threadIdx.x & 63, wave = wave_in_block();
     // Runs of outputs that share the counter's high word (one, nearly always).
     for (uint64_t b = end - cnt; b < end;) {
-        const uint32_t hi = (uint32_t)(b >> 32);
-        const PhiloxStream ps(hi, PURPOSE_REJ_SECTIONED, sa.seed);
-        const uint64_t seg_end = min(end, ((uint64_t)hi + 1) << 32);
-        // One trial per iteration; a lane whose trial accepts goes on to its
-        // next sample at once, so no lane waits for another lane's rejected
-        // trials (the trials of every sample are those of the
-        // one-sample-at-a-time loop).
-        uint32_t left = (uint32_t)((seg_end - b + REJ_SEC_THREADS - 1 - threadIdx.x) / REJ_SEC_THREADS);
-        uint32_t t = threadIdx.x, tr = 0;
-        while (left != 0) {
+        const PhiloxStream ps((uint32_t)(b >> 32), PURPOSE_REJ_SECTIONED, sa.seed);
+        const uint64_t seg_end = min(end, ((b >> 31) + 1) << 31);
+        // Each wave takes a share of the run.  One trial per iteration; the
+        // lanes whose trials accept go on to the share's next samples at once,
+        // whichever lane that is, so that no lane waits for another's
+        // rejected trials before the share runs out (the trials of every
+        // sample are those of the one-sample-at-a-time loop).  Bound by the
+        // trials' Philox rounds: 1e8 samples at 1.74 trials each 0.58 ms with
+        // a fixed set of samples a lane, 0.39 so.
+        const uint32_t m = (uint32_t)(seg_end - b);
+        const uint32_t per = (m + REJ_SEC_THREADS / 64 - 1) / (REJ_SEC_THREADS / 64);
+        const uint32_t w0 = min(m, (uint32_t)wave * per), w1 = min(m, w0 + per);
+        uint32_t t = w0 + lane, tr = 0, next = w0 + 64;
+        while (__ballot(t < w1) != 0ull) {
             const u32x4 r = ps.at((uint32_t)b + t, tr);
             const ulonglong2 v = rsect[scale64(word64(r), len)];
             ++tr;
-            if (coin64(r) <= v.x || tr >= REJ_SECTIONED_MAX_TRIALS) {
+            const bool done = t < w1 && (coin64(r) <= v.x || tr >= REJ_SECTIONED_MAX_TRIALS);
+            const uint64_t dones = __ballot(done);
+            if (done) {
                 const int32_t item = (int32_t)v.y;
                 if (sa.out) (sa.out + b)[t] = item;
                 if (CACHED) hc.add(sa.hist, item);
                 if (sa.checksum) csum += (uint64_t)(uint32_t)item;
-                t += REJ_SEC_THREADS;
+                t = next + lanes_below(dones);
                 tr = 0;
-                --left;
             }
+            next += (uint32_t)__popcll(dones);
         }
         b = seg_end;
     }
