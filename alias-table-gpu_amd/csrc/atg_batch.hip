@@ -207,17 +207,19 @@ __global__ __launch_bounds__(64) void seg_pack(SegArgs g, SegMap m) {
     tick_end(g, t);
 }
 
-// Small tables, a workgroup of one wave each from start to end (atg_small.h),
-// bound by the latency of its chains (30 us for 2,000 items).  16,384 tables
-// of 16 to 4,096 items, half of the items in tables of one section: 0.51 ms
-// through the phases alone, 0.39 with the classes before them, 0.30 with the
-// classes beside them.
+// Small tables, a workgroup each from start to end (atg_small.h), bound by
+// latency (30 us for 2,900 items in two sections, 9 of them the chains' steps),
+// so by how many fit a CU.  16,384 tables of 16 to 4,096 items: 0.51 ms through
+// the phases, 0.23 here.  Default shape, phases and here, us: 4,096 tables of
+// 3,800 items 658 and 267, 2,000 of 8,000 475 and 289, of 12,500 623 and 378; 8
+// of 12,000 66 and 55, of 2,000 58 and 33.
 template <typename T, int XU>
-__global__ __launch_bounds__(64) void seg_small(SegArgs g, SegMap m) {
+__global__ __launch_bounds__(64 * (64 * XU <= kShortSectionMax ? kSmallMaxWaves : kSmallLongWaves))
+void seg_small(SegArgs g, const int32_t* tab) {
     extern __shared__ double lds_raw[];
-    const int64_t t = m.tab[blockIdx.x];
+    const int64_t t = tab[blockIdx.x];
     if (threadIdx.x == 0) g.ticks[2 * t] = (uint64_t)wall_clock64();
-    small_build<T, true, XU, false>(table_args(g, t), nullptr, nullptr, lds_raw);
+    small_build<T, true, XU, false, true>(table_args(g, t), nullptr, nullptr, lds_raw);
     if (threadIdx.x == 0) g.ticks[2 * t + 1] = (uint64_t)wall_clock64();
 }
 
@@ -248,15 +250,23 @@ __global__ __launch_bounds__(256) void batch_sample(BatchSampleArgs a) {
 
 using namespace atg;
 
-enum { MAP_SUM, MAP_LOCAL, MAP_PLACE, MAP_DEG, MAP_SPLIT, MAP_KNOTS, MAP_PACK, MAP_TREE, MAP_ONE, MAP_SMALL, MAP_COUNT = MAP_SMALL + 4 };
+enum { MAP_SUM, MAP_LOCAL, MAP_PLACE, MAP_DEG, MAP_SPLIT, MAP_KNOTS, MAP_PACK, MAP_TREE, MAP_ONE, MAP_COUNT };
 
-// Classes of tables built by seg_small, by their one section's length: chunks
-// of 64 items a lane holds.  A class has one launch, with the LDS of its
-// largest table, so that small tables are not held to the occupancy of larger
-// ones.
-constexpr int kSmallClasses = MAP_COUNT - MAP_SMALL;
-constexpr int kSmallChunks[kSmallClasses] = {2, 8, 16, 32};
-constexpr size_t kBatchSmallLds = 50 * 1024;
+// Tables built by seg_small, in classes by their sections' length (kSmallChunks
+// chunks of 64 items a lane) and number (waves, a power of two) and by how
+// many tables fit a CU (one, two, more).  A class has one launch, with the LDS
+// of its largest table, so that small tables are not held to the occupancy of
+// larger ones; finer classes lose more at the ends of their launches than
+// occupancy gains (16,384 tables of 16 to 4,096 items 230 us, 238 with four
+// more tiers of LDS below 32 KB).
+constexpr int kSmallChunks[] = {2, 8, 16, 32};
+constexpr size_t kSmallTiers[] = {52 * 1024, 79 * 1024, 154 * 1024};  // of 160 KB, static LDS aside
+struct SmallClass {
+    int xu;            // index into kSmallChunks
+    int waves, tier;
+    int threads = 64;  // of the table with the most sections
+    size_t lds = 0;    // of the largest table
+};
 // Small tables hold at least one item in this many, or go through the phases
 // (100 of them among 1,024 tables of up to 2^20 items: 3.06 ms in the phases,
 // 3.10 by themselves).
@@ -266,6 +276,13 @@ constexpr int64_t kBatchSmallShare = 8;
 // per table) and the group's most sections of a table (tree levels).
 struct BatchGroup {
     SegMap maps[MAP_COUNT];
+    struct Small {
+        int cls;             // index into the batch's small_classes
+        const int32_t* tab;  // its tables
+        int64_t blocks;
+        int on;              // side stream; 2: the build's own
+    };
+    std::vector<Small> small;  // largest sections first
     int64_t G_max = 1;
     int64_t items = 0;
     int64_t ntables = 0;
@@ -281,7 +298,7 @@ struct atg_batch_s {
     int64_t Ls_max = 1;
     int32_t pack_cap_max = 16;          // largest pack LDS pool of the tables (items)
     std::vector<int8_t> small_class;    // table -> class of seg_small, -1: the phases
-    size_t small_lds[kSmallClasses] = {};  // LDS of the class's largest table
+    std::vector<SmallClass> small_classes;
     // Streams the small classes run on beside the phases, forked from and
     // joined to the build's stream.
     hipStream_t side[2] = {};
@@ -344,12 +361,18 @@ void bind_weights(atg_batch* b) {
         b->args[t].weights = (const char*)b->d_weights + (size_t)b->offsets[t] * es;
 }
 
-// The tables of class C of a group.
-template <typename T, int C>
-void launch_class(const atg_batch* b, const SegArgs& g, const BatchGroup& grp, hipStream_t s) {
-    const SegMap& m = grp.maps[MAP_SMALL + C];
-    if (m.blocks > 0)
-        hipLaunchKernelGGL((seg_small<T, kSmallChunks[C]>), dim3((unsigned)m.blocks), dim3(64), b->small_lds[C], s, g, m);
+// A class's tables of a group.
+template <typename T>
+hipError_t launch_class(const SmallClass& c, const SegArgs& g, const BatchGroup::Small& sm, hipStream_t s) {
+    static_assert(sizeof(kSmallChunks) / sizeof(int) == 4, "a kernel per length");
+    void (*const k[])(SegArgs, const int32_t*) = {seg_small<T, kSmallChunks[0]>, seg_small<T, kSmallChunks[1]>,
+                                                  seg_small<T, kSmallChunks[2]>, seg_small<T, kSmallChunks[3]>};
+    if (c.lds > kSmallLdsDefault) {
+        const hipError_t e = hipFuncSetAttribute((const void*)k[c.xu], hipFuncAttributeMaxDynamicSharedMemorySize, (int)c.lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(k[c.xu], dim3((unsigned)sm.blocks), dim3(c.threads), c.lds, s, g, sm.tab);
+    return hipSuccess;
 }
 
 #define HIP_TRY(call)                        \
@@ -373,26 +396,18 @@ hipError_t launch_batch(const atg_batch* b, hipStream_t s) {
         // map below (MAP_KNOTS and MAP_TREE are checked: a group of
         // one-section tables has no tree blocks).
         // The small classes share nothing with the phases or each other, and
-        // each is a few rounds of latency: they run beside the phases, the
-        // class of the longest tables by itself, and join the stream before
-        // the group ends.
-        const bool classes[2] = {M[MAP_SMALL + 3].blocks > 0,
-                                 M[MAP_SMALL].blocks + M[MAP_SMALL + 1].blocks + M[MAP_SMALL + 2].blocks > 0};
+        // each is a few rounds of latency: they run beside the phases on two
+        // streams (without phases, on the build's and one more), which join
+        // the build's before the group ends.
         const bool phases = M[MAP_SUM].blocks > 0;
-        hipStream_t on[2] = {s, s};
-        if (phases || (classes[0] && classes[1])) {
-            if (classes[0] || classes[1]) HIP_TRY(hipEventRecord(b->ev_fork, s));
-            for (int k = 0; k < 2; ++k)
-                if (classes[k] && (phases || k == 0)) {
-                    on[k] = b->side[k];
-                    HIP_TRY(hipStreamWaitEvent(on[k], b->ev_fork, 0));
-                }
-        }
-        static_assert(kSmallClasses == 4, "a launch per class");
-        launch_class<T, 3>(b, g, grp, on[0]);
-        launch_class<T, 2>(b, g, grp, on[1]);
-        launch_class<T, 1>(b, g, grp, on[1]);
-        launch_class<T, 0>(b, g, grp, on[1]);
+        hipStream_t on[3] = {b->side[0], b->side[1], s};
+        bool used[2] = {false, false};
+        for (const BatchGroup::Small& sm : grp.small)
+            if (sm.on < 2) used[sm.on] = true;
+        if (used[0] || used[1]) HIP_TRY(hipEventRecord(b->ev_fork, s));
+        for (int k = 0; k < 2; ++k)
+            if (used[k]) HIP_TRY(hipStreamWaitEvent(on[k], b->ev_fork, 0));
+        for (const BatchGroup::Small& sm : grp.small) HIP_TRY(launch_class<T>(b->small_classes[sm.cls], g, sm, on[sm.on]));
         if (phases) {
             hipLaunchKernelGGL(seg_sum<T>, grid(M[MAP_SUM]), dim3(256), 0, s, g, M[MAP_SUM]);
             hipLaunchKernelGGL(seg_sum_finish, grid(M[MAP_ONE]), dim3(256), 0, s, g, M[MAP_ONE]);
@@ -416,7 +431,7 @@ hipError_t launch_batch(const atg_batch* b, hipStream_t s) {
             hipLaunchKernelGGL(seg_pack, grid(M[MAP_PACK]), dim3(64), pack_lds_bytes(b->pack_cap_max), s, g, M[MAP_PACK]);
         }
         for (int k = 0; k < 2; ++k)
-            if (on[k] != s) {
+            if (used[k]) {
                 HIP_TRY(hipEventRecord(b->ev_join[k], on[k]));
                 HIP_TRY(hipStreamWaitEvent(s, b->ev_join[k], 0));
             }
@@ -460,7 +475,7 @@ atg_status make_groups(atg_batch* b, int64_t group_items) {
     auto blocks_of = [&](int ph, int64_t t) -> int64_t {
         const BuildArgs& a = b->args[t];
         const int64_t K = std::min<int64_t>(a.learned_segments, a.p_req);
-        if (ph >= MAP_SMALL || b->small_class[t] >= 0) return ph == MAP_SMALL + b->small_class[t] ? 1 : 0;
+        if (b->small_class[t] >= 0) return 0;
         switch (ph) {
             case MAP_SUM: return (a.G + 3) / 4;
             case MAP_LOCAL: return a.G;
@@ -491,6 +506,33 @@ atg_status make_groups(atg_batch* b, int64_t group_items) {
             if (nblk > 0x7FFFFFFF) return fail(ATG_EINVAL, "batch: %lld blocks in one launch", (long long)nblk);
             groups[g].maps[ph].blocks = nblk;
         }
+    // The small classes of each group, each on the stream with the least work
+    // so far, those of the longest sections first.  A table's start and end
+    // cost about as much as 300 items.
+    std::vector<int64_t> small_start;
+    for (int64_t g = 0; g < ngroups; ++g) {
+        int64_t load[3] = {0, 0, 0};
+        const int streams = groups[g].maps[MAP_SUM].blocks > 0 ? 2 : 3;
+        for (int c = (int)b->small_classes.size() - 1; c >= 0; --c) {
+            if (b->small_classes[c].lds == 0) continue;  // no tables
+            BatchGroup::Small sm{c, nullptr, 0, 0};
+            const int64_t at = (int64_t)tab.size();
+            int64_t work = 0;
+            for (int64_t t : members[g])
+                if (b->small_class[t] == c) {
+                    tab.push_back((int32_t)t);
+                    work += offsets[t + 1] - offsets[t] + 300;
+                }
+            sm.blocks = (int64_t)tab.size() - at;
+            if (sm.blocks == 0) continue;
+            sm.on = streams - 1;
+            for (int k = streams - 2; k >= 0; --k)
+                if (load[k] < load[sm.on]) sm.on = k;
+            load[sm.on] += work;
+            small_start.push_back(at);
+            groups[g].small.push_back(sm);
+        }
+    }
     int32_t* d_tab = nullptr;
     int64_t* d_base = nullptr;
     if (dalloc(&d_tab, tab.size()) != hipSuccess || dalloc(&d_base, base.size()) != hipSuccess) {
@@ -510,6 +552,9 @@ atg_status make_groups(atg_batch* b, int64_t group_items) {
             m.tab = d_tab + map_start[(size_t)ph * ngroups + g];
             m.base = d_base + (size_t)ph * ntables;
         }
+    size_t next_small = 0;
+    for (int64_t g = 0; g < ngroups; ++g)
+        for (BatchGroup::Small& sm : groups[g].small) sm.tab = d_tab + small_start[next_small++];
     // The old maps may still be read by enqueued launches.
     if (b->d_maptab || b->d_mapbase) (void)hipDeviceSynchronize();
     if (b->d_maptab) (void)hipFree(b->d_maptab);
@@ -661,24 +706,42 @@ atg_status atg_batch_create(atg_batch** out, const int64_t* offsets, int64_t nta
         a.p_req = z.p_req;
         a.pack_cap = pack_cap_items(n, z.p_req);
         b->pack_cap_max = std::max(b->pack_cap_max, a.pack_cap);
-        // One section and its lists within what leaves a CU three workgroups.
-        const size_t lds = SmallLds(n, z.p_req).bytes();
-        if (z.G == 1 && lds <= kBatchSmallLds) {
-            int c = 0;
-            while (n > 64 * kSmallChunks[c]) ++c;
-            b->small_class[t] = (int8_t)c;
-            b->small_lds[c] = std::max(b->small_lds[c], lds);
-        }
         a.splits = b->d_splits + osp[t];
         a.learned_segments = learned_knots(o.learned_segments, z.p_req);
     }
-    // A few small tables among large ones cost a launch more than they save.
+    // Small tables: a wave per section and all of the table within a CU's LDS.
     int64_t small_items = 0;
+    auto small_key = [&](int64_t t, SmallClass& c) {
+        const BuildArgs& a = b->args[t];
+        c.xu = 0;
+        c.waves = 1;
+        c.tier = 0;
+        while (a.Ls > 64 * kSmallChunks[c.xu]) ++c.xu;
+        while (a.G > c.waves) c.waves *= 2;
+        c.lds = SmallLds(a.n, a.p_req).compact_bytes();
+        while (c.tier < 2 && c.lds > kSmallTiers[c.tier]) ++c.tier;
+        return c.waves <= (a.Ls <= kShortSectionMax ? kSmallMaxWaves : kSmallLongWaves) && c.lds <= kSmallTiers[2];
+    };
+    SmallClass key;
     for (int64_t t = 0; t < ntables; ++t)
-        if (b->small_class[t] >= 0) small_items += offsets[t + 1] - offsets[t];
-    if (kBatchSmallShare * small_items < b->total) b->small_class.assign((size_t)ntables, -1);
-    else if (hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) != hipSuccess)
-        return cleanup(fail(ATG_EDEVICE, "atg_batch_create: events"));
+        if (small_key(t, key)) small_items += offsets[t + 1] - offsets[t];
+    // A few small tables among large ones cost a launch more than they save.
+    if (small_items > 0 && kBatchSmallShare * small_items >= b->total) {
+        std::vector<SmallClass>& cs = b->small_classes;
+        for (int xu = 0; xu < 4; ++xu)
+            for (int waves = 1; waves <= kSmallMaxWaves; waves *= 2)
+                for (int tier = 0; tier < 3; ++tier) cs.push_back(SmallClass{xu, waves, tier});
+        for (int64_t t = 0; t < ntables; ++t)
+            if (small_key(t, key)) {
+                int c = 0;
+                while (cs[c].xu != key.xu || cs[c].waves != key.waves || cs[c].tier != key.tier) ++c;
+                cs[c].lds = std::max(cs[c].lds, key.lds);
+                cs[c].threads = std::max(cs[c].threads, (int)(64 * b->args[t].G));
+                b->small_class[t] = (int8_t)c;
+            }
+        if (hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) != hipSuccess)
+            return cleanup(fail(ATG_EDEVICE, "atg_batch_create: events"));
+    }
     for (int k = 0; k < 2 && b->ev_fork; ++k)
         if (hipStreamCreateWithFlags(&b->side[k], hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&b->ev_join[k], hipEventDisableTiming) != hipSuccess)

@@ -192,6 +192,7 @@ constexpr int kSmallMaxWaves = 16;  // waves of a workgroup, one per section: se
 constexpr int kSmallLongWaves = 4;  // longer ones
 constexpr int64_t kSmallMaxItems = 8192;
 constexpr size_t kSmallLdsMax = 156 * 1024;  // of 160 KB, static LDS aside
+constexpr size_t kSmallLdsDefault = 63 * 1024;  // more, the static LDS aside, a kernel has to be allowed first
 bool small_build_ok(int64_t n, int64_t G, int64_t Ls, int64_t p_req);
 hipError_t launch_small(const BuildArgs& a, bool lists, double* W_out, uint32_t* error_out, hipStream_t s);
 

@@ -17,12 +17,14 @@
 namespace atg {
 
 // LDS of a table of n items and p_req requested splits.  The section weights
-// and, later, the prefixes share one array.
+// and, later, the prefixes share one array; the list weights and items have
+// their own unless the build is compact.
 struct SmallLds {
     int64_t items;  // entries of a list array: n items and two sentinels, even
     int64_t splits;
     __host__ __device__ SmallLds(int64_t n, int64_t p_req) : items((n + 3) & ~(int64_t)1), splits(p_req + 1) {}
     __host__ __device__ size_t bytes() const { return (size_t)items * (8 + 8 + 2 + 2) + (size_t)splits * 16; }
+    __host__ __device__ size_t compact_bytes() const { return (size_t)items * (8 + 2) + (size_t)splits * 16; }
 };
 
 // The light list followed by the heavy list (from entry numL) in LDS.
@@ -36,20 +38,62 @@ struct SmallLists {
     __device__ double hw(int j) const { return w[numL + j]; }
 };
 
+// Chunks c0 .. c0 + U - 1 of a section's leftovers into registers: cL chunks of
+// 64 lights, then the heavies.  lo, off: first position and rank of each
+// chain's leftovers (chain_positions), the lights' in the low halves; the
+// chunks' searches run interleaved.
+template <int U>
+__device__ __forceinline__ void list_chunks(SecLDS& L, int c0, int cL, int mL, int mH, int lane, bool chains,
+                                            uint32_t lo, uint32_t off, int first, int64_t start, double* w,
+                                            uint16_t* item) {
+    int r[U], t[U], sh[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const bool hv = c0 + u >= cL;
+        r[u] = ((hv ? c0 + u - cL : c0 + u) << 6) + lane;
+        sh[u] = hv ? 16 : 0;
+        t[u] = 0;
+    }
+    if (chains) {
+        for (int step = first; step >= 1; step >>= 1) {
+            int o[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) o[u] = __shfl((int)off, t[u] + step, 64);
+#pragma unroll
+            for (int u = 0; u < U; ++u) t[u] += (int)((uint32_t)o[u] >> sh[u] & 0xFFFFu) <= r[u] ? step : 0;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        int pos = r[u];
+        if (chains) {
+            const uint32_t b = (uint32_t)__shfl((int)lo, t[u], 64), c = (uint32_t)__shfl((int)off, t[u], 64);
+            pos = (int)(b >> sh[u] & 0xFFFFu) + r[u] - (int)(c >> sh[u] & 0xFFFFu);
+        }
+        if (r[u] < (sh[u] ? mH : mL)) {
+            w[u] = sh[u] ? L.Hw(pos) : L.Lw(pos);
+            item[u] = (uint16_t)(start + (sh[u] ? L.Hi(pos) : L.Li(pos)));
+        }
+    }
+}
+
 // XU: weights a lane holds (sections of up to 64 XU items).  LISTS: the lists
 // and splits go to HBM as well (for the copy-out of a single table).
 // W_out, error_out: nullable copies of the state's fields.
-template <typename T, bool AOS, int XU, bool LISTS>
+// COMPACT: for many tables at once, whose number in flight the LDS bounds.
+// One array holds the section weights, then the prefixes, then the list
+// weights, which wait in registers meanwhile.
+template <typename T, bool AOS, int XU, bool LISTS, bool COMPACT>
 __device__ __forceinline__ void small_build(const BuildArgs& a, double* W_out, uint32_t* error_out, double* lds) {
     __shared__ double ssum[kSmallMaxWaves], sagg[2][kSmallMaxWaves];
     __shared__ uint32_t scnt[2][kSmallMaxWaves];
     __shared__ uint32_t sfall;
     const SmallLds lay(a.n, a.p_req);
     double* A = lds;              // section weights, then prefixes (lights, then heavies)
-    double* B = A + lay.items;    // list weights
+    double* B = COMPACT ? A : A + lay.items;  // list weights
     Split* sp = reinterpret_cast<Split*>(B + lay.items);
     uint16_t* idx = reinterpret_cast<uint16_t*>(sp + lay.splits);  // section items, local to the section
-    uint16_t* item = idx + lay.items;                              // list items
+    uint16_t* item = COMPACT ? idx : idx + lay.items;              // list items
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = wave_in_block();
     const int G = (int)a.G, s = wave;
     const bool has = s < G;
@@ -146,76 +190,143 @@ __device__ __forceinline__ void small_build(const BuildArgs& a, double* W_out, u
     const int goffH = numL + __builtin_amdgcn_readlane((int)inclH, sl) - mH;
     int first = 1;
     while (2 * first < a.chains) first *= 2;
-    if (has) {
-        constexpr int U = XU < 4 ? XU : 4;
+    double tot[2] = {0.0, 0.0};
+    // Compact builds: the section's list entries, the lights' chunks first.
+    constexpr int GS = XU < 16 ? 3 : 4;  // chunks taken together
+    constexpr int NC = COMPACT ? (XU + 1 + GS - 1) / GS * GS : 1;
+    double lw[NC] = {};
+    uint16_t it[NC] = {};
+    const int cL = (mL + 63) >> 6, cAll = cL + ((mH + 63) >> 6);
+    if constexpr (COMPACT) {
+        // 3. The section's list entries into registers, then, the section
+        //    weights all read, 4. their local prefixes and items into place
+        //    and P(s) added.
+        static_assert(!LISTS, "list weights are not kept");
+        const uint32_t lo = (uint32_t)iLo | ((uint32_t)jLo << 16), off = (uint32_t)offL | ((uint32_t)offH << 16);
+#pragma unroll
+        for (int c0 = 0; c0 < NC; c0 += GS) {
+            if (c0 < cAll) list_chunks<GS>(L, c0, cL, mL, mH, lane, a.psa_plus, lo, off, first, start, &lw[c0], &it[c0]);
+        }
+        __syncthreads();
+        double carry = 0.0, aggL = 0.0;
+#pragma unroll
+        for (int c0 = 0; c0 < NC; c0 += GS) {
+            if (c0 >= cAll) continue;
+            double inc[GS];
+#pragma unroll
+            for (int u = 0; u < GS; ++u) inc[u] = wave_scan(lw[c0 + u]);
+#pragma unroll
+            for (int u = 0; u < GS; ++u) {
+                const int c = c0 + u;
+                const bool hv = c >= cL;
+                const int r = ((hv ? c - cL : c) << 6) + lane, dst = hv ? goffH : goffL;
+                // The lights' aggregate ends where the heavies' begins; chunks
+                // past the lists add zeros.
+                if (c == cL && cL < cAll) {
+                    aggL = carry;
+                    carry = 0.0;
+                }
+                const double local = carry + wave_shr1(inc[u]);
+                if (r < (hv ? mH : mL)) {
+                    A[dst + r] = local;
+                    item[dst + r] = it[c];
+                }
+                carry = carry + readlane_d(inc[u], 63);
+            }
+        }
+        if (cL >= cAll) {  // no heavies
+            aggL = carry;
+            carry = 0.0;
+        }
+        if (has && lane == 0) {
+            sagg[0][s] = aggL;
+            sagg[1][s] = carry;
+        }
+        __syncthreads();
 #pragma unroll 1
         for (int hv = 0; hv < 2; ++hv) {
+            const double g = lane < G ? sagg[hv][lane] : 0.0;
+            const double P = fold_blocks<5>(0.0, g, s, lane), Q = fold_blocks<5>(0.0, g, G, lane);
+            if (hv) tot[1] = Q;
+            else tot[0] = Q;
             const int m = hv ? mH : mL, dst = hv ? goffH : goffL;
-#pragma unroll 1
-            for (int g0 = 0; g0 < m; g0 += 64 * U) {
-                int pos[U];
-                if (a.psa_plus) {
-                    chain_positions<U>(g0 + lane, hv ? offH : offL, hv ? jLo : iLo, pos, first);
-                } else {
-#pragma unroll
-                    for (int u = 0; u < U; ++u) pos[u] = g0 + 64 * u + lane;
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int r = g0 + 64 * u + lane;
-                    if (r < m) {
-                        B[dst + r] = hv ? L.Hw(pos[u]) : L.Lw(pos[u]);
-                        item[dst + r] = (uint16_t)(start + (hv ? L.Hi(pos[u]) : L.Li(pos[u])));
+            for (int r = lane; r < m; r += 64) A[dst + r] = P + A[dst + r];
+        }
+        if (tid == 0) {
+            item[nLr] = (uint16_t)(a.n + 1);
+            item[numL + nHr] = (uint16_t)a.n;
+        }
+    } else {
+        if (has) {
+            constexpr int U = XU < 4 ? XU : 4;
+    #pragma unroll 1
+            for (int hv = 0; hv < 2; ++hv) {
+                const int m = hv ? mH : mL, dst = hv ? goffH : goffL;
+    #pragma unroll 1
+                for (int g0 = 0; g0 < m; g0 += 64 * U) {
+                    int pos[U];
+                    if (a.psa_plus) {
+                        chain_positions<U>(g0 + lane, hv ? offH : offL, hv ? jLo : iLo, pos, first);
+                    } else {
+    #pragma unroll
+                        for (int u = 0; u < U; ++u) pos[u] = g0 + 64 * u + lane;
+                    }
+    #pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int r = g0 + 64 * u + lane;
+                        if (r < m) {
+                            B[dst + r] = hv ? L.Hw(pos[u]) : L.Lw(pos[u]);
+                            item[dst + r] = (uint16_t)(start + (hv ? L.Hi(pos[u]) : L.Li(pos[u])));
+                        }
                     }
                 }
             }
         }
-    }
-    if (tid == 0) {
-        B[nLr] = 0.0;
-        item[nLr] = (uint16_t)(a.n + 1);
-        B[numL + nHr] = __builtin_inf();
-        item[numL + nHr] = (uint16_t)a.n;
-    }
-    __syncthreads();
-
-    // 4. Local prefixes into A (the section weights are all in B by now), the
-    //    sections' aggregates, then P(s) + local.
-    if (has) {
-#pragma unroll 1
-        for (int hv = 0; hv < 2; ++hv) {
-            const int m = hv ? mH : mL, dst = hv ? goffH : goffL;
-            double carry = 0.0;
-#pragma unroll 1
-            for (int r0 = 0; r0 < m; r0 += 64) {
-                const int r = r0 + lane;
-                const double inc = wave_scan(r < m ? B[dst + r] : 0.0);
-                const double local = carry + wave_shr1(inc);
-                if (r < m) A[dst + r] = local;
-                carry = carry + readlane_d(inc, 63);
-            }
-            if (lane == 0) sagg[hv][s] = carry;
+        if (tid == 0) {
+            B[nLr] = 0.0;
+            item[nLr] = (uint16_t)(a.n + 1);
+            B[numL + nHr] = __builtin_inf();
+            item[numL + nHr] = (uint16_t)a.n;
         }
-    }
-    __syncthreads();
-    double tot[2] = {0.0, 0.0};
-#pragma unroll 1
-    for (int hv = 0; hv < 2; ++hv) {
-        const double v = lane < G ? sagg[hv][lane] : 0.0;
-        const double P = fold_blocks<5>(0.0, v, s, lane), Q = fold_blocks<5>(0.0, v, G, lane);
-        if (hv) tot[1] = Q;
-        else tot[0] = Q;
+        __syncthreads();
+
+        // 4. Local prefixes into A (the section weights are all in B by now), the
+        //    sections' aggregates, then P(s) + local.
         if (has) {
-            const int m = hv ? mH : mL, dst = hv ? goffH : goffL;
-#pragma unroll 1
-            for (int r = lane; r < m; r += 64) {
-                const double pref = P + A[dst + r];
-                A[dst + r] = pref;
-                if (LISTS) {
-                    const int g = hv ? dst + r - numL : dst + r;
-                    (hv ? a.Hi : a.Li)[g] = (int32_t)item[dst + r];
-                    (hv ? a.Hw : a.Lw)[g] = B[dst + r];
-                    (hv ? a.Hp : a.Lp)[g] = pref;
+    #pragma unroll 1
+            for (int hv = 0; hv < 2; ++hv) {
+                const int m = hv ? mH : mL, dst = hv ? goffH : goffL;
+                double carry = 0.0;
+    #pragma unroll 1
+                for (int r0 = 0; r0 < m; r0 += 64) {
+                    const int r = r0 + lane;
+                    const double inc = wave_scan(r < m ? B[dst + r] : 0.0);
+                    const double local = carry + wave_shr1(inc);
+                    if (r < m) A[dst + r] = local;
+                    carry = carry + readlane_d(inc, 63);
+                }
+                if (lane == 0) sagg[hv][s] = carry;
+            }
+        }
+        __syncthreads();
+    #pragma unroll 1
+        for (int hv = 0; hv < 2; ++hv) {
+            const double v = lane < G ? sagg[hv][lane] : 0.0;
+            const double P = fold_blocks<5>(0.0, v, s, lane), Q = fold_blocks<5>(0.0, v, G, lane);
+            if (hv) tot[1] = Q;
+            else tot[0] = Q;
+            if (has) {
+                const int m = hv ? mH : mL, dst = hv ? goffH : goffL;
+    #pragma unroll 1
+                for (int r = lane; r < m; r += 64) {
+                    const double pref = P + A[dst + r];
+                    A[dst + r] = pref;
+                    if (LISTS) {
+                        const int g = hv ? dst + r - numL : dst + r;
+                        (hv ? a.Hi : a.Li)[g] = (int32_t)item[dst + r];
+                        (hv ? a.Hw : a.Lw)[g] = B[dst + r];
+                        (hv ? a.Hp : a.Lp)[g] = pref;
+                    }
                 }
             }
         }
@@ -244,6 +355,14 @@ __device__ __forceinline__ void small_build(const BuildArgs& a, double* W_out, u
 
     if (degenerate) {  // the same in every thread
         // Every leftover row carries its own mass.
+        if constexpr (COMPACT) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int r = ((c >= cL ? c - cL : c) << 6) + lane;
+                if (r < (c >= cL ? mH : mL)) store_row<AOS>(a, it[c], lw[c], (int32_t)it[c]);
+            }
+            return;
+        }
         for (int t = tid; t < nLr + nHr; t += (int)blockDim.x) {
             const int e = t < nLr ? t : t + 1;  // past the light sentinel
             store_row<AOS>(a, item[e], B[e], (int32_t)item[e]);
@@ -258,13 +377,31 @@ __device__ __forceinline__ void small_build(const BuildArgs& a, double* W_out, u
             r = Split{0, 0, 0.0};
         } else if (k == p) {
             r = Split{numL - 1, numH - 1, 0.0};
-        } else if (!bisect_split(k, p, nToSplit, wToSplit, A, numL, A + numL, B + numL, numH, r)) {
+        } else if (COMPACT ? !bisect_split(k, p, nToSplit, wToSplit, A, numL, A + numL, SpillLater{}, numH, r)
+                           : !bisect_split(k, p, nToSplit, wToSplit, A, numL, A + numL, B + numL, numH, r)) {
             atomicAdd(&sfall, 1u);
         }
         sp[k] = r;
         if (LISTS) a.splits[k] = r;
     }
     __syncthreads();
+    if constexpr (COMPACT) {
+        // The list weights over the prefixes, then the splits' spills.
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const bool hv = c >= cL;
+            const int r = ((hv ? c - cL : c) << 6) + lane;
+            if (r < (hv ? mH : mL)) A[(hv ? goffH : goffL) + r] = lw[c];
+        }
+        if (tid == 0) {
+            A[nLr] = 0.0;
+            A[numL + nHr] = __builtin_inf();
+        }
+        __syncthreads();
+        for (int64_t k = tid; k < p; k += blockDim.x)
+            if (k > 0) sp[k].spill = sp[k].spill + A[numL + sp[k].j] - split_target(k, p, nToSplit, wToSplit);
+        __syncthreads();
+    }
 
     // 6. Pack chains, a thread each.
     const SmallLists lists{B, item, numL};

@@ -10,7 +10,7 @@ namespace atg {
 template <typename T, bool AOS, int XU, int THREADS, bool LISTS>
 __global__ __launch_bounds__(THREADS) void build_small(BuildArgs a, double* W_out, uint32_t* error_out) {
     extern __shared__ double small_lds[];
-    small_build<T, AOS, XU, LISTS>(a, W_out, error_out, small_lds);
+    small_build<T, AOS, XU, LISTS, false>(a, W_out, error_out, small_lds);
 }
 
 template <typename T, bool AOS, bool LISTS>
@@ -21,7 +21,7 @@ static hipError_t launch_small_t(const BuildArgs& a, double* W_out, uint32_t* er
         : shorts    ? build_small<T, AOS, kShortSectionMax / 64, 64 * kSmallMaxWaves, LISTS>
                     : build_small<T, AOS, PSA_MAX_LEN / 64, 64 * kSmallLongWaves, LISTS>;
     const size_t lds = SmallLds(a.n, a.p_req).bytes();
-    if (lds > 65536 - 1024) {  // beyond 64 KB, static LDS included
+    if (lds > kSmallLdsDefault) {
         const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }

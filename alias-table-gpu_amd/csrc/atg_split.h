@@ -19,12 +19,28 @@ __device__ __forceinline__ int check_split(int64_t i, int64_t j, double target, 
     return 1;
 }
 
+// The number of list items before split k, and the weight they should hold.
+__device__ __forceinline__ int64_t split_items(int64_t k, int64_t p, int64_t nToSplit) {
+    return (int64_t)ceil(((double)nToSplit * (double)k) / (double)p);
+}
+__device__ __forceinline__ double split_target(int64_t k, int64_t p, int64_t nToSplit, double wToSplit) {
+    return (wToSplit * (double)split_items(k, p, nToSplit)) / (double)nToSplit;
+}
+
+// A split's spill, or, where the heavy weights come later, its prefix sum.
+struct SpillLater {};
+__device__ __forceinline__ double split_spill(double sigma, const double* Hw, int64_t j, double target) {
+    return sigma + Hw[j] - target;
+}
+__device__ __forceinline__ double split_spill(double sigma, SpillLater, int64_t, double) { return sigma; }
+
 // Bisection; 64 probes bound the loop (the reference spins forever when
 // FOUND is unreachable), then a deterministic clamp is returned.
+template <typename HW>
 __device__ __forceinline__ bool bisect_split(int64_t k, int64_t p, int64_t nToSplit, double wToSplit,
-                                             const double* Lp, int64_t numL, const double* Hp, const double* Hw,
+                                             const double* Lp, int64_t numL, const double* Hp, HW Hw,
                                              int64_t numH, Split& out) {
-    const int64_t n_ = (int64_t)ceil(((double)nToSplit * (double)k) / (double)p);
+    const int64_t n_ = split_items(k, p, nToSplit);
     const int64_t b0 = min(n_, numH) - 1;
     const double target = (wToSplit * (double)n_) / (double)nToSplit;
     int64_t lo = 0, hi = b0;
@@ -34,7 +50,7 @@ __device__ __forceinline__ bool bisect_split(int64_t k, int64_t p, int64_t nToSp
         const int64_t i = min(n_ - j, numL - 1);
         const int stt = check_split(i, j, target, Lp, numL, Hp, numH, sigma);
         if (stt == 0) {
-            out.i = (int32_t)i; out.j = (int32_t)j; out.spill = sigma + Hw[j] - target;
+            out.i = (int32_t)i; out.j = (int32_t)j; out.spill = split_spill(sigma, Hw, j, target);
             return true;
         }
         if (stt == 2) lo = j + 1; else hi = j;
@@ -42,7 +58,7 @@ __device__ __forceinline__ bool bisect_split(int64_t k, int64_t p, int64_t nToSp
     int64_t j = min(max<int64_t>(lo, 0), max<int64_t>(b0, 0));
     int64_t i = min(n_ - j, numL - 1);
     if (i < 0) i = 0;
-    out.i = (int32_t)i; out.j = (int32_t)j; out.spill = (Lp[i] + Hp[j]) + Hw[j] - target;
+    out.i = (int32_t)i; out.j = (int32_t)j; out.spill = split_spill(Lp[i] + Hp[j], Hw, j, target);
     return false;
 }
 

@@ -20,7 +20,13 @@ EDGES = [1, 2, 63, 64, 65, 127, 128, 129, 511, 512, 513, 1023, 1024, 1025, 2047]
     (EDGES, {"psa_plus": False}, 0),
     (EDGES * 2, {"chains": 1}, 0),
     (EDGES * 2 + [3000], {"split": "learned", "chains": 64}, 0),
-    (EDGES * 2, {"section_size": 300, "num_splits": -11}, 0),            # several sections: through the phases
+    (EDGES * 2, {"section_size": 300, "num_splits": -11}, 0),            # several sections
+    ([2049, 4095, 4096, 6143, 8190, 8192, 9000], {}, 0),                 # up to four long sections, past them the phases
+    ([2500, 8000] * 3, {"psa_plus": False}, 0),                          # every item in the lists
+    ([2500, 8000] * 3, {"chains": 64, "num_splits": -10}, 0),
+    ([9, 10, 11, 99, 640, 1279, 1290, 5110, 5130, 8000, 10_230, 10_300, 14_000, 16_000],
+     {"section_size": 0, "num_splits": 81_920, "chains": 16}, 0),             # eleven to sixteen sections; past them the phases
+    ([700, 13_000, 6_500] * 5 + [40_000], {"section_size": 0, "num_splits": 81_920}, 40_000),
 ])
 def test_small_tables_match_oracle(gpu, oracle, dtype, sizes, kw, group_items):
     offsets = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
