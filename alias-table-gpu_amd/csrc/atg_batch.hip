@@ -56,12 +56,20 @@ struct BatchSampleArgs {
     int32_t* out;             // ntables * per_table
 };
 
-// Blocks of the degenerate-table fill per table: one per 65,536 items, at
-// most 8 (a grid-stride loop covers the rest).  Most tables are not
-// degenerate and leave at once, so few blocks keep the launch short.
+// Blocks per table that fill a degenerate table's rows: one per 65,536 items,
+// at most 8 (a grid-stride loop covers the rest).  They are blocks of the
+// launch that starts the splits, which such a table has none of.
 __host__ __device__ inline int64_t degenerate_blocks(int64_t n) {
     const int64_t b = (n + 2 + 65535) / 65536;
     return b < 8 ? b : 8;
+}
+// Blocks of a table in the launches that find its splits by bisection, and in
+// the one before the learned search (the certificate's, then the knots').
+inline int64_t seg_split_blocks(const BuildArgs& a) {
+    return std::max<int64_t>((a.p_req - 1 + 255) / 256, degenerate_blocks(a.n));
+}
+inline int64_t seg_prepare_blocks(const BuildArgs& a) {
+    return std::max<int64_t>(1 + (std::min<int64_t>(a.learned_segments, a.p_req) + 1 + 255) / 256, degenerate_blocks(a.n));
 }
 
 __device__ __forceinline__ void seg_locate(const SegMap& m, int64_t& t, int64_t& blk) {
@@ -154,35 +162,34 @@ __global__ __launch_bounds__(256) void seg_place(SegArgs g, SegMap m) {
     else place_section<false, false>(a, s, (int)(threadIdx.x & 63));
 }
 
-__global__ __launch_bounds__(256) void seg_degenerate(SegArgs g, SegMap m) {
-    int64_t t, blk;
-    seg_locate(m, t, blk);
-    // No latency tick here: every table has pack blocks, which run later.
-    degenerate_block<true>(table_args(g, t), blk, degenerate_blocks(table_args(g, t).n));
-}
-
 __global__ __launch_bounds__(256) void seg_split(SegArgs g, SegMap m) {
     int64_t t, blk;
     seg_locate(m, t, blk);
-    split_bisect_block(table_args(g, t), blk);
+    const BuildArgs& a = table_args(g, t);
+    if (a.st->degenerate) {
+        if (blk < degenerate_blocks(a.n)) degenerate_block<true>(a, blk, degenerate_blocks(a.n));
+        return;
+    }
+    split_bisect_block(a, blk);
 }
 
-// The split certificate of every table of the group: one block per table.
-__global__ __launch_bounds__(256) void seg_cert(SegArgs g, SegMap m) {
-    const BuildArgs& a = table_args(g, m.tab[blockIdx.x]);
-    if (a.st->error) return;
-    cert_reduce_block(a, 0, 1);
-}
-
-__global__ __launch_bounds__(256) void seg_knots(SegArgs g, SegMap m) {
+// Before the learned search: a table's split certificate (block 0) and knots,
+// or a degenerate table's rows.
+__global__ __launch_bounds__(256) void seg_prepare(SegArgs g, SegMap m) {
     int64_t t, blk;
     seg_locate(m, t, blk);
     const BuildArgs& a = table_args(g, t);
     DevState* st = a.st;
-    if (st->error || st->degenerate) return;
-    const int64_t mm = blk * blockDim.x + threadIdx.x;
-    if (mm > min<int64_t>(a.learned_segments, st->p)) return;
-    if (knot_split(a, mm)) atomicAdd((unsigned long long*)&st->split_fallbacks, 1ull);
+    if (st->error) return;
+    const bool degenerate = st->degenerate != 0;
+    if (degenerate && blk < degenerate_blocks(a.n)) degenerate_block<true>(a, blk, degenerate_blocks(a.n));
+    if (blk == 0) {
+        cert_reduce_block(a, 0, 1);
+    } else if (!degenerate) {
+        const int64_t k = (blk - 1) * blockDim.x + threadIdx.x;
+        if (k <= min<int64_t>(a.learned_segments, st->p) && knot_split(a, k))
+            atomicAdd((unsigned long long*)&st->split_fallbacks, 1ull);
+    }
 }
 
 __global__ __launch_bounds__(256) void seg_learned(SegArgs g, SegMap m) {
@@ -250,7 +257,7 @@ __global__ __launch_bounds__(256) void batch_sample(BatchSampleArgs a) {
 
 using namespace atg;
 
-enum { MAP_SUM, MAP_LOCAL, MAP_PLACE, MAP_DEG, MAP_SPLIT, MAP_KNOTS, MAP_PACK, MAP_TREE, MAP_ONE, MAP_COUNT };
+enum { MAP_SUM, MAP_LOCAL, MAP_PLACE, MAP_SPLIT, MAP_PREPARE, MAP_PACK, MAP_TREE, MAP_ONE, MAP_COUNT };
 
 // Tables built by seg_small, in classes by their sections' length (kSmallChunks
 // chunks of 64 items a lane) and number (waves, a power of two) and by how
@@ -393,8 +400,8 @@ hipError_t launch_batch(const atg_batch* b, hipStream_t s) {
     for (const BatchGroup& grp : b->groups) {
         const SegMap* M = grp.maps;
         // A group with tables that go through the phases has blocks in each
-        // map below (MAP_KNOTS and MAP_TREE are checked: a group of
-        // one-section tables has no tree blocks).
+        // map below (MAP_TREE is checked: a group of one-section tables has
+        // no tree blocks).
         // The small classes share nothing with the phases or each other, and
         // each is a few rounds of latency: they run beside the phases on two
         // streams (without phases, on the build's and one more), which join
@@ -419,11 +426,8 @@ hipError_t launch_batch(const atg_batch* b, hipStream_t s) {
                 for (int b0 = 0; (grp.G_max >> b0) > 1; b0 += 9)
                     hipLaunchKernelGGL(seg_tree, grid(M[MAP_TREE]), dim3(256), 0, s, g, M[MAP_TREE], b0);
             hipLaunchKernelGGL(seg_place, grid(M[MAP_PLACE]), dim3(256), 0, s, g, M[MAP_PLACE]);
-            if (learned) hipLaunchKernelGGL(seg_cert, grid(M[MAP_ONE]), dim3(256), 0, s, g, M[MAP_ONE]);
-            hipLaunchKernelGGL(seg_degenerate, grid(M[MAP_DEG]), dim3(256), 0, s, g, M[MAP_DEG]);
             if (learned) {
-                if (M[MAP_KNOTS].blocks > 0)
-                    hipLaunchKernelGGL(seg_knots, grid(M[MAP_KNOTS]), dim3(256), 0, s, g, M[MAP_KNOTS]);
+                hipLaunchKernelGGL(seg_prepare, grid(M[MAP_PREPARE]), dim3(256), 0, s, g, M[MAP_PREPARE]);
                 hipLaunchKernelGGL(seg_learned, grid(M[MAP_SPLIT]), dim3(256), 0, s, g, M[MAP_SPLIT]);
             } else {
                 hipLaunchKernelGGL(seg_split, grid(M[MAP_SPLIT]), dim3(256), 0, s, g, M[MAP_SPLIT]);
@@ -474,16 +478,14 @@ atg_status make_groups(atg_batch* b, int64_t group_items) {
     }
     auto blocks_of = [&](int ph, int64_t t) -> int64_t {
         const BuildArgs& a = b->args[t];
-        const int64_t K = std::min<int64_t>(a.learned_segments, a.p_req);
         if (b->small_class[t] >= 0) return 0;
         switch (ph) {
             case MAP_SUM: return (a.G + 3) / 4;
             case MAP_LOCAL: return a.G;
             case MAP_PLACE: return (a.G + 3) / 4;
             case MAP_TREE: return a.G > 1 ? (a.G + 511) / 512 : 0;  // one section: no tree
-            case MAP_DEG: return degenerate_blocks(a.n);
-            case MAP_SPLIT: return std::max<int64_t>(1, (a.p_req - 1 + 255) / 256);
-            case MAP_KNOTS: return (K + 1 + 255) / 256;
+            case MAP_SPLIT: return seg_split_blocks(a);
+            case MAP_PREPARE: return seg_prepare_blocks(a);
             case MAP_ONE: return 1;
             default: return (a.p_req + 63) / 64;  // MAP_PACK
         }

@@ -42,6 +42,7 @@ struct BuildArgs {
     // learned split index
     int32_t learned_segments;
     int32_t* knot_j;          // learned_segments + 1 exact split j at the knots
+    int64_t direct_splits;    // the learned split leaves up to this many to bisection
     int32_t pack_method;      // atg_pack_method
     // Lean light lists: the placement writes only the light prefixes; the
     // light items and weights stay in the staging, found through sec_loff
@@ -164,7 +165,11 @@ constexpr int64_t kOwnSumMax = 2048;
 hipError_t launch_front(const BuildArgs& a, hipStream_t s);
 hipError_t launch_partition_local(const BuildArgs& a, hipStream_t s);
 hipError_t launch_partition_place(const BuildArgs& a, hipStream_t s);
-hipError_t launch_degenerate(const BuildArgs& a, hipStream_t s);
+// What the learned and P-ary splits and chunked splits start from: the
+// certificate (with want_cert), the knots on request, and a degenerate table's
+// rows.  launch_front leaves the certificate to it; launch_partition and
+// launch_partition_place, the phases by themselves, compute it too.
+hipError_t launch_split_prepare(const BuildArgs& a, bool knots, hipStream_t s);
 hipError_t launch_split(const BuildArgs& a, hipStream_t s);
 hipError_t launch_split_learned(const BuildArgs& a, hipStream_t s);
 hipError_t launch_split_pary(const BuildArgs& a, hipStream_t s);
@@ -177,7 +182,6 @@ int64_t split_blocks(const BuildArgs& a);
 int64_t pack_blocks(const BuildArgs& a);
 int64_t fill_blocks(int64_t n);
 hipError_t launch_split_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1);
-hipError_t launch_split_knots(const BuildArgs& a, hipStream_t s);
 hipError_t launch_split_learned_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1);
 hipError_t launch_split_pary_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1);
 hipError_t launch_pack_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1);

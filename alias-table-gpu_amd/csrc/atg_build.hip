@@ -90,10 +90,26 @@ __global__ __launch_bounds__(256) void partition_place(BuildArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// 3a. Degenerate tables: every leftover row carries its own mass.
+// 3a. What a searched split needs first, in one launch: the split certificate
+//     (blocks [0, cert)), the knots (blocks [cert, cert + knots)), and, in a
+//     degenerate table, which has no splits, its rows, by all blocks.  A table
+//     left with few splits has them all found here instead.
 template <bool AOS>
-__global__ void degenerate_fill(BuildArgs a) {
-    degenerate_block<AOS>(a, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(256) void split_prepare(BuildArgs a, int cert, int knots) {
+    DevState* st = a.st;
+    if (st->error) return;
+    const bool degenerate = st->degenerate != 0;
+    if (degenerate) degenerate_block<AOS>(a, blockIdx.x, gridDim.x);
+    const int b = (int)blockIdx.x;
+    if (!degenerate && st->p <= a.direct_splits) {
+        for (int64_t blk = b; blk * blockDim.x < st->p; blk += gridDim.x) split_bisect_block(a, blk);
+    } else if (b < cert) {
+        cert_reduce_block(a, b, cert);
+    } else if (b < cert + knots && !degenerate) {
+        const int64_t m = (int64_t)(b - cert) * blockDim.x + threadIdx.x;
+        if (m <= min<int64_t>(a.learned_segments, st->p) && knot_split(a, m))
+            atomicAdd((unsigned long long*)&st->split_fallbacks, 1ull);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -357,23 +373,7 @@ static hipError_t launch_partition_kernel(const BuildArgs& a, bool own_w, hipStr
 
 hipError_t launch_partition_local(const BuildArgs& a, hipStream_t s) { return launch_partition_kernel(a, false, s); }
 
-hipError_t launch_front(const BuildArgs& a, hipStream_t s) {
-    if (a.G > kOwnSumMax) {
-        const hipError_t e = launch_sum(a, s);
-        return e != hipSuccess ? e : launch_partition(a, s);
-    }
-    launch_sum_sections(a, s);
-    const hipError_t e = launch_partition_kernel(a, true, s);
-    return e != hipSuccess ? e : launch_partition_place(a, s);
-}
-
-hipError_t launch_partition(const BuildArgs& a, hipStream_t s) {
-    const hipError_t e = launch_partition_local(a, s);
-    if (e != hipSuccess) return e;
-    return launch_partition_place(a, s);
-}
-
-hipError_t launch_partition_place(const BuildArgs& a, hipStream_t s) {
+static hipError_t launch_place(const BuildArgs& a, hipStream_t s) {
     const dim3 g(blocks_for(a.G, 4)), b(256);
     if (a.G <= kDirectPrefixMax) {
         if (a.lean_lights) hipLaunchKernelGGL((partition_place<true, true>), g, b, 0, s, a);
@@ -384,8 +384,33 @@ hipError_t launch_partition_place(const BuildArgs& a, hipStream_t s) {
         if (a.lean_lights) hipLaunchKernelGGL((partition_place<true, false>), g, b, 0, s, a);
         else hipLaunchKernelGGL((partition_place<false, false>), g, b, 0, s, a);
     }
-    if (a.want_cert)
-        hipLaunchKernelGGL(cert_reduce, dim3(blocks_for(a.G, 256)), dim3(256), 0, s, a);  // a section per thread
+    return hipGetLastError();
+}
+
+hipError_t launch_front(const BuildArgs& a, hipStream_t s) {
+    hipError_t e;
+    if (a.G > kOwnSumMax) {
+        e = launch_sum(a, s);
+        if (e == hipSuccess) e = launch_partition_local(a, s);
+    } else {
+        launch_sum_sections(a, s);
+        e = launch_partition_kernel(a, true, s);
+    }
+    return e != hipSuccess ? e : launch_place(a, s);
+}
+
+hipError_t launch_partition(const BuildArgs& a, hipStream_t s) {
+    const hipError_t e = launch_partition_local(a, s);
+    if (e != hipSuccess) return e;
+    return launch_partition_place(a, s);
+}
+
+static int cert_blocks(const BuildArgs& a) { return a.want_cert ? (int)blocks_for(a.G, 256) : 0; }  // a section per thread
+
+hipError_t launch_partition_place(const BuildArgs& a, hipStream_t s) {
+    const hipError_t e = launch_place(a, s);
+    if (e != hipSuccess || !a.want_cert) return e;
+    hipLaunchKernelGGL(cert_reduce, dim3((unsigned)cert_blocks(a)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -398,12 +423,6 @@ hipError_t launch_lean_lights_fill(const BuildArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_degenerate(const BuildArgs& a, hipStream_t s) {
-    if (a.rows) hipLaunchKernelGGL(degenerate_fill<true>, dim3(1024), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(degenerate_fill<false>, dim3(1024), dim3(256), 0, s, a);
-    return hipGetLastError();
-}
-
 // Blocks of 256 splits (k = 1 .. p_req - 1) and of 64 pack chains (k = 1 .. p_req).
 int64_t split_blocks(const BuildArgs& a) { return a.p_req >= 2 ? blocks_for(a.p_req - 1, 256) : 0; }
 int64_t pack_blocks(const BuildArgs& a) { return blocks_for(a.p_req, 64); }
@@ -411,6 +430,16 @@ int64_t pack_blocks(const BuildArgs& a) { return blocks_for(a.p_req, 64); }
 // Blocks of a launch that also fills a degenerate table's rows: 4096 items a
 // block, at most 1024 blocks (each walks on from there).
 int64_t fill_blocks(int64_t n) { return std::min<int64_t>(1024, blocks_for(n, 4096)); }
+
+hipError_t launch_split_prepare(const BuildArgs& a, bool knots, hipStream_t s) {
+    const int cert = cert_blocks(a);
+    const int kb = knots ? (int)blocks_for(std::min<int64_t>(a.learned_segments, a.p_req) + 1, 256) : 0;
+    const int64_t direct = blocks_for(std::min(a.direct_splits, a.p_req), 256);
+    const dim3 g((unsigned)std::max(std::max<int64_t>(cert + kb, direct), fill_blocks(a.n)));
+    if (a.rows) hipLaunchKernelGGL(split_prepare<true>, g, dim3(256), 0, s, a, cert, kb);
+    else hipLaunchKernelGGL(split_prepare<false>, g, dim3(256), 0, s, a, cert, kb);
+    return hipGetLastError();
+}
 
 hipError_t launch_split_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1) {
     if (b1 > b0) hipLaunchKernelGGL(split_bisect<true>, dim3((unsigned)(b1 - b0)), dim3(256), 0, s, a, b0, 0);
