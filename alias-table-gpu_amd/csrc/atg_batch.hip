@@ -155,11 +155,16 @@ __global__ __launch_bounds__(256) void seg_place(SegArgs g, SegMap m) {
     const BuildArgs& a = table_args(g, t);
     if (a.st->error) return;
     const int64_t s = blk * 4 + wave_in_block();
-    if (s >= a.G) return;
+    const int lane = (int)(threadIdx.x & 63);
     // Lean lists as in a single table (1.3e8 leftovers of a 1,024-table FP32
     // batch: 0.88 -> 0.46 ms, its pack 1.19 -> 1.08).
-    if (a.lean_lights) place_section<true, false>(a, s, (int)(threadIdx.x & 63));
-    else place_section<false, false>(a, s, (int)(threadIdx.x & 63));
+    if (s == a.G) {
+        if (a.lean_lights) place_totals<true, false>(a, lane);
+        else place_totals<false, false>(a, lane);
+    } else if (s < a.G) {
+        if (a.lean_lights) place_section<true, false>(a, s, lane);
+        else place_section<false, false>(a, s, lane);
+    }
 }
 
 __global__ __launch_bounds__(256) void seg_split(SegArgs g, SegMap m) {
@@ -482,7 +487,7 @@ atg_status make_groups(atg_batch* b, int64_t group_items) {
         switch (ph) {
             case MAP_SUM: return (a.G + 3) / 4;
             case MAP_LOCAL: return a.G;
-            case MAP_PLACE: return (a.G + 3) / 4;
+            case MAP_PLACE: return a.G / 4 + 1;  // the sections and the totals
             case MAP_TREE: return a.G > 1 ? (a.G + 511) / 512 : 0;  // one section: no tree
             case MAP_SPLIT: return seg_split_blocks(a);
             case MAP_PREPARE: return seg_prepare_blocks(a);

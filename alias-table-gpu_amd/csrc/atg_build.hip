@@ -80,13 +80,13 @@ __global__ __launch_bounds__(256) void cert_reduce(BuildArgs a) {
     cert_reduce_block(a, blockIdx.x, gridDim.x);
 }
 
-// Four sections per block, one per wave.
+// Four sections per block, one per wave, and a wave for the totals.
 template <bool LEAN, bool DIRECT>
 __global__ __launch_bounds__(256) void partition_place(BuildArgs a) {
     if (a.st->error) return;
     const int64_t s = (int64_t)blockIdx.x * 4 + wave_in_block();
-    if (s >= a.G) return;
-    place_section<LEAN, DIRECT>(a, s, (int)(threadIdx.x & 63));
+    if (s < a.G) place_section<LEAN, DIRECT>(a, s, (int)(threadIdx.x & 63));
+    else if (s == a.G) place_totals<LEAN, DIRECT>(a, (int)(threadIdx.x & 63));
 }
 
 // ---------------------------------------------------------------------------
@@ -374,7 +374,7 @@ static hipError_t launch_partition_kernel(const BuildArgs& a, bool own_w, hipStr
 hipError_t launch_partition_local(const BuildArgs& a, hipStream_t s) { return launch_partition_kernel(a, false, s); }
 
 static hipError_t launch_place(const BuildArgs& a, hipStream_t s) {
-    const dim3 g(blocks_for(a.G, 4)), b(256);
+    const dim3 g(blocks_for(a.G + 1, 4)), b(256);
     if (a.G <= kDirectPrefixMax) {
         if (a.lean_lights) hipLaunchKernelGGL((partition_place<true, true>), g, b, 0, s, a);
         else hipLaunchKernelGGL((partition_place<false, true>), g, b, 0, s, a);

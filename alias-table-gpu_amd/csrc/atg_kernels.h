@@ -675,18 +675,58 @@ __device__ __forceinline__ void psa_section(const BuildArgs& a, double W_N, int6
 
 // Partition pass 2, section s by one wave: the section prefix P(s) from the
 // completed dyadic blocks, then the staged leftovers with prefixes
-// P(s) + local (the canonical chunked scan recomputed in the same order),
-// and for the last section the totals, sentinels and split inputs.
+// P(s) + local (the canonical chunked scan recomputed in the same order).
 // LEAN: the lean light lists (a.lean_lights), fixed at compile time so that
 // each kernel carries one path.
 // DIRECT: P(s) from the sections' own sums (no tree was built).
 template <bool LEAN, bool DIRECT>
 __device__ __forceinline__ void place_section(const BuildArgs& a, int64_t s, int lane) {
-    DevState* st = a.st;
     const int64_t start = min(a.n, s * a.Ls);
     // The block sums were completed by the previous launch.
     const uint64_t c0 = a.slots[s];  // this section's own counts
     const int mL = (int)(uint32_t)c0, mH = (int)(c0 >> 32);
+    // Groups of PC chunks of 64 leftovers: all loads of a group in flight
+    // together, the chunk scans independent, then the carries chained left to
+    // right (the same operations in the same order as one chunk at a time).
+    constexpr int PC = place_chunks<LEAN>();
+    double v[PC];
+    int32_t item[PC];
+    // Lean lists: the lights keep their items and weights in the staging.
+    auto load_group = [&](bool heavy, int g0) {
+        const int m = heavy ? mH : mL;
+        const bool full = heavy || !LEAN;
+        const int64_t src = start + (heavy ? mL : 0);
+        // Chunks past the list are skipped; in the last one, ranks past
+        // the list read its last entry (no exec masks around the loads)
+        // and count as 0.
+        if (g0 + 64 * PC <= m) {
+#pragma unroll
+            for (int u = 0; u < PC; ++u) {
+                v[u] = __builtin_nontemporal_load(&a.stage_w[src + g0 + 64 * u + lane]);
+                item[u] = full ? __builtin_nontemporal_load(&a.stage_i[src + g0 + 64 * u + lane]) : 0;
+            }
+        } else {
+            // The list's last group: a scalar base and 32-bit lane offsets.
+            const char* bw = reinterpret_cast<const char*>(a.stage_w + src + g0);
+            const char* bi = reinterpret_cast<const char*>(a.stage_i + src + g0);
+            const int lim = m - 1 - g0;
+#pragma unroll
+            for (int u = 0; u < PC; ++u) {
+                const uint32_t rc = (uint32_t)min(64 * u + lane, lim);
+                v[u] = 0.0;
+                item[u] = 0;
+                if (64 * u <= lim) {
+                    v[u] = __builtin_nontemporal_load(reinterpret_cast<const double*>(bw + rc * 8u));
+                    if (full) item[u] = __builtin_nontemporal_load(reinterpret_cast<const int32_t*>(bi + rc * 4u));
+                }
+            }
+        }
+    };
+    // AHEAD (few sections, bound by latency): each group's loads are issued
+    // before the group before it is scanned and stored, the first one's before
+    // the prefix is found.
+    constexpr bool AHEAD = DIRECT;
+    if (AHEAD && mL + mH > 0) load_group(mL == 0, 0);
     const Prefix P = DIRECT ? block_prefix_direct(a, (int)s, lane) : block_prefix_done(a, s, lane);
     const int64_t goffL = (int64_t)(uint32_t)P.c, goffH = (int64_t)(P.c >> 32);
     // Split certificate (learned split only): the extreme increments between
@@ -699,54 +739,29 @@ __device__ __forceinline__ void place_section(const BuildArgs& a, int64_t s, int
         const bool heavy = hv == 1;
         const int m = heavy ? mH : mL;
         if (m == 0) continue;
-        const int64_t src = start + (heavy ? mL : 0);
         const double Pv = heavy ? P.h : P.l;
         int32_t* oi = heavy ? a.Hi : a.Li;
         double* ow = heavy ? a.Hw : a.Lw;
         double* op = heavy ? a.Hp : a.Lp;
         const int64_t goff = heavy ? goffH : goffL;
-        // Lean lists: the lights keep their items and weights in the staging.
         const bool full = heavy || !LEAN;
         double ext = heavy ? __builtin_inf() : 0.0;
-        constexpr int PC = place_chunks<LEAN>();
-        // Groups of PC chunks of 64: all loads of a group in flight
-        // together, the chunk scans independent, then the carries chained left
-        // to right (the same operations in the same order as one chunk at a
-        // time).
         double carry = 0.0;
         for (int g0 = 0; g0 < m; g0 += 64 * PC) {
-            double v[PC], inc[PC];
-            int32_t item[PC];
-            // Chunks past the list are skipped; in the last one, ranks past
-            // the list read its last entry (no exec masks around the loads)
-            // and count as 0.
-            if (g0 + 64 * PC <= m) {
+            double w[PC], inc[PC];
+            int32_t it[PC];
+            if (!AHEAD) load_group(heavy, g0);
 #pragma unroll
-                for (int u = 0; u < PC; ++u) {
-                    v[u] = __builtin_nontemporal_load(&a.stage_w[src + g0 + 64 * u + lane]);
-                    item[u] = full ? __builtin_nontemporal_load(&a.stage_i[src + g0 + 64 * u + lane]) : 0;
-                }
-            } else {
-                // The list's last group: a scalar base and 32-bit lane offsets.
-                const char* bw = reinterpret_cast<const char*>(a.stage_w + src + g0);
-                const char* bi = reinterpret_cast<const char*>(a.stage_i + src + g0);
-                const int lim = m - 1 - g0;
-#pragma unroll
-                for (int u = 0; u < PC; ++u) {
-                    const uint32_t rc = (uint32_t)min(64 * u + lane, lim);
-                    v[u] = 0.0;
-                    item[u] = 0;
-                    if (64 * u <= lim) {
-                        v[u] = __builtin_nontemporal_load(reinterpret_cast<const double*>(bw + rc * 8u));
-                        if (full) item[u] = __builtin_nontemporal_load(reinterpret_cast<const int32_t*>(bi + rc * 4u));
-                    }
-                }
+            for (int u = 0; u < PC; ++u) {
+                w[u] = g0 + 64 * u + lane < m ? v[u] : 0.0;
+                it[u] = item[u];
+            }
+            if (AHEAD) {
+                const bool more = g0 + 64 * PC < m;
+                if (more || (!heavy && mH > 0)) load_group(heavy || !more, more ? g0 + 64 * PC : 0);
             }
 #pragma unroll
-            for (int u = 0; u < PC; ++u)
-                if (g0 + 64 * u + lane >= m) v[u] = 0.0;
-#pragma unroll
-            for (int u = 0; u < PC; ++u) inc[u] = wave_scan(v[u]);
+            for (int u = 0; u < PC; ++u) inc[u] = wave_scan(w[u]);
 #pragma unroll
             for (int u = 0; u < PC; ++u) {
                 const int r0 = g0 + 64 * u;
@@ -757,8 +772,8 @@ __device__ __forceinline__ void place_section(const BuildArgs& a, int64_t s, int
                     const double carry_next = carry + readlane_d(inc[u], 63);
                     if (r < m) {
                         if (full) {
-                            oi[goff + r] = item[u];
-                            ow[goff + r] = v[u];
+                            oi[goff + r] = it[u];
+                            ow[goff + r] = w[u];
                         }
                         op[goff + r] = pref;
                     }
@@ -799,27 +814,31 @@ __device__ __forceinline__ void place_section(const BuildArgs& a, int64_t s, int
         const int64_t q1 = mL > 0 ? (goffL + mL - 1) >> kLightDirShift : q0 - 1;
         for (int64_t q = q0 + lane; q <= q1; q += 64) a.sec_ldir[q] = (uint32_t)s;
     }
-    if (s == a.G - 1) {
-        // Totals P(G), sentinels (AliasTableSplitGpu.cu:366-385) and the split inputs.
-        const Prefix Tot = DIRECT ? block_prefix_direct(a, (int)a.G, lane) : block_prefix_done(a, a.G, lane);
-        if (lane == 0) {
-            const int64_t nLr = (int64_t)(uint32_t)Tot.c, nHr = (int64_t)(Tot.c >> 32);
-            if (LEAN) a.sec_loff[a.G] = (uint32_t)nLr;
-            a.Li[nLr] = (int32_t)(a.n + 1); a.Lw[nLr] = 0.0; a.Lp[nLr] = Tot.l;
-            a.Hi[nHr] = (int32_t)a.n; a.Hw[nHr] = __builtin_inf(); a.Hp[nHr] = Tot.h;
-            const int64_t numL = nLr + 1, numH = nHr + 1;
-            st->numL = numL;
-            st->numH = numH;
-            st->degenerate = (nLr == 0 || nHr == 0) ? 1u : 0u;
-            int64_t p = a.p_req;
-            if (a.psa_plus) { p = min(p, (numL + numH) / 10); if (p < 2) p = 2; }
-            st->p = st->degenerate ? 0 : p;
-            st->nToSplit = numL + numH - 2;
-            st->wToSplit = Tot.l + Tot.h;
-        }
-    }
 }
 
+// After the sections, by a wave of its own (of the last section's it would be
+// the launch's tail): the totals P(G), sentinels (AliasTableSplitGpu.cu:366-385)
+// and the split inputs.
+template <bool LEAN, bool DIRECT>
+__device__ __forceinline__ void place_totals(const BuildArgs& a, int lane) {
+    DevState* st = a.st;
+    const Prefix Tot = DIRECT ? block_prefix_direct(a, (int)a.G, lane) : block_prefix_done(a, a.G, lane);
+    if (lane == 0) {
+        const int64_t nLr = (int64_t)(uint32_t)Tot.c, nHr = (int64_t)(Tot.c >> 32);
+        if (LEAN) a.sec_loff[a.G] = (uint32_t)nLr;
+        a.Li[nLr] = (int32_t)(a.n + 1); a.Lw[nLr] = 0.0; a.Lp[nLr] = Tot.l;
+        a.Hi[nHr] = (int32_t)a.n; a.Hw[nHr] = __builtin_inf(); a.Hp[nHr] = Tot.h;
+        const int64_t numL = nLr + 1, numH = nHr + 1;
+        st->numL = numL;
+        st->numH = numH;
+        st->degenerate = (nLr == 0 || nHr == 0) ? 1u : 0u;
+        int64_t p = a.p_req;
+        if (a.psa_plus) { p = min(p, (numL + numH) / 10); if (p < 2) p = 2; }
+        st->p = st->degenerate ? 0 : p;
+        st->nToSplit = numL + numH - 2;
+        st->wToSplit = Tot.l + Tot.h;
+    }
+}
 
 // ---------------------------------------------------------------------------
 // W, pass 1: section sums, one wave per section (block blk of nblk holds
