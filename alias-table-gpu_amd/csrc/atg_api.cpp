@@ -138,8 +138,8 @@ struct atg_table_s {
         a.tree_scratch_half = tree_half;
         a.slots = d_slots;
         a.sec_cert = d_sec_cert;
-        // The learned and P-ary searches need it.
-        a.want_cert = opts.split_method != ATG_SPLIT_BISECT || split_by_index(opts.split_method, p_req);
+        // The learned, P-ary and grouped searches need it.
+        a.want_cert = opts.split_method != ATG_SPLIT_BISECT || split_by_group(opts.split_method, p_req);
         a.stage_w = d_stage_w;
         a.stage_i = d_stage_i;
         a.Li = d_Li; a.Lw = d_Lw; a.Lp = d_Lp;
@@ -154,7 +154,7 @@ struct atg_table_s {
         a.splits = d_splits;
         a.pack_cap = pack_cap_items(n, p_req);
         a.learned_segments = learned_knots(opts.learned_segments, p_req);
-        a.direct_splits = opts.split_method == ATG_SPLIT_BISECT ? kIndexedSplits / 2 : 0;
+        a.direct_splits = split_by_group(opts.split_method, p_req) ? kGroupedSplits / 2 : 0;
         a.knot_j = d_knots;
         a.pack_method = opts.pack_method;
         a.sec_loff = d_sec_loff;
@@ -362,8 +362,9 @@ atg_status atg_build_phase(atg_table* t, int32_t phase, void* stream) {
             t->placed = true;
             break;
         case ATG_PHASE_SPLIT:
-            if (split_by_index(t->opts.split_method, t->p_req)) HIPCHK(launch_split_learned(a, s));
+            if (t->opts.split_method == ATG_SPLIT_LEARNED) HIPCHK(launch_split_learned(a, s));
             else if (t->opts.split_method == ATG_SPLIT_PARY) HIPCHK(launch_split_pary(a, s));
+            else if (split_by_group(t->opts.split_method, t->p_req)) HIPCHK(launch_split_grouped(a, s));
             else HIPCHK(launch_split(a, s));
             break;
         case ATG_PHASE_PACK:
@@ -384,16 +385,18 @@ static bool build_split_pack_interleaved(atg_table* t, const BuildArgs& a, hipSt
     const int64_t SB = split_blocks(a), PB = pack_blocks(a);
     const int C = (int)std::min<int64_t>(kInterleaveChunks, SB);
     if (C < 2) return false;
-    const bool learned = split_by_index(t->opts.split_method, t->p_req), pary = t->opts.split_method == ATG_SPLIT_PARY;
+    const bool learned = t->opts.split_method == ATG_SPLIT_LEARNED, pary = t->opts.split_method == ATG_SPLIT_PARY;
+    const bool grouped = split_by_group(t->opts.split_method, t->p_req);
     hipStream_t sp = t->sp_stream;
     err = hipEventRecord(t->ev_fork, s);
     if (err == hipSuccess) err = hipStreamWaitEvent(sp, t->ev_fork, 0);
     if (err == hipSuccess) err = launch_split_prepare(a, learned, sp);
     for (int c = 0; c < C && err == hipSuccess; ++c) {
         const int64_t b0 = SB * c / C, b1 = SB * (c + 1) / C;
-        err = learned ? launch_split_learned_blocks(a, sp, b0, b1)
-              : pary  ? launch_split_pary_blocks(a, sp, b0, b1)
-                      : launch_split_blocks(a, sp, b0, b1);
+        err = learned   ? launch_split_learned_blocks(a, sp, b0, b1)
+              : pary    ? launch_split_pary_blocks(a, sp, b0, b1)
+              : grouped ? launch_split_grouped_blocks(a, sp, b0, b1)
+                        : launch_split_blocks(a, sp, b0, b1);
         if (err == hipSuccess) err = hipEventRecord(t->ev_chunk[c], sp);
     }
     for (int c = 0; c < C && err == hipSuccess; ++c) {
@@ -479,14 +482,13 @@ atg_status atg_get_stats(atg_table* t, atg_stats* out) {
     out->num_sections = t->G;
     out->section_len = t->Ls;
     out->split_fallbacks = (int64_t)st.split_fallbacks;
-    // Of the search that was asked for, not of the index a bisection may use.
-    const bool bisect = t->opts.split_method == ATG_SPLIT_BISECT;
-    out->learned_fallbacks = bisect ? 0 : (int64_t)st.learned_fallbacks;
+    out->learned_fallbacks = (int64_t)st.learned_fallbacks;
     out->degenerate = (int32_t)st.degenerate;
     double mdl, mdh;
     std::memcpy(&mdl, &st.cert_max_dL, 8);
     std::memcpy(&mdh, &st.cert_min_dH, 8);
-    out->monotone = st.cert_done && !bisect ? (mdl < mdh ? 1 : 0) : -1;
+    // Of the searches that report it; a bisection may compute it for itself.
+    out->monotone = st.cert_done && t->opts.split_method != ATG_SPLIT_BISECT ? (mdl < mdh ? 1 : 0) : -1;
     if (t->events && t->built) {
         float ms;
         const int map[5][2] = {{0, 1}, {1, 2}, {2, 3}, {3, 4}, {4, 5}};

@@ -42,7 +42,7 @@ struct BuildArgs {
     // learned split index
     int32_t learned_segments;
     int32_t* knot_j;          // learned_segments + 1 exact split j at the knots
-    int64_t direct_splits;    // the learned split leaves up to this many to bisection
+    int64_t direct_splits;    // up to this many splits launch_split_prepare finds by bisection
     int32_t pack_method;      // atg_pack_method
     // Lean light lists: the placement writes only the light prefixes; the
     // light items and weights stay in the staging, found through sec_loff
@@ -173,6 +173,7 @@ hipError_t launch_split_prepare(const BuildArgs& a, bool knots, hipStream_t s);
 hipError_t launch_split(const BuildArgs& a, hipStream_t s);
 hipError_t launch_split_learned(const BuildArgs& a, hipStream_t s);
 hipError_t launch_split_pary(const BuildArgs& a, hipStream_t s);
+hipError_t launch_split_grouped(const BuildArgs& a, hipStream_t s);
 hipError_t launch_pack(const BuildArgs& a, hipStream_t s);
 // Lean light lists written out as lists (Li, Lw) from the staging.
 hipError_t launch_lean_lights_fill(const BuildArgs& a, hipStream_t s);
@@ -183,6 +184,7 @@ int64_t pack_blocks(const BuildArgs& a);
 int64_t fill_blocks(int64_t n);
 hipError_t launch_split_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1);
 hipError_t launch_split_learned_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1);
+hipError_t launch_split_grouped_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1);
 hipError_t launch_split_pary_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1);
 hipError_t launch_pack_blocks(const BuildArgs& a, hipStream_t s, int64_t b0, int64_t b1);
 hipError_t launch_split_rows(const Row* rows, double* w, int32_t* al, int64_t n, hipStream_t s);

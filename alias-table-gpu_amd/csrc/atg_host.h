@@ -19,18 +19,18 @@ int device_cus();
 atg_status state_status(const DevState& st);
 // Sets the chain count and requested splits of a created table in place.
 atg_status table_set_shape(atg_table* t, int32_t chains, int64_t num_splits);
-// Whether the splits are found through the learned index: on request, and, as
-// it returns the bisection's splits, where so many are to be found that its
-// narrow searches pay for the knots (builds, us, bisection and index: 1e7
-// items, 417,000 splits 257 and 239, 156,000 256 and 266; 3e7 items, 469,000
-// 653 and 605, 150,000 624 and 628; 1e8, 500,000 1,853 and 1,823, 1.6e6 2,001
-// and 1,756, 4.2e6 2,098 and 1,772).  A table that turns out to have fewer than
-// half of that (many items finished by the partition) takes the bisection.
-constexpr int64_t kIndexedSplits = (int64_t)1 << 18;
-inline bool split_by_index(int32_t split_method, int64_t p_req) {
-    return split_method == ATG_SPLIT_LEARNED || (split_method == ATG_SPLIT_BISECT && p_req >= kIndexedSplits);
+// Whether a bisection is done wave by wave inside brackets (split_grouped),
+// which needs the split certificate.  Builds, us, over the whole lists and so:
+// 1e7 items, 417,000 splits 257 and 232, 156,000 257 and 256, 82,000 244 and
+// 252; 3e7 items, 469,000 653 and 593; 1e8, 500,000 1,853 and 1,790, 1.6e6 2,001
+// and 1,748, 4.2e6 2,098 and 1,804; where the certificate fails, 3e7 and 1.2e6
+// 723 and 748, 1e8 and 2.6e6 2,209 and 2,234.  A table that turns out to have
+// fewer than half of the line (many items finished by the partition) is
+// bisected in the certificate's launch.
+constexpr int64_t kGroupedSplits = (int64_t)1 << 18;
+inline bool split_by_group(int32_t split_method, int64_t p_req) {
+    return split_method == ATG_SPLIT_BISECT && p_req >= kGroupedSplits;
 }
-
 // Sets the split method, knot count and split/pack interleave of a created
 // table (knobs that leave the table's rows unchanged).
 atg_status table_set_method(atg_table* t, int32_t split_method, int32_t learned_segments, int32_t interleave);

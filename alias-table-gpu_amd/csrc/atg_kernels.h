@@ -1237,6 +1237,65 @@ __device__ __forceinline__ uint32_t knot_split(const BuildArgs& a, int64_t m) {
     return fb;
 }
 
+// Split k between the splits km < k < km1 whose heavies are lo and hi: gallop
+// from their linear interpolation until the answer is bracketed, then bisect.
+// Under the certificate what it finds is the bisection's split.
+__device__ __forceinline__ bool bracket_split(const BuildArgs& a, int64_t k, int64_t km, int64_t km1, int64_t lo, int64_t hi, Split& out) {
+    const DevState* st = a.st;
+    const int64_t numL = st->numL, numH = st->numH;
+    const int64_t n_ = split_items(k, st->p, st->nToSplit);
+    const int64_t b0 = min(n_, numH) - 1;
+    const double target = split_target(k, st->p, st->nToSplit, st->wToSplit);
+    if (hi > b0) hi = b0;
+    if (lo < 0) lo = 0;
+    if (lo <= hi) {
+        // Model prediction: linear interpolation inside the segment.
+        int64_t j = lo + ((hi - lo) * (k - km)) / (km1 - km);
+        double sigma = 0.0;
+        int stt = check_split(min(n_ - j, numL - 1), j, target, a.Lp, numL, a.Hp, numH, sigma);
+        // Gallop from the prediction until the answer is bracketed, then bisect.
+        int64_t a0 = lo, b1 = hi;
+        if (stt == 2) {  // RIGHT: answer above j
+            a0 = j + 1;
+            int64_t step = 1;
+            while (true) {
+                const int64_t t = j + step;
+                if (t >= hi) { b1 = hi; break; }
+                const int s2 = check_split(min(n_ - t, numL - 1), t, target, a.Lp, numL, a.Hp, numH, sigma);
+                if (s2 == 0) { j = t; stt = 0; break; }
+                if (s2 == 1) { b1 = t; break; }
+                a0 = t + 1;
+                step <<= 1;
+            }
+        } else if (stt == 1) {  // LEFT: answer below j
+            b1 = j;
+            int64_t step = 1;
+            while (true) {
+                const int64_t t = j - step;
+                if (t <= lo) { a0 = lo; break; }
+                const int s2 = check_split(min(n_ - t, numL - 1), t, target, a.Lp, numL, a.Hp, numH, sigma);
+                if (s2 == 0) { j = t; stt = 0; break; }
+                if (s2 == 2) { a0 = t + 1; break; }
+                b1 = t;
+                step <<= 1;
+            }
+        }
+        for (int it = 0; stt != 0 && it < 64 && a0 <= b1; ++it) {
+            j = (a0 + b1) / 2;
+            stt = check_split(min(n_ - j, numL - 1), j, target, a.Lp, numL, a.Hp, numH, sigma);
+            if (stt == 2) a0 = j + 1;
+            else if (stt == 1) b1 = j - 1;
+        }
+        if (stt == 0) {
+            out.i = (int32_t)min(n_ - j, numL - 1);
+            out.j = (int32_t)j;
+            out.spill = sigma + a.Hw[j] - target;
+            return true;
+        }
+    }
+    return false;
+}
+
 // Split k (0 < k < p, not a knot) from the model: interpolate between the
 // knots, gallop, bisect inside the bracket; full bisection when the
 // certificate is missing or the bracket search fails.
@@ -1263,57 +1322,7 @@ __device__ __forceinline__ uint32_t learned_split(const BuildArgs& a, int64_t k)
     Split out;
     bool ok = false;
     if (dl < dh) {
-        const int64_t n_ = (int64_t)ceil(((double)nToSplit * (double)k) / (double)p);
-        const int64_t b0 = min(n_, numH) - 1;
-        const double target = (wToSplit * (double)n_) / (double)nToSplit;
-        int64_t lo = a.knot_j[m], hi = a.knot_j[m + 1];
-        if (hi > b0) hi = b0;
-        if (lo < 0) lo = 0;
-        if (lo <= hi) {
-            // Model prediction: linear interpolation inside the segment.
-            int64_t j = lo + ((hi - lo) * (k - km)) / (km1 - km);
-            double sigma = 0.0;
-            int stt = check_split(min(n_ - j, numL - 1), j, target, a.Lp, numL, a.Hp, numH, sigma);
-            // Gallop from the prediction until the answer is bracketed, then bisect.
-            int64_t a0 = lo, b1 = hi;
-            if (stt == 2) {  // RIGHT: answer above j
-                a0 = j + 1;
-                int64_t step = 1;
-                while (true) {
-                    const int64_t t = j + step;
-                    if (t >= hi) { b1 = hi; break; }
-                    const int s2 = check_split(min(n_ - t, numL - 1), t, target, a.Lp, numL, a.Hp, numH, sigma);
-                    if (s2 == 0) { j = t; stt = 0; break; }
-                    if (s2 == 1) { b1 = t; break; }
-                    a0 = t + 1;
-                    step <<= 1;
-                }
-            } else if (stt == 1) {  // LEFT: answer below j
-                b1 = j;
-                int64_t step = 1;
-                while (true) {
-                    const int64_t t = j - step;
-                    if (t <= lo) { a0 = lo; break; }
-                    const int s2 = check_split(min(n_ - t, numL - 1), t, target, a.Lp, numL, a.Hp, numH, sigma);
-                    if (s2 == 0) { j = t; stt = 0; break; }
-                    if (s2 == 2) { a0 = t + 1; break; }
-                    b1 = t;
-                    step <<= 1;
-                }
-            }
-            for (int it = 0; stt != 0 && it < 64 && a0 <= b1; ++it) {
-                j = (a0 + b1) / 2;
-                stt = check_split(min(n_ - j, numL - 1), j, target, a.Lp, numL, a.Hp, numH, sigma);
-                if (stt == 2) a0 = j + 1;
-                else if (stt == 1) b1 = j - 1;
-            }
-            if (stt == 0) {
-                out.i = (int32_t)min(n_ - j, numL - 1);
-                out.j = (int32_t)j;
-                out.spill = sigma + a.Hw[j] - target;
-                ok = true;
-            }
-        }
+        ok = bracket_split(a, k, km, km1, a.knot_j[m], a.knot_j[m + 1], out);
     }
     uint32_t flags = 0;
     if (!ok) {

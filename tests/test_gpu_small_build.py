@@ -142,14 +142,14 @@ def test_mid_size_routes_match_oracle(gpu, oracle, n, section, dist, p):
 
 
 @pytest.mark.parametrize("n,section,dist,p,interleave", [
-    (2_621_440, 2048, "pareto", 1 << 18, False),     # the fewest splits that go through the index
+    (2_621_440, 2048, "pareto", 1 << 18, False),     # the fewest splits found in groups
     (2_621_440, 2048, "pareto", (1 << 18) - 1, False),
     (2_621_440, 2048, "exponential", 1 << 18, True),   # few splits left: found by bisection all the same
     (3_000_000, 40, "unit_uniform", 300_000, False),   # short chains leave heavies of less than the mean
     (3_000_000, 1000, "heavy_mix", 300_000, True),
     (2_700_000, 1000, "all_equal", 270_000, False),    # degenerate
 ])
-def test_indexed_bisection_matches_oracle(gpu, oracle, n, section, dist, p, interleave):
+def test_grouped_bisection_matches_oracle(gpu, oracle, n, section, dist, p, interleave):
     w = np.full(n, 2.5) if dist == "all_equal" else weights(n, dist)
     t = gpu_build(w, section_size=section, num_splits=p, interleave=interleave)
     ref = oracle.build(w, section_size=section, num_splits=p)
