@@ -104,7 +104,7 @@ __global__ __launch_bounds__(256) void seg_sum(SegArgs g, SegMap m) {
     seg_locate(m, t, blk);
     if (threadIdx.x == 0) atomicMin((unsigned long long*)&g.ticks[2 * t], (unsigned long long)wall_clock64());
     const BuildArgs& a = table_args(g, t);
-    sum_sections_block<T>(a, blk, (a.G + 3) / 4);
+    sum_sections_block<T>(a, blk);
 }
 
 // One block per table of the group.

@@ -28,7 +28,7 @@ struct BuildArgs {
     double* stage_w;          // n: leftovers staged by partition pass 1 (weights)
     int32_t* stage_i;         // n: leftovers staged by partition pass 1 (items)
     uint64_t* sec_cert;       // 6 G: per-section split-certificate data (bit patterns)
-    int32_t want_cert;        // compute the split certificate (learned split)
+    int32_t want_cert;        // compute the split certificate (learned, P-ary and grouped splits)
     int32_t* Li; double* Lw; double* Lp;  // leftover lights (capacity n + 2)
     int32_t* Hi; double* Hw; double* Hp;  // leftover heavies (capacity n + 2)
     Row* rows;                // AoS table or null

@@ -3,18 +3,20 @@
 //
 // Phases (one stream, no host round trips):
 //   1. sum_sections : per-section FP64 sums (one wave per section), weight
-//                     validation; sum_finish: the canonical 64-ary tree -> W, W/N.
+//                     validation; sum_finish: the canonical 64-ary tree -> W,
+//                     W/N (few sections: every partition wave does it).
 //   2. partition_local : one wave per section: all loads issued at once,
 //                     stable light/heavy partition into LDS, PSA+ greedy
-//                     chains writing finished rows, leftover order, the
-//                     canonical local-scan aggregates published into the
-//                     dyadic block tree of section sums (completed by the
-//                     second child to arrive), leftovers staged in place.
-//      partition_place : per section, P(s) from O(log G) completed blocks
-//                     (the association the oracle defines), leftover lists
-//                     with prefix sums, the split certificate, the sentinels.
-//                     No section ever waits for another to finish its work.
-//   3. degenerate_fill (only when one leftover class is empty), split, pack.
+//                     chains, finished rows, leftover order, the canonical
+//                     local-scan aggregates, leftovers staged in place.
+//      block_tree   : the dyadic tree of the section sums (many sections).
+//      partition_place : per section, P(s) from O(log G) blocks (the
+//                     association the oracle defines) or, for few sections,
+//                     from their own sums; leftover lists with prefix sums,
+//                     the split certificate's data; a wave for the totals and
+//                     sentinels.  No section ever waits for another's work.
+//   3. split (rows of a degenerate table in its first launch), pack.
+// Small tables take one launch in place of all (atg_small.h).
 #include <algorithm>
 
 #include "atg_kernels.h"
@@ -23,7 +25,7 @@ namespace atg {
 
 template <typename T>
 __global__ __launch_bounds__(256) void sum_sections(BuildArgs a) {
-    sum_sections_block<T>(a, blockIdx.x, gridDim.x);
+    sum_sections_block<T>(a, blockIdx.x);
 }
 
 __global__ __launch_bounds__(1024) void sum_finish(BuildArgs a) {
@@ -33,9 +35,9 @@ __global__ __launch_bounds__(1024) void sum_finish(BuildArgs a) {
 // ---------------------------------------------------------------------------
 // 2. PSA+ / plain partition in two passes.  The section prefixes of the
 //    leftover sums use the dyadic-block association of the oracle: each
-//    section publishes its aggregate as the level-0 block, the child that
-//    completes a pair second publishes the parent (pass 1), and P(s) folds
-//    the blocks of s's binary digits from high to low (pass 2).
+//    section stores its aggregate as the level-0 block (pass 1), block_tree
+//    builds the levels above, and P(s) folds the blocks of s's binary digits
+//    from high to low (pass 2).
 // As many waves as fit the chip at once; wave w runs sections w, w + grid,
 // ... and loads each next section while the current one's chains run.
 // XU: weights per lane held for a section (sections of up to 64 XU items);

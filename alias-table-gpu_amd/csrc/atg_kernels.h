@@ -729,7 +729,7 @@ __device__ __forceinline__ void place_section(const BuildArgs& a, int64_t s, int
     if (AHEAD && mL + mH > 0) load_group(mL == 0, 0);
     const Prefix P = DIRECT ? block_prefix_direct(a, (int)s, lane) : block_prefix_done(a, s, lane);
     const int64_t goffL = (int64_t)(uint32_t)P.c, goffH = (int64_t)(P.c >> 32);
-    // Split certificate (learned split only): the extreme increments between
+    // Split certificate (want_cert): the extreme increments between
     // consecutive stored prefixes inside the section, and the section's first
     // and last prefix of each class; the pairs across sections are closed by
     // cert_reduce_block.
@@ -841,10 +841,10 @@ __device__ __forceinline__ void place_totals(const BuildArgs& a, int lane) {
 }
 
 // ---------------------------------------------------------------------------
-// W, pass 1: section sums, one wave per section (block blk of nblk holds
-// sections 4 blk .. 4 blk + 3).
+// W, pass 1: section sums, one wave per section (block blk holds sections
+// 4 blk .. 4 blk + 3).
 template <typename T>
-__device__ __forceinline__ void sum_sections_block(const BuildArgs& a, int64_t blk, int64_t nblk) {
+__device__ __forceinline__ void sum_sections_block(const BuildArgs& a, int64_t blk) {
     const int lane = threadIdx.x & 63, wave = wave_in_block();
     const T* w = (const T*)a.weights;
     const int64_t s = blk * (blockDim.x >> 6) + wave;

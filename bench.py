@@ -37,14 +37,14 @@ METRIC = "build Gitems/s + Gsamples/s at N=1e8 (%HBM peak); learned/batched vs p
 HBM_PEAK_GBS = 8000.0
 KERNEL_PHASES = ("sum", "partition_local", "partition_place", "split", "pack")
 KERNEL_NAMES = {"sum": "sum_sections+sum_finish", "partition_local": "partition_local",
-                "partition_place": "block_tree+partition_place", "split": "split_bisect or split_knots+split_learned",
-                "pack": "pack_staged"}
+                "partition_place": "block_tree+partition_place", "split": "split_bisect, split_prepare+split_grouped or split_prepare+split_learned",
+                "pack": "pack_staged or pack_windowed"}
 # HBM bytes per launch measured with rocprofv3 FETCH_SIZE + WRITE_SIZE
 # (scaled by the counters of a device copy of known size) for the headline
 # workload at the given shape; the file holds the commands and the counts.
 MEASURED_TRAFFIC = {
     (100_000_000, 2048, 16, 1_562_500, "partition_local"): (
-        2_312_409_000, "profiles/build_pareto1e8_s2048_c16_p1562500_hbm_traffic.md"),
+        3_084_134_000, "profiles/build_pareto1e8_s2048_c16_p1562500_hbm_traffic.md"),
 }
 
 
