@@ -98,6 +98,15 @@ __device__ __forceinline__ int lanes_below(uint64_t m) {
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
+// The lane of m's set bit with k set bits below it.
+__device__ __forceinline__ int nth_lane(uint64_t m, int k) {
+    int lane = 0;
+#pragma unroll
+    for (int step = 32; step >= 1; step >>= 1)
+        if (__popcll(m & ((1ull << (lane + step)) - 1)) <= k) lane += step;
+    return lane;
+}
+
 // Orders one wave's LDS writes before its later LDS reads by other lanes.  A
 // wave's LDS operations execute in issue order, so wavefront-scope fences
 // (compiler barriers, no wait instructions) suffice; a workgroup-scope fence

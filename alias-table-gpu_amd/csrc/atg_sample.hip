@@ -502,7 +502,7 @@ __global__ __launch_bounds__(1024) void rej_scan_totals(RejArgs a) {
 // longer than REJ_WAVE slots becomes tasks of REJ_TASK slots for
 // rej_fill_long, so that heavy items, however clustered, hold up no wave for
 // long; a wave within the budget writes every run itself.  2e7 items (160 MB),
-// 3.5e7 slots (560 MB): 153 us, 199 with a search per slot and streaming
+// 3.5e7 slots (560 MB): 156 us, 199 with a search per slot and streaming
 // stores.
 template <typename T>
 __global__ __launch_bounds__(REJ_THREADS) void rej_fill(RejArgs a) {
@@ -586,7 +586,11 @@ __global__ __launch_bounds__(REJ_THREADS) void rej_fill(RejArgs a) {
             lex = il - ell;
             L = (uint32_t)__builtin_amdgcn_readlane((int)il, 63);
         }
-        int o0 = (int)(base + u * 64) - 1;  // the item of the last start before the pass
+        // An item has slots unless N w overflowed: without such items the o-th
+        // start is lane o's.
+        const uint64_t some = __ballot(cu != 0);
+        const bool gaps = (some & (some + 1)) != 0ull;
+        int o0 = -1;  // the last start before the pass
         for (uint32_t v0 = 0; v0 < L; v0 += 64) {
             const uint32_t v = v0 + lane;
             if (cu != 0 && lex - v0 < 64u) mark[lex - v0] = frac;
@@ -596,14 +600,15 @@ __global__ __launch_bounds__(REJ_THREADS) void rej_fill(RejArgs a) {
             wave_lds_sync();
             const bool start = m < 1.0;
             const uint64_t starts = __ballot(start);
-            const int o = o0 + lanes_below(starts) + (start ? 1 : 0);
+            int o = o0 + lanes_below(starts) + (start ? 1 : 0);
             o0 += __popcll(starts);
+            if (gaps) o = nth_lane(some, o);
             uint64_t f = round0;
-            if (any_long != 0ull) f = (uint64_t)__shfl((unsigned long long)(first - lex), o & 63, 64);
+            if (any_long != 0ull) f = (uint64_t)__shfl((unsigned long long)(first - lex), o, 64);
             if (v < L) {
                 RejEntry e;
                 e.accept = start ? m : 1.0;
-                e.item = o;
+                e.item = (int32_t)(base + u * 64 + o);
                 e.pad = 0;
                 rej_store(&a.A[f + v], e);
             }
@@ -836,7 +841,7 @@ __global__ __launch_bounds__(REJ_SEC_THREADS) void rej_sample_sectioned(RejSecAr
         const uint4 v = *reinterpret_cast<const uint4*>(&a.A[start + s]);
         const double acc = __longlong_as_double(((long long)v.y << 32) | v.x);
         ulonglong2 e;
-        e.x = acc >= 1.0 ? ~0ull : ((uint64_t)(acc * 0x1.0p53) << 11) | 0x7FFull;
+        e.x = !(acc < 1.0) ? ~0ull : ((uint64_t)(acc * 0x1.0p53) << 11) | 0x7FFull;
         e.y = v.z;
         rsect[s] = e;
     }

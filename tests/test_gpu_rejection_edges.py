@@ -47,3 +47,14 @@ def test_edges_match_oracle(gpu, oracle, case):
         t.rejection_sample_sectioned(count, seed=count, section_slots=1024, out=out)
         exp = oracle.sample_rejection_sectioned(A, w, W, 1024, count, count)
         np.testing.assert_array_equal(out.cpu().numpy(), exp, err_msg=f"count={count}")
+
+
+def test_items_whose_count_overflows_have_no_slots(gpu):
+    # N w is infinite for three items (W is not): the others keep theirs.
+    n, big = 5000, [100, 127, 1500]
+    w = np.ones(n)
+    w[big] = 5e304
+    t = atg.Table(n)
+    t.set_weights(w)
+    t.rejection_build()
+    np.testing.assert_array_equal(t.rejection_array(), np.delete(np.arange(n), big))
