@@ -419,7 +419,8 @@ class Table:
 
 
 class Batch:
-    """Many independent tables built together, one launch per phase (atg_batch_*).
+    """Many independent tables built together, one launch per phase,
+    small tables by a workgroup each (atg_batch_*).
 
     Table t owns weights[offsets[t]:offsets[t+1]] and is built exactly as a
     `Table` with the same options would build it alone."""

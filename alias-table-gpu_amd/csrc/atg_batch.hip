@@ -3,7 +3,8 @@
 //
 // The tables are dealt into groups (largest table first, each to the group
 // with the fewest items so far; one group unless batch_group_items is set).
-// Every phase of a group is one launch over the group's tables: a block finds
+// Small tables are built by a workgroup each (seg_small).  For the others every
+// phase of a group is one launch over the group's tables: a block finds
 // its table and its block within the table from a block->table map built at
 // creation, then runs exactly the device code of the single-table kernels
 // (the same launch shape per table: one wave per section, one wave per 64
