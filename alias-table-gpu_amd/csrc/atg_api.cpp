@@ -73,6 +73,7 @@ struct atg_table_s {
     uint32_t* d_sec_ldir = nullptr;  // lean light lists: the section of every 1024th light
     bool placed = false;             // the staging and sec_loff of the last partition are current
     bool lists_full = false;         // the last build left whole lists (no staging): a one-launch build
+    bool staged = false;             // the staging and section sums hold a partition (a one-launch build has none)
     double* d_stage_w = nullptr;
     int32_t* d_stage_i = nullptr;
     int32_t *d_Li = nullptr, *d_Hi = nullptr;
@@ -351,13 +352,19 @@ atg_status atg_build_phase(atg_table* t, int32_t phase, void* stream) {
         case ATG_PHASE_SUM: HIPCHK(launch_sum(a, s)); break;
         case ATG_PHASE_PARTITION:
             HIPCHK(launch_partition(a, s));
+            t->staged = true;
             t->placed = true;
             break;
         case ATG_PHASE_PARTITION_LOCAL:
             t->placed = false;
             HIPCHK(launch_partition_local(a, s));
+            t->staged = true;
             break;
         case ATG_PHASE_PARTITION_PLACE:
+            // A one-launch build leaves no staging, and the placement takes its
+            // positions from what the local pass left there: run it first.
+            if (!t->staged) HIPCHK(launch_partition_local(a, s));
+            t->staged = true;
             HIPCHK(launch_partition_place(a, s));
             t->placed = true;
             break;
@@ -419,6 +426,7 @@ atg_status atg_build(atg_table* t, void* stream) {
         small_build_ok(t->n, t->G, t->Ls, t->p_req)) {
         HIPCHK(launch_small(t->args(), true, nullptr, nullptr, s));
         t->placed = false;
+        t->staged = false;
         t->lists_full = true;
         t->built = true;
         return ATG_OK;
@@ -427,6 +435,7 @@ atg_status atg_build(atg_table* t, void* stream) {
         t->lists_full = false;
         const BuildArgs a = t->args();
         HIPCHK(launch_front(a, s));
+        t->staged = true;
         t->placed = true;
         hipError_t err = hipSuccess;
         if (build_split_pack_interleaved(t, a, s, err)) {
@@ -445,6 +454,7 @@ atg_status atg_build(atg_table* t, void* stream) {
     if (!t->events) {
         t->lists_full = false;
         HIPCHK(launch_front(t->args(), s));
+        t->staged = true;
         t->placed = true;
         first = ATG_PHASE_SPLIT;
     }
