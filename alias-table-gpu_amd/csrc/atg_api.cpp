@@ -724,7 +724,7 @@ atg_status atg_sample(atg_table* t, atg_sample_kind kind, uint64_t count, uint64
             HIPCHK(launch_sample_basic(a, s));
         } else if (kind == ATG_SAMPLE_SECTIONED) {
             if (section_rows <= 0) section_rows = 4096;
-            if (section_rows > 8192) return fail(ATG_EINVAL, "atg_sample: section_rows %lld > 8192", (long long)section_rows);
+            if (section_rows > kMaxSectionRows) return fail(ATG_EINVAL, "atg_sample: section_rows %lld > %lld", (long long)section_rows, (long long)kMaxSectionRows);
             a.SS = section_rows;
             a.nsec = (t->n + section_rows - 1) / section_rows;
             if (a.nsec > t->sec_counts_cap) {
@@ -916,8 +916,9 @@ atg_status atg_rejection_sample_sectioned(atg_table* t, uint64_t count, uint64_t
     if (!t) return fail(ATG_EINVAL, "atg_rejection_sample_sectioned: NULL table");
     if (!t->rej_built) return fail(ATG_ESTATE, "atg_rejection_sample_sectioned: rejection structure not built");
     if (section_slots <= 0) section_slots = 4096;
-    if (section_slots > 8192)
-        return fail(ATG_EINVAL, "atg_rejection_sample_sectioned: section_slots %lld > 8192", (long long)section_slots);
+    if (section_slots > kMaxSectionRows)
+        return fail(ATG_EINVAL, "atg_rejection_sample_sectioned: section_slots %lld > %lld", (long long)section_slots,
+                    (long long)kMaxSectionRows);
     hipStream_t s = (hipStream_t)stream;
     if (!t->rej_size_known) {
         // |A| sizes the launch: read back once per rejection build.

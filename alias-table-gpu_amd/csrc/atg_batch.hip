@@ -380,8 +380,10 @@ hipError_t launch_class(const SmallClass& c, const SegArgs& g, const BatchGroup:
     static_assert(sizeof(kSmallChunks) / sizeof(int) == 4, "a kernel per length");
     void (*const k[])(SegArgs, const int32_t*) = {seg_small<T, kSmallChunks[0]>, seg_small<T, kSmallChunks[1]>,
                                                   seg_small<T, kSmallChunks[2]>, seg_small<T, kSmallChunks[3]>};
+    // The limit is state of the process: always the most that any class needs,
+    // so that no launch lowers it under another batch's or a captured one.
     if (c.lds > kSmallLdsDefault) {
-        const hipError_t e = hipFuncSetAttribute((const void*)k[c.xu], hipFuncAttributeMaxDynamicSharedMemorySize, (int)c.lds);
+        const hipError_t e = hipFuncSetAttribute((const void*)k[c.xu], hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallTiers[2]);
         if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL(k[c.xu], dim3((unsigned)sm.blocks), dim3(c.threads), c.lds, s, g, sm.tab);

@@ -23,6 +23,10 @@ enum : uint32_t {
 // low-acceptance slots can need many, but it draws few samples.
 #define REJ_SECTIONED_MAX_TRIALS (1u << 20)
 
+// The longest section (rows of a table, slots of A) that a sectioned sampler
+// stages: 128 KB of a CU's 160 KB of LDS, beside the counts.
+constexpr int64_t kMaxSectionRows = 8192;
+
 struct SampleArgs {
     const Row* rows;       // AoS table or null
     const double* tw;      // SoA table or null

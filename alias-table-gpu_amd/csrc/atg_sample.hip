@@ -939,11 +939,14 @@ static void launch_sparse(const SampleArgs& a, hipStream_t s) {
 static size_t sectioned_lds(int64_t rows, bool hist) { return (size_t)rows * sizeof(Row) + (hist ? 8 * kSecHistSlots : 0); }
 
 // A block per section with `lds` bytes; beyond 64 KB a kernel has to be
-// allowed its LDS first.
+// allowed its LDS first.  The limit is state of the process: always that of the
+// longest sections with counts, so that no call lowers it under another
+// thread's launch or a captured one.
 template <typename... Args>
 static hipError_t launch_sectioned(void (*k)(Args...), int64_t nsec, int threads, size_t lds, hipStream_t s, Args... args) {
     if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 (int)sectioned_lds(kMaxSectionRows, true));
         if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL(k, dim3((unsigned)nsec), dim3(threads), lds, s, args...);

@@ -21,8 +21,10 @@ static hipError_t launch_small_t(const BuildArgs& a, double* W_out, uint32_t* er
         : shorts    ? build_small<T, AOS, kShortSectionMax / 64, 64 * kSmallMaxWaves, LISTS>
                     : build_small<T, AOS, PSA_MAX_LEN / 64, 64 * kSmallLongWaves, LISTS>;
     const size_t lds = SmallLds(a.n, a.p_req).bytes();
+    // The limit is state of the process: always the most that any table needs,
+    // so that no call lowers it under another thread's launch or a captured one.
     if (lds > kSmallLdsDefault) {
-        const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLdsMax);
         if (e != hipSuccess) return e;
     }
     // A wave per section and a thread per pack chain.

@@ -66,3 +66,29 @@ def test_sparse_sections_match_oracle(gpu, oracle, layout, n, rows, count):
     np.testing.assert_array_equal(out.cpu().numpy()[:count], exp)
     t.sample(count, 31, section_rows=rows, hist=hist)
     np.testing.assert_array_equal(hist.cpu().numpy(), np.bincount(exp, minlength=n))
+
+
+@pytest.mark.parametrize("layout", ["aos", "soa"])
+def test_longest_sections_with_counts(gpu, oracle, layout):
+    """8,192 rows or slots and the block's counters: the most LDS of a draw."""
+    torch = gpu
+    n, count = 50_001, 60_000
+    w = atg.generate_weights("pareto", n, seed=9, param=1.1)
+    t = atg.Table(n, layout=layout)
+    t.set_weights(w)
+    t.build()
+    tw, ta = t.table()
+    out = torch.empty(count, dtype=torch.int32, device="cuda")
+    hist = torch.zeros(n, dtype=torch.int32, device="cuda")
+    t.sample(count, 31, section_rows=8192, out=out, hist=hist)
+    exp = oracle.sample_sectioned(tw, ta, t.stats()["W_N"], 8192, count, 31)
+    np.testing.assert_array_equal(out.cpu().numpy(), exp)
+    np.testing.assert_array_equal(hist.cpu().numpy(), np.bincount(exp, minlength=n))
+    t.rejection_build()
+    W = t.rejection_weight_sum()
+    _, A = oracle.rejection_build(w, W)
+    hist.zero_()
+    t.rejection_sample_sectioned(count, 32, section_slots=8192, out=out, hist=hist)
+    exp = oracle.sample_rejection_sectioned(A, w, W, 8192, count, 32)
+    np.testing.assert_array_equal(out.cpu().numpy(), exp)
+    np.testing.assert_array_equal(hist.cpu().numpy(), np.bincount(exp, minlength=n))
