@@ -420,10 +420,9 @@ atg_status atg_build(atg_table* t, void* stream) {
     if (!t->weights_set) return fail(ATG_ESTATE, "atg_build: weights not set");
     hipStream_t s = (hipStream_t)stream;
     t->last_stream = s;
-    // A small table in one launch.  Not where the phases are timed or overlapped
-    // on request, nor for the searches whose certificate the stats report.
-    if (t->opts.split_method == ATG_SPLIT_BISECT && !t->opts.interleave && !t->events &&
-        small_build_ok(t->n, t->G, t->Ls, t->p_req)) {
+    // A small table in one launch, but not where the phases are timed or
+    // overlapped on request.
+    if (!t->opts.interleave && !t->events && one_launch_ok(t->opts, t->n, t->G, t->Ls, t->p_req)) {
         HIPCHK(launch_small(t->args(), true, nullptr, nullptr, s));
         t->placed = false;
         t->staged = false;

@@ -7,6 +7,7 @@
 #include <cstddef>
 
 #include "../../include/atg.h"
+#include "atg_build.h"
 #include "atg_types.h"
 
 namespace atg {
@@ -30,6 +31,12 @@ atg_status table_set_shape(atg_table* t, int32_t chains, int64_t num_splits);
 constexpr int64_t kGroupedSplits = (int64_t)1 << 18;
 inline bool split_by_group(int32_t split_method, int64_t p_req) {
     return split_method == ATG_SPLIT_BISECT && p_req >= kGroupedSplits;
+}
+// Whether a build takes the one-launch kernel, which stands for the default
+// methods: a pack or split that the caller chose runs as chosen (and reports
+// its certificate and fallbacks).
+inline bool one_launch_ok(const atg_build_opts& o, int64_t n, int64_t G, int64_t Ls, int64_t p_req) {
+    return o.split_method == ATG_SPLIT_BISECT && o.pack_method == ATG_PACK_CHUNKED && small_build_ok(n, G, Ls, p_req);
 }
 // Sets the split method, knot count and split/pack interleave of a created
 // table (knobs that leave the table's rows unchanged).

@@ -155,7 +155,7 @@ extern "C" atg_status atg_build_noalloc(const void* weights, atg_dtype dtype, in
     a.pack_method = o.pack_method;
 
     hipStream_t s = (hipStream_t)stream;
-    if (small_build_ok(n, G, Ls, p_req)) {
+    if (one_launch_ok(o, n, G, Ls, p_req)) {
         HIPCHK(launch_small(a, false, W_out, error_out, s));
         return ATG_OK;
     }

@@ -47,7 +47,10 @@ typedef enum {
 
 /* Pack of the leftover lists into rows (Variant::pack and sharedMemory,
  * AliasTableSplitGpu.cuh:38-94, dispatched in performPack,
- * AliasTableSplitGpu.cu:506-591).  Every method writes the same rows. */
+ * AliasTableSplitGpu.cu:506-591).  Every method writes the same rows.  Small
+ * tables of the default methods (bisection, CHUNKED) are built by one kernel;
+ * with any other split or pack method atg_build and atg_build_noalloc run the
+ * kernels of that method at every size. */
 typedef enum {
     ATG_PACK_CHUNKED = 0,    /* one wave per 64 chains, their lists staged in LDS in rounds
                                 (the role of PackMethodBasicShared / PackMethodChunkedShared); default */
@@ -337,8 +340,10 @@ atg_status atg_generate_batch(int32_t dist, int64_t ntables, int64_t lo, int64_t
 
 typedef struct atg_batch_s atg_batch;
 
-/* Tables t = 0..ntables-1 own weights[offsets[t], offsets[t+1]).  Each table is
- * built exactly as atg_build would build it alone with the same options. */
+/* Tables t = 0..ntables-1 own weights[offsets[t], offsets[t+1]).  Each table's
+ * rows are exactly those that atg_build would build alone with the same
+ * options.  Small tables may be built by a workgroup each, which finds their
+ * splits by bisection whatever split_method is (the same splits). */
 atg_status atg_batch_create(atg_batch** out, const int64_t* offsets_host, int64_t ntables,
                             atg_dtype dtype, const atg_build_opts* opts);
 void atg_batch_destroy(atg_batch* b);

@@ -1,0 +1,37 @@
+"""Which kernels a call launches: explicit choices of the caller, and the
+rules on sizes."""
+import pytest
+
+import atg
+from launches import kernels
+
+pytestmark = pytest.mark.gpu
+
+
+def build(torch, n, **kw):
+    t = atg.Table(n, **kw)
+    t.set_weights(atg.generate_weights("pareto", n, seed=3, param=1.1))
+    return kernels(torch, t.build)
+
+
+def noalloc(torch, n, **kw):
+    w = torch.from_numpy(atg.generate_weights("pareto", n, seed=3, param=1.1)).cuda()
+    rows = torch.zeros(2 * n, dtype=torch.float64, device="cuda")
+    atg.build_noalloc(w, rows)  # finds the scratch array, outside the capture
+    return kernels(torch, lambda s: atg.build_noalloc(w, rows, stream=s, **kw))
+
+
+@pytest.mark.parametrize("n", [11, 1000, 5000])
+def test_small_tables_keep_explicit_methods(gpu, n):
+    """The one-launch build stands for the default pack and the bisection; a
+    pack or split method that the caller names is the one that runs."""
+    assert build(gpu, n) == ["build_small"]
+    assert noalloc(gpu, n) == ["build_small"]
+    for pack, psa in (("basic", True), ("basic", False), ("no_weights", False)):
+        ks = build(gpu, n, pack=pack, psa_plus=psa)
+        assert "pack_basic" in ks and "build_small" not in ks
+        ks = noalloc(gpu, n, pack=pack, psa_plus=psa)
+        assert "pack_basic" in ks and "build_small" not in ks
+    for split, kernel in (("learned", "split_learned"), ("pary", "split_pary")):
+        assert kernel in build(gpu, n, split=split)
+        assert kernel in noalloc(gpu, n, split=split)
