@@ -265,21 +265,6 @@ using namespace atg;
 
 enum { MAP_SUM, MAP_LOCAL, MAP_PLACE, MAP_SPLIT, MAP_PREPARE, MAP_PACK, MAP_TREE, MAP_ONE, MAP_COUNT };
 
-// Tables built by seg_small, in classes by their sections' length (kSmallChunks
-// chunks of 64 items a lane) and number (waves, a power of two) and by how
-// many tables fit a CU (one, two, more).  A class has one launch, with the LDS
-// of its largest table, so that small tables are not held to the occupancy of
-// larger ones; finer classes lose more at the ends of their launches than
-// occupancy gains (16,384 tables of 16 to 4,096 items 230 us, 238 with four
-// more tiers of LDS below 32 KB).
-constexpr int kSmallChunks[] = {2, 8, 16, 32};
-constexpr size_t kSmallTiers[] = {52 * 1024, 79 * 1024, 154 * 1024};  // of 160 KB, static LDS aside
-struct SmallClass {
-    int xu;            // index into kSmallChunks
-    int waves, tier;
-    int threads = 64;  // of the table with the most sections
-    size_t lds = 0;    // of the largest table
-};
 // Small tables hold at least one item in this many, or go through the phases
 // (100 of them among 1,024 tables of up to 2^20 items: 3.06 ms in the phases,
 // 3.10 by themselves).
@@ -719,18 +704,10 @@ atg_status atg_batch_create(atg_batch** out, const int64_t* offsets, int64_t nta
         a.splits = b->d_splits + osp[t];
         a.learned_segments = learned_knots(o.learned_segments, z.p_req);
     }
-    // Small tables: a wave per section and all of the table within a CU's LDS.
     int64_t small_items = 0;
     auto small_key = [&](int64_t t, SmallClass& c) {
         const BuildArgs& a = b->args[t];
-        c.xu = 0;
-        c.waves = 1;
-        c.tier = 0;
-        while (a.Ls > 64 * kSmallChunks[c.xu]) ++c.xu;
-        while (a.G > c.waves) c.waves *= 2;
-        c.lds = SmallLds(a.n, a.p_req).compact_bytes();
-        while (c.tier < 2 && c.lds > kSmallTiers[c.tier]) ++c.tier;
-        return c.waves <= (a.Ls <= kShortSectionMax ? kSmallMaxWaves : kSmallLongWaves) && c.lds <= kSmallTiers[2];
+        return small_class_of(a.n, a.G, a.Ls, a.p_req, c);
     };
     SmallClass key;
     for (int64_t t = 0; t < ntables; ++t)

@@ -27,6 +27,35 @@ struct SmallLds {
     __host__ __device__ size_t compact_bytes() const { return (size_t)items * (8 + 2) + (size_t)splits * 16; }
 };
 
+// Tables built by seg_small, in classes by their sections' length (kSmallChunks
+// chunks of 64 items a lane) and number (waves, a power of two) and by how
+// many tables fit a CU (one, two, more).  A class has one launch, with the LDS
+// of its largest table, so that small tables are not held to the occupancy of
+// larger ones; finer classes lose more at the ends of their launches than
+// occupancy gains (16,384 tables of 16 to 4,096 items 230 us, 238 with four
+// more tiers of LDS below 32 KB).
+constexpr int kSmallChunks[] = {2, 8, 16, 32};
+constexpr size_t kSmallTiers[] = {52 * 1024, 79 * 1024, 154 * 1024};  // of 160 KB, static LDS aside
+struct SmallClass {
+    int xu;            // index into kSmallChunks
+    int waves, tier;
+    int threads = 64;  // of the table with the most sections
+    size_t lds = 0;    // of the largest table
+};
+// The class of a table of n items in G sections of Ls, false: not small.  Small
+// tables have a wave per section and fit a CU's LDS.
+inline bool small_class_of(int64_t n, int64_t G, int64_t Ls, int64_t p_req, SmallClass& c) {
+    if (G > (Ls <= kShortSectionMax ? kSmallMaxWaves : kSmallLongWaves)) return false;
+    c.xu = 0;
+    c.waves = 1;
+    c.tier = 0;
+    while (Ls > 64 * kSmallChunks[c.xu]) ++c.xu;
+    while (G > c.waves) c.waves *= 2;
+    c.lds = SmallLds(n, p_req).compact_bytes();
+    while (c.tier < 2 && c.lds > kSmallTiers[c.tier]) ++c.tier;
+    return c.lds <= kSmallTiers[2];
+}
+
 // The light list followed by the heavy list (from entry numL) in LDS.
 struct SmallLists {
     const double* w;

@@ -1,0 +1,57 @@
+"""The host rules that choose kernels by size, compiled from the library's own
+headers and asked on the CPU, also for sizes too large to allocate."""
+import os
+import subprocess
+
+import pytest
+
+import build_lib
+
+PROGRAM = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "atg_small.h"
+using namespace atg;
+int main(int argc, char** argv) {
+    auto arg = [&](int k) { return atoll(argv[k]); };
+    const char* what = argv[1];
+    if (what[0] == 's') {  // small_class n G Ls p
+        SmallClass c;
+        if (small_class_of(arg(2), arg(3), arg(4), arg(5), c)) printf("%d %d %d\n", kSmallChunks[c.xu], c.waves, c.tier);
+        else printf("none\n");
+    }
+    return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    src, exe = str(d / "rules.cpp"), str(d / "rules")
+    with open(src, "w") as f:
+        f.write(PROGRAM)
+    r = subprocess.run([build_lib.HIPCC, "-O1", "-std=c++17", "-x", "hip", "--cuda-host-only",
+                        f"--offload-arch={build_lib.ARCH}", "-I" + build_lib.CSRC, src, "-o", exe],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+
+    def ask(*args):
+        return subprocess.run([exe] + [str(a) for a in args], capture_output=True, text=True, check=True,
+                              timeout=10).stdout.strip()
+    return ask
+
+
+@pytest.mark.parametrize("n,G,Ls,p,want", [
+    (1, 1, 1, 2, "2 1 0"),
+    (1000, 11, 100, 100, "2 16 0"),
+    (1600, 16, 100, 160, "2 16 0"),
+    (1700, 17, 100, 170, "none"),              # a section more than a workgroup has waves
+    (8192, 4, 2048, 200, "32 4 2"),
+    (9000, 5, 2048, 200, "none"),              # a long section more
+    (14_000, 15, 1000, 1400, "none"),          # past a CU's LDS
+    ((1 << 30) + 1, (1 << 30) + 1, 1, 2, "none"),   # more sections than an int's powers of two
+    ((1 << 31) - 17, (1 << 31) - 17, 1, 2, "none"),
+])
+def test_small_class(rule, n, G, Ls, p, want):
+    assert rule("small_class", n, G, Ls, p) == want
