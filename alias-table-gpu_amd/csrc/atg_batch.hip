@@ -12,7 +12,7 @@
 // weights built alone with the same options.  The groups run one after the
 // other, so a table is done when its group is.  Per-table latencies come from
 // the 100 MHz device clock: the first block of the table's sum phase to the
-// last block of its pack.
+// last block of its pack, or a small table's workgroup from start to end.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -233,6 +233,7 @@ void seg_small(SegArgs g, const int32_t* tab) {
     const int64_t t = tab[blockIdx.x];
     if (threadIdx.x == 0) g.ticks[2 * t] = (uint64_t)wall_clock64();
     small_build<T, true, XU, false, true>(table_args(g, t), nullptr, nullptr, lds_raw);
+    __syncthreads();  // the table ends with the last wave's chains
     if (threadIdx.x == 0) g.ticks[2 * t + 1] = (uint64_t)wall_clock64();
 }
 

@@ -86,8 +86,8 @@ typedef struct {
     int64_t batch_group_items; /* batch only: the tables are dealt into groups of about this many
                                 items (largest table first, each to the lightest group) and the
                                 phases run group after group, so a table's build latency is its
-                                group's, not the whole batch's; <= 0: one group.  Same tables
-                                either way. */
+                                group's (a small table's: its workgroup's), not the whole
+                                batch's; <= 0: one group.  Same tables either way. */
     int32_t pack_method;     /* atg_pack_method (Variant::pack + sharedMemory); same table for each */
     int32_t reserved0;       /* 0 */
 } atg_build_opts;
@@ -370,7 +370,8 @@ atg_status atg_batch_use_graph(atg_batch* b, int32_t enable);
  * local to table t. */
 atg_status atg_batch_sample(atg_batch* b, uint64_t per_table, uint64_t seed, int32_t* out,
                             void* stream);
-/* Per-table build latency in ns from device timestamps (last build). */
+/* Per-table build latency in ns from device timestamps (last build): first to
+ * last phase, or, for a small table, start to end of its workgroup. */
 atg_status atg_batch_latencies(atg_batch* b, double* ns_per_table);
 
 /* ---- autotuner ----------------------------------------------------------- */
