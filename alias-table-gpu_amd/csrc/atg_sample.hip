@@ -6,6 +6,8 @@
 // Randomness: Philox4x32-10, key = seed, counter = (output position, purpose,
 // extra).  Every sample is a pure function of (table, seed, position), so any
 // launch shape yields the same output.
+#include <algorithm>
+
 #include "atg_device.h"
 #include "atg_sample.h"
 
@@ -36,6 +38,14 @@ constexpr int kHistThreads = 512;
 // Samples a block draws at least, so that clearing and flushing its slots
 // (8 per thread each) stays small beside them.
 constexpr int kHistMinPerBlock = 8192;
+// Calls of fewer samples count in HBM: few of them meet on one counter.
+constexpr uint64_t kHistMinCount = 2 * kHistMinPerBlock;
+// Blocks that few samples are spread over all the same, down to a sample a
+// thread: fewer draw round after round while the card idles (16,384 and 65,536
+// samples of 300,000 uniform items 23.0 and 23.6 us in two and eight blocks,
+// 4.9 and 7.1 in 32 and 128; counted in HBM 5.1 and 5.2, but 6.0 and 16.9 of
+// Pareto items, whose hot ones queue there, against 4.8 and 6.3).
+constexpr uint64_t kHistSpread = 128;
 
 template <int SLOTS>
 struct HistCache {
@@ -895,10 +905,9 @@ static inline unsigned grid_for(uint64_t count, unsigned block, unsigned cap) {
 }
 
 hipError_t launch_sample_basic(const SampleArgs& a, hipStream_t s) {
-    // Counts per item: through LDS once two blocks have their least share of
-    // samples; below that few samples meet on one counter.
-    if (a.hist && a.count >= 2 * (uint64_t)kHistMinPerBlock) {
-        const unsigned g = grid_for(a.count, kHistMinPerBlock, 256 * 4);
+    if (a.hist && a.count >= kHistMinCount) {
+        const uint64_t spread = std::min(kHistSpread, a.count / kHistThreads);
+        const unsigned g = (unsigned)std::max<uint64_t>(spread, grid_for(a.count, kHistMinPerBlock, 256 * 4));
         if (a.rows) hipLaunchKernelGGL((sample_basic<true, true>), dim3(g), dim3(kHistThreads), 0, s, a);
         else hipLaunchKernelGGL((sample_basic<false, true>), dim3(g), dim3(kHistThreads), 0, s, a);
         return hipGetLastError();

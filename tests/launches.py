@@ -32,7 +32,7 @@ def _names():
 
 
 def launches(torch, call):
-    """[(kernel, blocks, threads)] that call(stream) enqueues."""
+    """[(kernel, blocks, threads, dynamic LDS)] that call(stream) enqueues."""
     L = atg.lib()
     stream = torch.cuda.Stream()
     graph = C.c_void_p()
@@ -53,10 +53,10 @@ def launches(torch, call):
         if kind.value == 0:
             p = _KernelNode()
             assert L.hipGraphKernelNodeGetParams(C.c_void_p(node), C.byref(p)) == 0
-            found.append((_names().get(p.func, "?"), p.grid.x, p.block.x))
+            found.append((_names().get(p.func, "?"), p.grid.x, p.block.x, p.shared))
     assert L.hipGraphDestroy(graph) == 0
     return found
 
 
 def kernels(torch, call):
-    return [name for name, _, _ in launches(torch, call)]
+    return [k[0] for k in launches(torch, call)]

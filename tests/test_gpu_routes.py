@@ -3,7 +3,7 @@ rules on sizes."""
 import pytest
 
 import atg
-from launches import kernels
+from launches import kernels, launches
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +35,20 @@ def test_small_tables_keep_explicit_methods(gpu, n):
     for split, kernel in (("learned", "split_learned"), ("pary", "split_pary")):
         assert kernel in build(gpu, n, split=split)
         assert kernel in noalloc(gpu, n, split=split)
+
+
+def counted(torch, n, count, kind, rows=4096):
+    t = atg.Table(n)
+    t.set_weights(atg.generate_weights("pareto", n, seed=3, param=1.1))
+    t.build()
+    t.sync()
+    hist = torch.zeros(n, dtype=torch.int32, device="cuda")
+    return launches(torch, lambda s: t.sample(count, 1, kind=kind, section_rows=rows, hist=hist, stream=s))
+
+
+@pytest.mark.parametrize("count", [16_383, 16_384, 20_001, 65_536, 200_000, 1_000_000])
+def test_basic_counts_of_few_samples_fill_the_card(gpu, count):
+    """Few samples with counts are spread over blocks down to a sample a
+    thread, up to 128 blocks."""
+    (_, blocks, threads, _), = counted(gpu, 300_000, count, "basic")
+    assert blocks * threads >= min(count - threads, 128 * 512)
