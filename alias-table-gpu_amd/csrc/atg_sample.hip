@@ -932,8 +932,12 @@ template <bool AOS>
 static void launch_sparse(const SampleArgs& a, hipStream_t s) {
     const bool counts = a.nsec <= kSparseCounts;
     if (!counts) hipLaunchKernelGGL(section_counts, dim3((unsigned)((a.nsec + 63) / 64)), dim3(64), 0, s, a);
-    if (a.hist && a.count >= 2 * (uint64_t)kHistMinPerBlock) {
-        const unsigned g = grid_for(min(a.count / kHistMinPerBlock, (uint64_t)(a.nsec + 7) / 8), 1, 256 * 4);
+    if (a.hist && a.count >= kHistMinCount) {
+        // As many blocks as their waves have sections: each section costs a wave
+        // a few dependent reads however few its samples (16,384 and 65,536
+        // samples of 3e6 rows, us: a block for every 8,192 of them 314 and 98,
+        // so 10 and 12; without counts 6.9 and 7.3).
+        const unsigned g = grid_for((uint64_t)a.nsec, kHistThreads / 64, 256 * 4);
         const dim3 b(kHistThreads);
         if (counts) hipLaunchKernelGGL((sample_sectioned_sparse<AOS, true, true>), dim3(g), b, 0, s, a);
         else hipLaunchKernelGGL((sample_sectioned_sparse<AOS, true, false>), dim3(g), b, 0, s, a);

@@ -43,6 +43,7 @@ def counted(torch, n, count, kind, rows=4096):
     t.build()
     t.sync()
     hist = torch.zeros(n, dtype=torch.int32, device="cuda")
+    t.sample(count, 1, kind=kind, section_rows=rows)  # grows the buffer of the sections' counts
     return launches(torch, lambda s: t.sample(count, 1, kind=kind, section_rows=rows, hist=hist, stream=s))
 
 
@@ -52,3 +53,14 @@ def test_basic_counts_of_few_samples_fill_the_card(gpu, count):
     thread, up to 128 blocks."""
     (_, blocks, threads, _), = counted(gpu, 300_000, count, "basic")
     assert blocks * threads >= min(count - threads, 128 * 512)
+
+
+@pytest.mark.parametrize("n,rows,count", [(3_000_000, 4096, 16_384), (3_000_000, 4096, 300_000),
+                                          (3_000_000, 200, 20_000), (300_000, 4096, 16_384)])
+def test_sparse_counts_have_a_wave_per_section(gpu, n, rows, count):
+    """Draws that read their rows one by one find each section's samples by a
+    wave: with counts there are as many waves as sections, or the card is full."""
+    ks = counted(gpu, n, count, "sectioned", rows)
+    name, blocks, threads, _ = ks[-1]
+    assert name == "sample_sectioned_sparse"
+    assert blocks * threads // 64 >= min((n + rows - 1) // rows, 8192)
