@@ -92,3 +92,19 @@ def test_longest_sections_with_counts(gpu, oracle, layout):
     exp = oracle.sample_rejection_sectioned(A, w, W, 8192, count, 32)
     np.testing.assert_array_equal(out.cpu().numpy(), exp)
     np.testing.assert_array_equal(hist.cpu().numpy(), np.bincount(exp, minlength=n))
+
+
+@pytest.mark.parametrize("count", [1, 2047, 2048])
+def test_few_staged_counts(gpu, count):
+    """Staged draws below and at the fewest samples that count in LDS."""
+    torch = gpu
+    n = 1000
+    t = atg.Table(n)
+    t.set_weights(atg.generate_weights("pareto", n, seed=3, param=1.1))
+    t.build()
+    t.rejection_build()
+    out = torch.empty(count, dtype=torch.int32, device="cuda")
+    for draw in (lambda **k: t.sample(count, 5, **k), lambda **k: t.rejection_sample_sectioned(count, 5, **k)):
+        hist = torch.zeros(n, dtype=torch.int32, device="cuda")
+        draw(out=out, hist=hist)
+        np.testing.assert_array_equal(hist.cpu().numpy(), np.bincount(out.cpu().numpy(), minlength=n))

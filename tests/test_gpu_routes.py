@@ -64,3 +64,17 @@ def test_sparse_counts_have_a_wave_per_section(gpu, n, rows, count):
     name, blocks, threads, _ = ks[-1]
     assert name == "sample_sectioned_sparse"
     assert blocks * threads // 64 >= min((n + rows - 1) // rows, 8192)
+
+
+@pytest.mark.parametrize("count,counters", [(2047, 0), (2048, 16_384)])
+def test_staged_counts_of_few_samples(gpu, count, counters):
+    """Staged sections hold LDS counters from 2,048 samples on."""
+    n, hist = 1000, gpu.zeros(1000, dtype=gpu.int32, device="cuda")
+    name, _, _, lds = counted(gpu, n, count, "sectioned")[-1]
+    assert (name, lds) == ("sample_sectioned", 4096 * 16 + counters)
+    t = atg.Table(n)
+    t.set_weights(atg.generate_weights("pareto", n, seed=3, param=1.1))
+    t.rejection_build()
+    t.rejection_sample_sectioned(count, 1)  # reads the array's size back, outside the capture
+    name, _, _, lds = launches(gpu, lambda s: t.rejection_sample_sectioned(count, 1, hist=hist, stream=s))[-1]
+    assert (name, lds) == ("rej_sample_sectioned", 4096 * 16 + counters)
