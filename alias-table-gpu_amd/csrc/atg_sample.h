@@ -83,6 +83,15 @@ struct RejSecArgs {
     uint64_t* sec_counts;  // 2 nsec: count and first output of each section
 };
 
+#define REJ_SEC_THREADS 1024
+// A wave's share of m samples of a section of A: a lane's worth at least, so
+// that few samples don't leave each of the block's 16 waves with a few lanes at
+// work (1e6 samples of 2e7 items, 114 a section, with m / 16: 146 us, 120
+// before the waves had shares; so 113).
+__host__ __device__ inline uint32_t rej_share(uint32_t m) {
+    const uint32_t per = (m + REJ_SEC_THREADS / 64 - 1) / (REJ_SEC_THREADS / 64);
+    return per < 64 ? 64 : per;
+}
 hipError_t launch_sample_basic(const SampleArgs& a, hipStream_t s);
 // masses: recompute the section masses and their prefix (a new A or section size).
 hipError_t launch_rejection_sample_sectioned(const RejSecArgs& a, const SampleArgs& sa, bool masses, hipStream_t s);

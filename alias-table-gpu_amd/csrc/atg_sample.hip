@@ -734,7 +734,7 @@ __global__ __launch_bounds__(256) void rej_sample(RejArgs a, SampleArgs sa) {
 // sum of P(s) over the section: the sample count of each section comes from
 // the halving tree with q from the exclusive prefix of the M_k, and inside a
 // section a sample repeats trials on uniform slots of the LDS-staged section.
-#define REJ_SEC_THREADS 1024
+#define REJ_STAGE 4  // slots a thread stages at once
 
 __device__ __forceinline__ double rej_accept_prob(double accept) {
     return accept >= 1.0 ? 1.0 : (floor(accept * 0x1.0p53) + 1.0) * 0x1.0p-53;
@@ -848,13 +848,25 @@ __global__ __launch_bounds__(REJ_SEC_THREADS) void rej_sample_sectioned(RejSecAr
     const int64_t k = blockIdx.x;
     const uint64_t start = (uint64_t)k * (uint64_t)a.SS;
     const uint32_t len = (uint32_t)(min(a.A_size, start + (uint64_t)a.SS) - start);
-    for (uint32_t s = threadIdx.x; s < len; s += blockDim.x) {
-        const uint4 v = *reinterpret_cast<const uint4*>(&a.A[start + s]);
-        const double acc = __longlong_as_double(((long long)v.y << 32) | v.x);
-        ulonglong2 e;
-        e.x = !(acc < 1.0) ? ~0ull : ((uint64_t)(acc * 0x1.0p53) << 11) | 0x7FFull;
-        e.y = v.z;
-        rsect[s] = e;
+    // REJ_STAGE slots per thread in flight, or the conversion of one delays the
+    // load of the next (20,000 samples with counts of 2e7 items, us: 118 one by
+    // one, 110 so, 105 before there was a conversion and counters).
+    for (uint32_t s0 = threadIdx.x; s0 < len; s0 += REJ_STAGE * REJ_SEC_THREADS) {
+        uint4 v[REJ_STAGE];
+#pragma unroll
+        for (int q = 0; q < REJ_STAGE; ++q) {
+            const uint32_t s = min(s0 + q * REJ_SEC_THREADS, len - 1);
+            v[q] = *reinterpret_cast<const uint4*>(&a.A[start + s]);
+        }
+#pragma unroll
+        for (int q = 0; q < REJ_STAGE; ++q) {
+            const uint32_t s = s0 + q * REJ_SEC_THREADS;
+            const double acc = __longlong_as_double(((long long)v[q].y << 32) | v[q].x);
+            ulonglong2 e;
+            e.x = !(acc < 1.0) ? ~0ull : ((uint64_t)(acc * 0x1.0p53) << 11) | 0x7FFull;
+            e.y = v[q].z;
+            if (s < len) rsect[s] = e;
+        }
     }
     __syncthreads();
     const uint64_t cnt = a.sec_counts[2 * k], end = a.sec_counts[2 * k + 1] + cnt;
@@ -872,7 +884,7 @@ __global__ __launch_bounds__(REJ_SEC_THREADS) void rej_sample_sectioned(RejSecAr
         // trials' Philox rounds: 1e8 samples at 1.74 trials each 0.58 ms with
         // a fixed set of samples a lane, 0.39 so.
         const uint32_t m = (uint32_t)(seg_end - b);
-        const uint32_t per = (m + REJ_SEC_THREADS / 64 - 1) / (REJ_SEC_THREADS / 64);
+        const uint32_t per = rej_share(m);
         const uint32_t w0 = min(m, (uint32_t)wave * per), w1 = min(m, w0 + per);
         uint32_t t = w0 + lane, tr = 0, next = w0 + 64;
         while (__ballot(t < w1) != 0ull) {

@@ -10,6 +10,7 @@ import build_lib
 PROGRAM = r"""
 #include <cstdio>
 #include <cstdlib>
+#include "atg_sample.h"
 #include "atg_small.h"
 using namespace atg;
 int main(int argc, char** argv) {
@@ -20,6 +21,7 @@ int main(int argc, char** argv) {
         if (small_class_of(arg(2), arg(3), arg(4), arg(5), c)) printf("%d %d %d\n", kSmallChunks[c.xu], c.waves, c.tier);
         else printf("none\n");
     }
+    if (what[0] == 'r') printf("%u\n", rej_share((uint32_t)arg(2)));  // rej_share m
     return 0;
 }
 """
@@ -55,3 +57,10 @@ def rule(tmp_path_factory):
 ])
 def test_small_class(rule, n, G, Ls, p, want):
     assert rule("small_class", n, G, Ls, p) == want
+
+
+@pytest.mark.parametrize("m,want", [(1, 64), (64, 64), (114, 64), (1024, 64), (1025, 65), (40_000, 2500),
+                                    ((1 << 31) - 1, 1 << 27)])
+def test_rejection_share(rule, m, want):
+    """16 shares hold every sample, none of fewer than a wave's lanes."""
+    assert rule("rej_share", m) == str(want) and 16 * want >= m
