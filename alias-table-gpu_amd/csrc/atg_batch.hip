@@ -231,10 +231,16 @@ __global__ __launch_bounds__(64 * (64 * XU <= kShortSectionMax ? kSmallMaxWaves 
 void seg_small(SegArgs g, const int32_t* tab) {
     extern __shared__ double lds_raw[];
     const int64_t t = tab[blockIdx.x];
-    if (threadIdx.x == 0) g.ticks[2 * t] = (uint64_t)wall_clock64();
+    __shared__ uint32_t ended;  // waves that have left the build
+    if (threadIdx.x == 0) {
+        ended = 0u;  // the build's first barrier comes before any wave leaves it
+        g.ticks[2 * t] = (uint64_t)wall_clock64();
+    }
     small_build<T, true, XU, false, true>(table_args(g, t), nullptr, nullptr, lds_raw);
-    __syncthreads();  // the table ends with the last wave's chains
-    if (threadIdx.x == 0) g.ticks[2 * t + 1] = (uint64_t)wall_clock64();
+    // The table ends with its last wave.  A barrier would keep the places of
+    // the waves that are done from the next table's (16,384 tables of 16 to 500
+    // items and 16 waves, without PSA+: 0.62 ms, 0.82 with a barrier).
+    if ((threadIdx.x & 63) == 0 && atomicAdd(&ended, 1u) == blockDim.x / 64 - 1) g.ticks[2 * t + 1] = (uint64_t)wall_clock64();
 }
 
 // Basic alias sampling of every table: sample k of table t uses the Philox
