@@ -472,13 +472,31 @@ atg_status make_groups(atg_batch* b, int64_t group_items) {
             group_of[t] = (int32_t)g;
         }
         for (int64_t t = 0; t < ntables; ++t) members[group_of[t]].push_back(t);
-        for (int64_t g = 0; g < ngroups; ++g)
-            for (int64_t t : members[g])
-                if (b->small_class[t] < 0) groups[g].G_max = std::max(groups[g].G_max, b->args[t].G);
+    }
+    // Small tables of a group go by themselves where they are all of it or
+    // enough (small_beside_ok).
+    std::vector<int8_t> small((size_t)ntables, 0);
+    for (int64_t g = 0; g < ngroups; ++g) {
+        int64_t sections = 0, others = 0;
+        std::vector<int8_t> used(b->small_classes.size(), 0);
+        for (int64_t t : members[g]) {
+            if (b->small_class[t] < 0) {
+                ++others;
+                continue;
+            }
+            sections += b->args[t].G;
+            used[b->small_class[t]] = 1;
+        }
+        const int classes = (int)std::count(used.begin(), used.end(), 1);
+        const bool ok = others == 0 || small_beside_ok(sections, classes);
+        for (int64_t t : members[g]) {
+            small[t] = ok && b->small_class[t] >= 0;
+            if (!small[t]) groups[g].G_max = std::max(groups[g].G_max, b->args[t].G);
+        }
     }
     auto blocks_of = [&](int ph, int64_t t) -> int64_t {
         const BuildArgs& a = b->args[t];
-        if (b->small_class[t] >= 0) return 0;
+        if (small[t]) return 0;
         switch (ph) {
             case MAP_SUM: return (a.G + 3) / 4;
             case MAP_LOCAL: return a.G;
@@ -521,7 +539,7 @@ atg_status make_groups(atg_batch* b, int64_t group_items) {
             const int64_t at = (int64_t)tab.size();
             int64_t work = 0;
             for (int64_t t : members[g])
-                if (b->small_class[t] == c) {
+                if (small[t] && b->small_class[t] == c) {
                     tab.push_back((int32_t)t);
                     work += offsets[t + 1] - offsets[t] + 300;
                 }

@@ -56,6 +56,17 @@ inline bool small_class_of(int64_t n, int64_t G, int64_t Ls, int64_t p_req, Smal
     return c.lds <= kSmallTiers[2];
 }
 
+// Whether a group's small tables, so many sections of so many classes, pay for
+// launches of their own beside the phases of its other tables: the fork, the
+// launches and the join cost 15 to 20 us and each class some more, and the
+// phases take a wave per section.  In the phases and so, us, with few larger
+// tables beside: 64 tables of 11 sections, one class 57 and 73; 2,000 of one
+// section 75 and 80, 10,000 255 and 112; 400 of 11 sections 93 and 73.  Sizes
+// log-uniform over a hundredfold or more, sections by classes and two: 47 by 10
+// 57 and 137, 459 by 9 67 and 152, 2,680 by 9 332 and 381, 5,593 by 7 267 and
+// 261, 7,610 by 10 234 and 204, 22,595 by 7 311 and 206.
+inline bool small_beside_ok(int64_t sections, int classes) { return sections >= 640 * (int64_t)(classes + 2); }
+
 // The light list followed by the heavy list (from entry numL) in LDS.
 struct SmallLists {
     const double* w;

@@ -21,6 +21,7 @@ int main(int argc, char** argv) {
         if (small_class_of(arg(2), arg(3), arg(4), arg(5), c)) printf("%d %d %d\n", kSmallChunks[c.xu], c.waves, c.tier);
         else printf("none\n");
     }
+    if (what[0] == 'b') printf("%d\n", (int)small_beside_ok(arg(2), (int)arg(3)));  // beside sections classes
     if (what[0] == 'r') printf("%u\n", rej_share((uint32_t)arg(2)));  // rej_share m
     return 0;
 }
@@ -64,3 +65,9 @@ def test_small_class(rule, n, G, Ls, p, want):
 def test_rejection_share(rule, m, want):
     """16 shares hold every sample, none of fewer than a wave's lanes."""
     assert rule("rej_share", m) == str(want) and 16 * want >= m
+
+
+@pytest.mark.parametrize("sections,classes,want", [
+    (47, 8, 0), (704, 1, 0), (1919, 1, 0), (1920, 1, 1), (3839, 4, 0), (3840, 4, 1), (22_595, 5, 1)])
+def test_small_tables_beside_others(rule, sections, classes, want):
+    assert rule("beside", sections, classes) == str(want)
