@@ -64,10 +64,20 @@ inline int64_t light_dir_size(int64_t n) { return (n >> kLightDirShift) + 2; }
 // at 100 670 / 658 and 754 / 664; 1e8 at 100 (staged) 2,080 / 2,128 and 2,261 /
 // 2,120, at 150 2,041 / 2,062 and 2,542 / 2,141, at 200 2,077 / 2,055 and 2,826
 // / 2,116.
+// The card holds 3,072 of its waves, kWindowRound chains (12 of 13 KB of LDS a
+// CU).  Up to half a round more, most of the card waits for the few left over,
+// which only longer chains outweigh (Pareto and the mix of heavies, sections
+// of 2048, 110,000 chains: 7e6 items 159 / 181 and 149 / 164, 1.1e7 250 / 269
+// and 218 / 237, 1.4e7 316 / 317 and 270 / 280; over twelve distributions and
+// shapes the windowed builds take 1.07, 1.04 and 0.97 of the staged ones, of
+// 80,000 and 160,000 chains at n / p = 100 0.95 and 0.94).
+constexpr int64_t kWindowRound = 3072 * 32;
 inline bool pack_windowed_ok(int64_t n, int64_t p_req, int32_t pack_method) {
     if (pack_method != PACK_CHUNKED || p_req <= 0) return false;
     const int64_t per = n / p_req;
-    return per > 256 || (per >= 32 && 30 * per * per > p_req);
+    if (per > 256) return true;
+    const bool tail = p_req > kWindowRound && 2 * p_req < 3 * kWindowRound;
+    return per >= 32 && (tail ? 7 : 30) * per * per > p_req;
 }
 // Tables below this many items keep whole lists: finding a light in the
 // staging takes the pack a few dependent reads, which the smaller writes pay

@@ -22,6 +22,7 @@ int main(int argc, char** argv) {
         else printf("none\n");
     }
     if (what[0] == 'b') printf("%d\n", (int)small_beside_ok(arg(2), (int)arg(3)));  // beside sections classes
+    if (what[0] == 'w') printf("%d\n", (int)pack_windowed_ok(arg(2), arg(3), PACK_CHUNKED));  // windowed n p
     if (what[0] == 'r') printf("%u\n", rej_share((uint32_t)arg(2)));  // rej_share m
     return 0;
 }
@@ -71,3 +72,15 @@ def test_rejection_share(rule, m, want):
     (47, 8, 0), (704, 1, 0), (1919, 1, 0), (1920, 1, 1), (3839, 4, 0), (3840, 4, 1), (22_595, 5, 1)])
 def test_small_tables_beside_others(rule, sections, classes, want):
     assert rule("beside", sections, classes) == str(want)
+
+
+@pytest.mark.parametrize("n,p,want", [
+    (1_000_000, 30_700, 1), (1_000_000, 31_000, 0),
+    (5_120_000, 80_000, 1), (98_304 * 64, 98_304, 1),
+    (98_305 * 64, 98_305, 0), (7_040_000, 110_000, 0), (11_000_000, 110_000, 0),   # a second round of few waves
+    (14_080_000, 110_000, 1), (147_455 * 128, 147_455, 0), (147_456 * 80, 147_456, 1),
+    (16_000_000, 160_000, 1), (100_000_000, 1_000_000, 0), (100_000_000, 666_000, 1),
+    (257 * 110_000, 110_000, 1),
+])
+def test_windowed_pack(rule, n, p, want):
+    assert rule("windowed", n, p) == str(want)

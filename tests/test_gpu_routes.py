@@ -4,6 +4,7 @@ import pytest
 
 import atg
 from launches import kernels, launches
+from test_gpu_build import assert_same_build
 
 pytestmark = pytest.mark.gpu
 
@@ -78,3 +79,17 @@ def test_staged_counts_of_few_samples(gpu, count, counters):
     t.rejection_sample_sectioned(count, 1)  # reads the array's size back, outside the capture
     name, _, _, lds = launches(gpu, lambda s: t.rejection_sample_sectioned(count, 1, hist=hist, stream=s))[-1]
     assert (name, lds) == ("rej_sample_sectioned", 4096 * 16 + counters)
+
+
+@pytest.mark.parametrize("n,p,pack", [(98_304 * 60, 98_304, "pack_windowed"), (98_305 * 64, 98_305, "pack_staged"),
+                                      (147_456 * 75, 147_456, "pack_windowed")])
+def test_pack_at_the_end_of_a_round(gpu, oracle, n, p, pack):
+    """Where the windowed pack's waves just fit the card, have a few more than
+    that, and again have enough: the pack that runs, and its rows."""
+    w = atg.generate_weights("heavy_mix", n, seed=3, param=0.9)
+    t = atg.Table(n, section_size=2048, num_splits=p)
+    t.set_weights(w)
+    assert pack in kernels(gpu, t.build)
+    t.build()
+    t.sync()
+    assert_same_build(t, oracle.build(w, section_size=2048, num_splits=p), n)
