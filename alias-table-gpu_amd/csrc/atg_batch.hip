@@ -395,7 +395,8 @@ hipError_t launch_batch(const atg_batch* b, hipStream_t s) {
     hipLaunchKernelGGL(seg_reset_ticks, dim3((unsigned)std::min<int64_t>((b->ntables + 255) / 256, 4096)), dim3(256),
                        0, s, g);
     const size_t lds = psa_lds_bytes(b->Ls_max);
-    const int64_t resident = resident_blocks((const void*)seg_local<T, true>, 64, lds);
+    const int64_t resident_later = resident_blocks((const void*)seg_local<T, true>, 64, lds);
+    const int64_t resident_step = resident_blocks((const void*)seg_local<T, false>, 64, lds);
     const bool learned = b->opts.split_method == ATG_SPLIT_LEARNED;
     for (const BatchGroup& grp : b->groups) {
         const SegMap* M = grp.maps;
@@ -418,7 +419,8 @@ hipError_t launch_batch(const atg_batch* b, hipStream_t s) {
         if (phases) {
             hipLaunchKernelGGL(seg_sum<T>, grid(M[MAP_SUM]), dim3(256), 0, s, g, M[MAP_SUM]);
             hipLaunchKernelGGL(seg_sum_finish, grid(M[MAP_ONE]), dim3(256), 0, s, g, M[MAP_ONE]);
-            const bool later = rows_later_ok(M[MAP_LOCAL].blocks, resident);
+            const bool later = batch_rows_later_ok(M[MAP_LOCAL].blocks, resident_later, grp.items, b->Ls_max);
+            const int64_t resident = later ? resident_later : resident_step;
             hipLaunchKernelGGL((later ? seg_local<T, true> : seg_local<T, false>),
                                dim3((unsigned)std::min<int64_t>(M[MAP_LOCAL].blocks, resident)), dim3(64), lds, s, g,
                                M[MAP_LOCAL]);

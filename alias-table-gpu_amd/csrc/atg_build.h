@@ -152,13 +152,33 @@ inline size_t psa_lds_bytes(int64_t Ls_max) {
     const size_t need = (size_t)Ls_max * 10, past = ((size_t)Ls_max + 8) * 8;
     return ((need > past ? need : past) + 15) & ~(size_t)15;
 }
+// Sections of at most this many items run the partition kernel that holds
+// half the weight registers.
+constexpr int64_t kShortSectionMax = 1024;
 // Rows written after the chains rather than by each of their steps: pays
-// where the device is full of sections and HBM is what counts (1e8 items at
+// where the device is full of sections and the rows go to HBM (1e8 items at
 // sections of 2048: the pass takes 0.74 against 0.82 ms; uniform weights at
 // sections of 1000: 0.74 against 1.12), costs the extra pass over the section
 // where each has a wave to itself from the start (101 sections: 21 against 18
-// us; 1,049 sections: the same).
-inline bool rows_later_ok(int64_t sections, int64_t resident) { return sections > resident; }
+// us; 1,049 sections: the same).  16-byte rows that fit the 256 MB of the
+// Infinity Cache are joined there anyway, and then only short sections, four
+// waves a SIMD, hide the pass (builds, later / by step, 5e6 to 1.4e7 items:
+// sections of 2048, 16 chains 1.15-1.22 uniform, 1.09-1.16 exponential, 0.97-1.02
+// Pareto, 0.95 heavy mix; sections of 1000 0.96-1.05, 0.93-1.01, 0.95-1.02,
+// 0.95; 2e7 and more at 2048 1.03-1.09, 0.88-1.07, 0.95-1.05, 0.92).  Split rows,
+// 8 and 4 bytes, come in smaller pieces and pay at any size (sections of 1000
+// 0.71-0.88 uniform and exponential).
+constexpr int64_t kCachedRows = (int64_t)1 << 24;
+inline bool rows_later_ok(int64_t sections, int64_t resident, bool aos, int64_t n, int64_t Ls_max) {
+    return sections > resident && (!aos || n > kCachedRows || Ls_max <= kShortSectionMax);
+}
+// A batch's kernel holds sections of any length at two waves a SIMD: it hides
+// the pass nowhere, and short chains leave it nothing to gain (later / by step:
+// sections of 1000 0.98-1.12 at any size; of 2048, 32 chains 0.99-1.06 up to 2e7
+// items, 0.84-0.95 uniform and exponential, 1.0-1.04 Pareto from 6e7).
+inline bool batch_rows_later_ok(int64_t sections, int64_t resident, int64_t items, int64_t Ls_max) {
+    return sections > resident && items > kCachedRows && Ls_max > kShortSectionMax;
+}
 int64_t resident_blocks(const void* f, int threads, size_t lds);
 // Up to this many sections the placement folds P(s) from the sections' own
 // sums, without the tree's launches (builds, us, with and without the tree:

@@ -63,9 +63,6 @@ __device__ __forceinline__ double section_sum(const T* w, int64_t start, int64_t
 
 
 #define PSA_MAX_LEN 2048
-// Sections of at most this many items run the partition kernel that holds
-// half the weight registers.
-constexpr int64_t kShortSectionMax = 1024;
 // Lights of a chain a partition wave looks at together (2, 3, 6 and 8 were no
 // faster over Pareto, exponential, uniform and Zipf weights).
 constexpr int kRun = 4;

@@ -22,6 +22,8 @@ int main(int argc, char** argv) {
         else printf("none\n");
     }
     if (what[0] == 'b') printf("%d\n", (int)small_beside_ok(arg(2), (int)arg(3)));  // beside sections classes
+    if (what[0] == 'l') printf("%d\n", (int)rows_later_ok(arg(2), arg(3), arg(4) != 0, arg(5), arg(6)));  // later sections resident aos n Ls
+    if (what[0] == 'g') printf("%d\n", (int)batch_rows_later_ok(arg(2), arg(3), arg(4), arg(5)));  // group_later sections resident items Ls
     if (what[0] == 'w') printf("%d\n", (int)pack_windowed_ok(arg(2), arg(3), PACK_CHUNKED));  // windowed n p
     if (what[0] == 'r') printf("%u\n", rej_share((uint32_t)arg(2)));  // rej_share m
     return 0;
@@ -84,3 +86,21 @@ def test_small_tables_beside_others(rule, sections, classes, want):
 ])
 def test_windowed_pack(rule, n, p, want):
     assert rule("windowed", n, p) == str(want)
+
+
+@pytest.mark.parametrize("sections,resident,aos,n,Ls,want", [
+    (2048, 2048, 1, 1 << 22, 2048, 0), (2048, 2048, 0, 1 << 22, 2048, 0),      # a wave each from the start
+    (2442, 2048, 1, 5_000_000, 2048, 0), (8192, 2048, 1, 1 << 24, 2048, 0),    # long sections, rows in the cache
+    (8193, 2048, 1, (1 << 24) + 1, 2048, 1), (48_829, 2048, 1, 100_000_000, 2048, 1),
+    (2442, 2048, 0, 5_000_000, 2048, 1),                                       # split rows
+    (10_001, 4096, 1, 10_000_019, 1000, 1), (5001, 4096, 1, 5_000_000, 1024, 1), (5001, 4096, 1, 5_000_000, 1025, 0),
+])
+def test_rows_later(rule, sections, resident, aos, n, Ls, want):
+    assert rule("later", sections, resident, aos, n, Ls) == str(want)
+
+
+@pytest.mark.parametrize("sections,resident,items,Ls,want", [
+    (100_000, 2048, 100_000_000, 1000, 0), (100_000, 2048, 100_000_000, 2048, 1),
+    (2048, 2048, 100_000_000, 2048, 0), (8192, 2048, 1 << 24, 2048, 0)])
+def test_group_rows_later(rule, sections, resident, items, Ls, want):
+    assert rule("group_later", sections, resident, items, Ls) == str(want)

@@ -46,3 +46,28 @@ def test_batch_with_many_sections_matches_single_tables(gpu, oracle):
     ow, oa, oW = oracle.build_batch(w, offsets, chains=8, section_size=64, num_splits=-38)
     assert np.array_equal(W.view(np.uint64), oW.view(np.uint64))
     assert np.array_equal(rw.view(np.uint64), ow.view(np.uint64)) and np.array_equal(ra, oa)
+
+
+@pytest.mark.parametrize("n,dist", [((1 << 24) + 5, "exponential"), ((1 << 24) - 5, "exponential")])
+def test_long_sections_around_the_cached_rows(gpu, oracle, n, dist):
+    """16-byte rows of sections of 2048 just past and just within what the rule
+    takes for cached: whole sections after the chains, and rows by each step."""
+    w = atg.generate_weights(dist, n, seed=17)
+    t = gpu_build(w, chains=17, section_size=2048, num_splits=n // 64)
+    assert_same_build(t, oracle.build(w, chains=17, section_size=2048, num_splits=n // 64), n)
+
+
+def test_large_batch_with_many_long_sections(gpu, oracle):
+    """A batch whose rows are written after the chains."""
+    sizes = [3_000_000, 1, 2047, 2048, 2049, 64, 4_500_000, 100_001] * 3
+    offsets = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+    assert offsets[-1] > 1 << 24
+    w = atg.generate_weights("exponential", int(offsets[-1]), seed=3)
+    b = atg.Batch(offsets, section_size=2048, chains=32, num_splits=-38)
+    b.set_weights(w)
+    b.build()
+    b.sync()
+    rw, ra, W = b.tables()
+    ow, oa, oW = oracle.build_batch(w, offsets, chains=32, section_size=2048, num_splits=-38)
+    assert np.array_equal(W.view(np.uint64), oW.view(np.uint64))
+    assert np.array_equal(rw.view(np.uint64), ow.view(np.uint64)) and np.array_equal(ra, oa)
