@@ -72,12 +72,17 @@ inline int64_t light_dir_size(int64_t n) { return (n >> kLightDirShift) + 2; }
 // shapes the windowed builds take 1.07, 1.04 and 0.97 of the staged ones, of
 // 80,000 and 160,000 chains at n / p = 100 0.95 and 0.94).
 constexpr int64_t kWindowRound = 3072 * 32;
+// Lists that fit the staged pack's pool (1,024 items) at once or nearly are
+// staged at once (whole builds, windowed by
+// staged: 1,000 items at n / p = 100 1.1 to 1.8, at 200 1.1 to 1.4; 2,000 0.8 to
+// 1.2 at 64, 1.1 to 1.6 at 200; 3,000 0.65 to 1.1 at 64).
+constexpr int64_t kWindowMinItems = 2048;
 inline bool pack_windowed_ok(int64_t n, int64_t p_req, int32_t pack_method) {
     if (pack_method != PACK_CHUNKED || p_req <= 0) return false;
     const int64_t per = n / p_req;
     if (per > 256) return true;
     const bool tail = p_req > kWindowRound && 2 * p_req < 3 * kWindowRound;
-    return per >= 32 && (tail ? 7 : 30) * per * per > p_req;
+    return n > kWindowMinItems && per >= 32 && (tail ? 7 : 30) * per * per > p_req;
 }
 // Tables below this many items keep whole lists: finding a light in the
 // staging takes the pack a few dependent reads, which the smaller writes pay

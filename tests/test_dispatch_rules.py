@@ -83,6 +83,7 @@ def test_small_tables_beside_others(rule, sections, classes, want):
     (14_080_000, 110_000, 1), (147_455 * 128, 147_455, 0), (147_456 * 80, 147_456, 1),
     (16_000_000, 160_000, 1), (100_000_000, 1_000_000, 0), (100_000_000, 666_000, 1),
     (257 * 110_000, 110_000, 1),
+    (100, 2, 0), (2048, 20, 0), (2049, 20, 1), (1000, 3, 1),                       # lists that are staged at once
 ])
 def test_windowed_pack(rule, n, p, want):
     assert rule("windowed", n, p) == str(want)

@@ -93,3 +93,16 @@ def test_pack_at_the_end_of_a_round(gpu, oracle, n, p, pack):
     t.build()
     t.sync()
     assert_same_build(t, oracle.build(w, section_size=2048, num_splits=p), n)
+
+
+@pytest.mark.parametrize("n,p,pack", [(100, 2, "pack_staged"), (2048, 10, "pack_staged"), (2049, 10, "pack_windowed")])
+def test_pack_of_small_tables(gpu, oracle, n, p, pack):
+    """Tables whose lists the staged pack holds at once, or nearly."""
+    w = atg.generate_weights("unit_uniform", n, seed=3)
+    for psa in (True, False):
+        t = atg.Table(n, num_splits=p, split="learned", psa_plus=psa)
+        t.set_weights(w)
+        assert pack in kernels(gpu, t.build)
+        t.build()
+        t.sync()
+        assert_same_build(t, oracle.build(w, num_splits=p, psa_plus=psa), n)
