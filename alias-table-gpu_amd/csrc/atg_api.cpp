@@ -72,7 +72,6 @@ struct atg_table_s {
     uint32_t* d_sec_loff = nullptr;  // lean light lists: lights before each section
     uint32_t* d_sec_ldir = nullptr;  // lean light lists: the section of every 1024th light
     bool placed = false;             // the staging and sec_loff of the last partition are current
-    bool lists_full = false;         // the last build left whole lists (no staging): a one-launch build
     bool staged = false;             // the staging and section sums hold a partition (a one-launch build has none)
     double* d_stage_w = nullptr;
     int32_t* d_stage_i = nullptr;
@@ -160,7 +159,7 @@ struct atg_table_s {
         a.pack_method = opts.pack_method;
         a.sec_loff = d_sec_loff;
         a.sec_ldir = d_sec_ldir;
-        a.lean_lights = d_sec_loff && d_sec_ldir && !lists_full && lean_lights_ok(n, p_req, opts.pack_method) ? 1 : 0;
+        a.lean_lights = d_sec_loff && d_sec_ldir && lean_lights_ok(n, p_req, opts.pack_method) ? 1 : 0;
         return a;
     }
 };
@@ -264,7 +263,7 @@ atg_status atg_create(atg_table** out, int64_t n, atg_dtype dtype, atg_layout la
     ALLOC(t->d_state, 1);
     ALLOC(t->d_section_sums, t->G);
     ALLOC(t->d_tree, 2 * t->tree_half);
-    ALLOC(t->d_slots, 3 * t->tree_total + (t->tree_total + 1) / 2 + 1);
+    ALLOC(t->d_slots, 3 * t->tree_total);
     ALLOC(t->d_Li, n + 2);
     ALLOC(t->d_Hi, n + 2);
     ALLOC(t->d_Lw, n + 2);
@@ -345,8 +344,6 @@ atg_status atg_build_phase(atg_table* t, int32_t phase, void* stream) {
     if (!t->weights_set) return fail(ATG_ESTATE, "atg_build_phase: weights not set");
     hipStream_t s = (hipStream_t)stream;
     t->last_stream = s;
-    if (phase == ATG_PHASE_PARTITION || phase == ATG_PHASE_PARTITION_LOCAL || phase == ATG_PHASE_PARTITION_PLACE)
-        t->lists_full = false;
     const BuildArgs a = t->args();
     switch (phase) {
         case ATG_PHASE_SUM: HIPCHK(launch_sum(a, s)); break;
@@ -426,12 +423,10 @@ atg_status atg_build(atg_table* t, void* stream) {
         HIPCHK(launch_small(t->args(), true, nullptr, nullptr, s));
         t->placed = false;
         t->staged = false;
-        t->lists_full = true;
         t->built = true;
         return ATG_OK;
     }
     if (t->opts.interleave && t->sp_stream && !t->events) {
-        t->lists_full = false;
         const BuildArgs a = t->args();
         HIPCHK(launch_front(a, s));
         t->staged = true;
@@ -451,7 +446,6 @@ atg_status atg_build(atg_table* t, void* stream) {
     static const int before[4] = {0, 1, 3, 4};  // event recorded before each phase
     int first = 0;
     if (!t->events) {
-        t->lists_full = false;
         HIPCHK(launch_front(t->args(), s));
         t->staged = true;
         t->placed = true;

@@ -665,7 +665,7 @@ atg_status atg_batch_create(atg_batch** out, const int64_t* offsets, int64_t nta
         od[t] = nd;
         nd += align_up(z.G, 32) + align_up(2 * z.half, 32) + 5 * align_up(n + 2, 32);
         os[t] = ns;
-        ns += align_up(3 * z.tree_total + (z.tree_total + 1) / 2 + 1, 32) + align_up(6 * z.G, 32);
+        ns += align_up(3 * z.tree_total, 32) + align_up(6 * z.G, 32);
         oi[t] = ni;
         ni += 3 * align_up(n + 2, 64) + align_up(o.learned_segments + 2, 64) + align_up(z.G + 1, 64) +
               align_up(light_dir_size(n), 64);
@@ -711,7 +711,7 @@ atg_status atg_batch_create(atg_batch** out, const int64_t* offsets, int64_t nta
         const int64_t cap = align_up(n + 2, 32);
         a.Lw = d; a.Lp = d + cap; a.Hw = d + 2 * cap; a.Hp = d + 3 * cap; a.stage_w = d + 4 * cap;
         a.slots = b->d_slots + os[t];
-        a.sec_cert = a.slots + align_up(3 * z.tree_total + (z.tree_total + 1) / 2 + 1, 32);
+        a.sec_cert = a.slots + align_up(3 * z.tree_total, 32);
         a.want_cert = o.split_method == ATG_SPLIT_LEARNED;
         int32_t* ip = b->d_ipool + oi[t];
         const int64_t icap = align_up(n + 2, 64);

@@ -122,9 +122,10 @@ extern "C" atg_status atg_build_noalloc(const void* weights, atg_dtype dtype, in
     a.section_sums = c.take<double>(G);
     a.tree_scratch = c.take<double>(2 * tree_half);
     a.tree_scratch_half = tree_half;
+    // More than the 3 values a block: which shapes fit the scratch is part of the interface.
     a.slots = c.take<uint64_t>(3 * tree_total + (tree_total + 1) / 2 + 1);
     a.sec_cert = c.take<uint64_t>(6 * G);
-    a.want_cert = o.split_method != ATG_SPLIT_BISECT || split_by_group(o.split_method, p_req);
+    a.want_cert = o.split_method != ATG_SPLIT_BISECT;
     a.stage_w = c.take<double>(n);
     a.stage_i = c.take<int32_t>(n);
     a.Li = c.take<int32_t>(n + 2);
@@ -151,7 +152,6 @@ extern "C" atg_status atg_build_noalloc(const void* weights, atg_dtype dtype, in
     a.p_req = p_req;
     a.pack_cap = pack_cap_items(n, p_req);
     a.learned_segments = learned_knots(o.learned_segments, p_req);
-    a.direct_splits = split_by_group(o.split_method, p_req) ? kGroupedSplits / 2 : 0;
     a.pack_method = o.pack_method;
 
     hipStream_t s = (hipStream_t)stream;
@@ -162,10 +162,9 @@ extern "C" atg_status atg_build_noalloc(const void* weights, atg_dtype dtype, in
     hipLaunchKernelGGL(clear_state, dim3(1), dim3(64), 0, s, a.st);
     HIPCHK(hipGetLastError());
     HIPCHK(launch_front(a, s));
-    HIPCHK(o.split_method == ATG_SPLIT_LEARNED       ? launch_split_learned(a, s)
-           : o.split_method == ATG_SPLIT_PARY        ? launch_split_pary(a, s)
-           : split_by_group(o.split_method, p_req)   ? launch_split_grouped(a, s)
-                                                     : launch_split(a, s));
+    HIPCHK(o.split_method == ATG_SPLIT_LEARNED ? launch_split_learned(a, s)
+           : o.split_method == ATG_SPLIT_PARY  ? launch_split_pary(a, s)
+                                               : launch_split(a, s));
     HIPCHK(launch_pack(a, s));
     const char* st = reinterpret_cast<const char*>(a.st);
     if (W_out) HIPCHK(hipMemcpyAsync(W_out, st + offsetof(DevState, W), sizeof(double), hipMemcpyDeviceToDevice, s));
