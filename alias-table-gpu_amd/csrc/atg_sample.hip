@@ -932,11 +932,18 @@ hipError_t launch_sample_basic(const SampleArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Up to one sample in kSparseRows rows, the drawn rows are read one by one: a
+// Up to one sample in sparse_rows rows, the drawn rows are read one by one: a
 // drawn row costs a 128-byte line of its eight rows (staged against read one
 // by one, us: 1e8 rows, n/16 samples 288 and 151, n/8 290 and 242, n/4 307
 // and 423; 2^20 rows, n/64 9.9 and 6.8, n/8 10.3 and 9.1, n/4 10.5 and 12.1).
-constexpr uint64_t kSparseRows = 8;
+// Split rows stage less and cost two lines a sample, which pays for fewer
+// samples of long sections of large tables (staged against one by one, us:
+// sections of 4096, 3e6 rows n/8 16.9 and 13.1, 1e7 32 and 35, n/12 31 and 27;
+// 1e8 n/8 255 and 306, n/12 252 and 240; of 8192 1e7 n/8 33 and 42, n/12 33 and
+// 31; of 1024, the staging of many sections, n/8 45 and 29).
+inline uint64_t sparse_rows(bool aos, int64_t n, int64_t section) {
+    return aos || section < 4096 || n <= ((int64_t)1 << 22) ? 8 : 12;
+}
 // Sections whose counts the sampling waves find themselves: the descent takes
 // a wave about as long as one thread, so it pays while every section's wave
 // is resident at once.
@@ -987,7 +994,7 @@ static hipError_t launch_sectioned(void (*k)(Args...), int64_t nsec, int threads
 }
 
 hipError_t launch_sample_sectioned(const SampleArgs& a, hipStream_t s) {
-    if (a.count <= (uint64_t)a.n / kSparseRows) {
+    if (a.count <= (uint64_t)a.n / sparse_rows(a.rows != nullptr, a.n, a.SS)) {
         if (a.rows) launch_sparse<true>(a, s);
         else launch_sparse<false>(a, s);
         return hipGetLastError();

@@ -106,3 +106,23 @@ def test_pack_of_small_tables(gpu, oracle, n, p, pack):
         t.build()
         t.sync()
         assert_same_build(t, oracle.build(w, num_splits=p, psa_plus=psa), n)
+
+
+@pytest.mark.parametrize("layout,n,rows,count,sparse", [
+    ("aos", 100_003, 4096, 12_500, True), ("aos", 100_003, 4096, 12_501, False),
+    ("soa", 100_003, 4096, 12_500, True), ("soa", 100_003, 4096, 12_501, False),
+    ("aos", 4_200_000, 4096, 525_000, True), ("soa", 4_200_000, 4096, 350_000, True),
+    ("soa", 4_200_000, 4096, 350_001, False), ("soa", 4_200_000, 8192, 525_000, False),
+    ("soa", 4_200_000, 4095, 525_000, True)])
+def test_line_of_sparse_draws(gpu, oracle, layout, n, rows, count, sparse):
+    """Few samples a row read the drawn rows, fewer where a row is in two pieces."""
+    t = atg.Table(n, layout=layout)
+    t.set_weights(atg.generate_weights("pareto", n, seed=3, param=1.1))
+    t.build()
+    tw, ta = t.table()
+    out = gpu.empty(count, dtype=gpu.int32, device="cuda")
+    t.sample(1, 4, section_rows=rows)  # grows the buffer of the sections' counts
+    ks = kernels(gpu, lambda s: t.sample(count, 4, section_rows=rows, out=out, stream=s))
+    assert (ks[-1] == "sample_sectioned_sparse") == sparse
+    t.sample(count, 4, section_rows=rows, out=out)
+    assert (out.cpu().numpy() == oracle.sample_sectioned(tw, ta, t.stats()["W_N"], rows, count, 4)).all()
