@@ -127,10 +127,10 @@ inline int32_t pack_cap_items(int64_t n, int64_t p_req) {
     int64_t cap = (64 * (per + 1) + 2 + 15) / 16 * 16;
     return (int32_t)(cap < kPackPoolItems ? cap : kPackPoolItems);
 }
-// A pack round that fits fewer chains than this into the pool, and not all
-// that are left, hands them to their lanes, each reading the lists from HBM
-// (chains that all fit are staged: whole builds of 500 and 1,000 items in two
-// to five chains 45 -> 34 us).
+// A pack round that fits fewer chains than this into the pool, and not all of
+// the wave's, hands the chains that are left to their lanes, each reading the
+// lists from HBM (a wave's chains that all fit are staged: whole builds of 500
+// and 1,000 items in two to five chains 45 -> 34 us).
 constexpr int kPackMinStagedChains = 8;
 // Weight (8 B), item (4 B) and recorded alias (4 B) per pool item, and the
 // spare weight slot the light steps record into (16 B keep the alignment).

@@ -365,10 +365,10 @@ static void (*partition_local_kernel(const BuildArgs& a))(BuildArgs) {
 
 static hipError_t launch_partition_kernel(const BuildArgs& a, bool own_w, hipStream_t s) {
     const size_t lds = psa_lds_bytes(a.Ls_max);
-    void (*k)(BuildArgs) = partition_local_kernel<true, false>(a);
+    void (*k)(BuildArgs) = own_w ? partition_local_kernel<false, true>(a) : partition_local_kernel<true, false>(a);
     int64_t resident = resident_blocks((const void*)k, 64, lds);
-    if (own_w || !rows_later_ok(a.G, resident, a.rows != nullptr, a.n, a.Ls_max)) {
-        k = own_w ? partition_local_kernel<false, true>(a) : partition_local_kernel<false, false>(a);
+    if (!own_w && !rows_later_ok(a.G, resident, a.rows != nullptr, a.n, a.Ls_max)) {
+        k = partition_local_kernel<false, false>(a);
         resident = resident_blocks((const void*)k, 64, lds);
     }
     hipLaunchKernelGGL(k, dim3((unsigned)std::min<int64_t>(a.G, resident)), dim3(64), lds, s, a);

@@ -1457,7 +1457,7 @@ __device__ __forceinline__ void pack_staged_block(const BuildArgs& a, int64_t bl
         const int Ia = __shfl(prev.i, ta, 64), Ja = __shfl(prev.j, ta, 64);
         const bool fits = mine && lane >= ta && (cur.i - Ia) + (cur.j - Ja + 1) <= cap;
         const int tb = ta + __popcll(__ballot(fits));
-        if (tb < nch && tb - ta < kPackMinStagedChains && !a.lean_lights) {
+        if ((ta > 0 || tb < nch) && tb - ta < kPackMinStagedChains && !a.lean_lights) {
             // Long chains: so few fit the pool at once that the rounds would
             // run the wave's chains nearly one after another; every lane
             // runs its own chain from the lists in HBM instead, all at once.
